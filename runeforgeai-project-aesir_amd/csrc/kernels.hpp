@@ -142,6 +142,24 @@ int32_t launch_qf_gemm_wide(hipStream_t s, int epi, int nt, const void *A, int64
 // 32-bit byte ranges), and that product stored as f16 C [M][N] (context stream and partials).
 bool gemm_qf_wide_ok(int64_t M, int64_t K, int64_t N);
 int32_t launch_gemm_qf_mfma(aesir_ctx *ctx, const void *A, int64_t M, int64_t K, const QFMat &w, int64_t N, void *C);
+// Short-chunk GEMM (skinny.hip) of 1 to 64 activation rows on a matrix of any type, K % 128 == 0.
+// A weight matrix of N rows: f16 [N][K] (type F16: w), int8 quants [N][K] and f16 block scales
+// [N][K / 32] (Q8_0: w, s), 16-byte aligned, or the tiled planes of a repacked type (qf).
+struct SkinnyMat {
+    int32_t type = 0;
+    const void *w = nullptr, *s = nullptr;
+    QFMat qf;
+};
+constexpr int64_t kSkinnyMaxRows = 64;
+struct SkinnyPlan {
+    int nw = 0;  // waves per workgroup; 0: the shape is not taken
+    int64_t splits = 1;
+};
+SkinnyPlan skinny_plan(int64_t M, int64_t K, int64_t N, int32_t type, bool may_split);
+// C = epilogue epi (GemmEpi) of A W^T, or with splits > 1 the f32 partials part[z][M][ldp] (columns
+// 0 .. N - 1 of rows of ldp).
+int32_t launch_gemm_skinny(hipStream_t s, int epi, const SkinnyMat &w, const void *A, int64_t M, int64_t K, int64_t N,
+                           void *C, int64_t ldc, float *part, int64_t ldp, const SkinnyPlan &p);
 // y[n] = f16(sum_k x[k] w[n, k]) for one row of x (the per-op GEMV of a repacked matrix).
 int32_t launch_qf_gemv_store(hipStream_t s, const QFMat &w, int64_t N, int64_t K, const void *x, void *y);
 // Decode-step GEMVs of repacked matrices with the fused epilogues (see the F16 launchers).

@@ -14,8 +14,9 @@
 //   in lane l).
 //   Small-N GEMMs also split K over grid.z to put enough weight bytes in flight; their f32
 //   partials are summed in a fixed order by the epilogue kernel (deterministic, no atomics).
-//   Chunks of more than 64 positions use the wide-tile kernel below (the whole chunk in one
-//   128-row M tile, 8 waves, 128-wide K chunks) instead; this 32-row kernel serves shorter chunks.
+//   Chunks of up to 64 positions run on the short-chunk GEMM (skinny.hip) and longer ones on the
+//   wide-tile kernel below (the whole chunk in one 128-row M tile, 8 waves, 128-wide K chunks);
+//   this 32-row kernel serves the widths that are a multiple of 64 but not of 128.
 //   At M = 128 the GEMM is HBM-bound (128 flop/byte against MI355X's 312 flop/byte ridge).
 #include <cmath>
 #include <vector>
@@ -33,9 +34,7 @@ namespace aesir {
 // with 64-wide K chunks. Measured on MI355X (TinyLlama 128-token prefill, ms, when this kernel
 // served every chunk): M tile 128 / 256 workgroups 2.39; 64 / 256 2.31; 64 / 512 2.23; 32 / 512
 // 2.22; 32 / 1024 2.37. Smaller tiles re-read the weights from L2 (one HBM read) but copy less of
-// A per workgroup and fit more workgroups per CU. (The 8-wave wide-tile kernel below, with
-// 128-wide chunks, does better with the whole 128-row chunk in one tile; this kernel now serves
-// chunks of 64 rows or fewer.)
+// A per workgroup and fit more workgroups per CU.
 constexpr int kGemmMT = 32;
 constexpr int kGemmWgTarget = 512;
 constexpr int kGemmMF = kGemmMT / 16;   // MFMA row fragments per wave
@@ -677,8 +676,33 @@ static int32_t prefill_gemm_blas(aesir_model *m, hipStream_t s, const void *W, c
     return AESIR_OK;
 }
 
+static SkinnyMat skinny_mat(const WMat &w) {
+    SkinnyMat k;
+    k.type = w.type;
+    if (qf_type(w.type)) k.qf = wmat_qf(w);
+    else k.w = w.w, k.s = w.s0;
+    return k;
+}
+
+// The short-chunk GEMM with the split count reduced to the partial buffer; `defer` and *splits_out as
+// launch_mfma's.
+template <int EPI>
+static int32_t launch_skinny(hipStream_t s, const SkinnyMat &w, const void *A, int64_t M, int64_t K, int64_t N, void *C,
+                             int64_t ldc, float *part, int64_t part_floats, SkinnyPlan p, bool defer, int64_t *splits_out) {
+    while (p.splits > 1 && p.splits * M * N > part_floats) p.splits--;
+    AESIR_TRY(launch_gemm_skinny(s, EPI, w, A, M, K, N, C, ldc, part, N, p));
+    if (splits_out) *splits_out = p.splits;
+    if (p.splits > 1 && !defer) {
+        hipLaunchKernelGGL(gemm_reduce_kernel<EPI>, dim3((unsigned)((M * N + 255) / 256)), dim3(256), 0, s, (const float *)part,
+                           p.splits, M, N, (h16 *)C, ldc);
+        AESIR_LAUNCH_CHECK("gemm_reduce_kernel");
+    }
+    return AESIR_OK;
+}
+
 // A GEMM of the prefill on the model's matrix w (rows N, K wide): F16 weights in chunks of
-// kBlasMinRows rows or more on hipBLASLt (prefill_gemm_blas); repacked types on the wide-tile
+// kBlasMinRows rows or more on hipBLASLt (prefill_gemm_blas); chunks of up to kSkinnyMaxRows rows on
+// the short-chunk GEMM, whatever the type; repacked types on the wide-tile
 // kernel that dequantizes in registers (launch_qf_gemm_wide) where the wide tile applies, else
 // through an f16 copy in m->pf_wdeq; F16 and Q8_0 weights on launch_mfma. `defer` and *splits_out
 // as launch_mfma's (split partials left in m->pf_part). *part_out: the library path's deferred
@@ -703,6 +727,8 @@ static int32_t prefill_gemm(aesir_model *m, hipStream_t s, const WMat &w, const 
         }
     }
     if (part_out) *part_out = nullptr;
+    if (const SkinnyPlan sp = skinny_plan(M, K, N, w.type, EPI != kEpiSwiglu); sp.nw)
+        return launch_skinny<EPI>(s, skinny_mat(w), A, M, K, N, C, ldc, m->pf_part, m->pf_part_floats, sp, defer, splits_out);
     if (!qf_type(w.type))
         return launch_mfma<EPI>(s, A, M, K, w.w, N, C, ldc, m->pf_part, m->pf_part_floats, name, defer, splits_out,
                                 w.type == AESIR_GGML_Q8_0 ? w.s0 : nullptr);
@@ -745,6 +771,13 @@ int32_t launch_gemm_qf_mfma(aesir_ctx *ctx, const void *A, int64_t M, int64_t K,
 
 int32_t launch_gemm_f16_mfma(aesir_ctx *ctx, const void *A, int64_t M, int64_t K, const void *B, int64_t N, void *C) {
     if (!mfma_shape_ok(A, M, K, B, N)) return launch_gemm_f16(ctx, A, M, K, B, N, C);
+    if (const SkinnyPlan sp = skinny_plan(M, K, N, AESIR_GGML_F16, true); sp.nw) {
+        SkinnyMat w;
+        w.type = AESIR_GGML_F16;
+        w.w = B;
+        return launch_skinny<kEpiStore>(ctx->stream, w, A, M, K, N, C, N, ctx->scratch.attn_part,
+                                        ctx->scratch.attn_part_floats, sp, false, nullptr);
+    }
     return launch_mfma<kEpiStore>(ctx->stream, A, M, K, B, N, C, N, ctx->scratch.attn_part,
                                   ctx->scratch.attn_part_floats, "gemm_mfma_kernel");
 }
@@ -1462,7 +1495,17 @@ static int32_t prefill_chunk(aesir_model *m, const int64_t *tokens_host, int64_t
         if (!xn_ready) AESIR_TRY(norm_rows(L.attn_norm));
         xn_ready = false;
         int64_t qkv_splits = 1;
-        if (mfma && L.qkv_split > 0) {
+        const SkinnyPlan qsp = L.qkv_split > 0 ? skinny_plan(n, d, qkv_n, L.qkv.type, true) : SkinnyPlan{};
+        if (mfma && qsp.nw) {
+            // a two-part Q/K/V of a short chunk: one launch per part, columns side by side
+            SkinnyPlan p = qsp;
+            while (p.splits > 1 && p.splits * n * qkv_n > m->pf_part_floats) p.splits--;
+            const int64_t na = L.qkv_split;
+            AESIR_TRY(launch_gemm_skinny(s, kEpiStore, skinny_mat(L.qkv), Xn, n, d, na, QKV, qkv_n, m->pf_part, qkv_n, p));
+            AESIR_TRY(launch_gemm_skinny(s, kEpiStore, skinny_mat(L.qkv_b), Xn, n, d, qkv_n - na, QKV + na, qkv_n,
+                                         m->pf_part + na, qkv_n, p));
+            qkv_splits = p.splits;
+        } else if (mfma && L.qkv_split > 0) {
             // a two-part Q/K/V: both parts dequantized into the f16 scratch matrix, then the F16 GEMM
             AESIR_TRY(launch_qf_dequant(s, wmat_qf(L.qkv), L.qkv_split, d, 1, nullptr, m->pf_wdeq, d));
             AESIR_TRY(launch_qf_dequant(s, wmat_qf(L.qkv_b), qkv_n - L.qkv_split, d, 1, nullptr,

@@ -1,0 +1,58 @@
+"""The short-chunk GEMM (1 to 64 activation rows, skinny.hip) at the edges of its tiles.
+
+Rows on both sides of the 16-row activation tiles, weight rows that end inside a 16-row block, a
+workgroup (64 or 128 rows) or a group of 4, one and an odd number of 128-wide K segments, and K splits.
+The bound is that of one f16 rounding of an f32 sum: 1 ulp, or 2^-17 of the sum of |products| (summation
+order over at most 2^14 terms in f32, taken generously) where cancellation leaves less.
+"""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+RNG = np.random.default_rng(77)
+
+
+@pytest.fixture(scope="module")
+def A():
+    import aesir_hip
+
+    return aesir_hip
+
+
+@pytest.fixture(scope="module")
+def ctx(A):
+    c = A.Context(1 << 30)
+    yield c
+    c.close()
+
+
+@pytest.fixture(autouse=True)
+def well_scope(ctx):
+    off = ctx.offset
+    yield
+    ctx.synchronize()
+    ctx.reset(off)
+
+
+def check(got, a, w):
+    a, w = a.astype(np.float64), w.astype(np.float64)
+    want = a @ w.T
+    ulp = np.spacing(np.abs(want).astype(np.float16)).astype(np.float64)
+    err = np.abs(got.astype(np.float64) - want)
+    noise = 2.0 ** -17 * (np.abs(a) @ np.abs(w).T)
+    assert np.all(err <= np.maximum(ulp, noise)), float((err - np.maximum(ulp, noise)).max())
+
+
+@pytest.mark.parametrize("M,K,N", [(2, 128, 1), (15, 128, 17), (16, 256, 64), (17, 384, 130), (32, 4096, 62),
+                                   (33, 2176, 300), (48, 256, 4100), (49, 640, 1023), (64, 4096, 4096),
+                                   (64, 14336, 70), (5, 5632, 2048)])
+def test_f16_edges(A, ctx, M, K, N):
+    a = RNG.standard_normal((M, K)).astype(np.float16)
+    b = (RNG.standard_normal((N, K)) * 0.02).astype(np.float16)
+    c = ctx.tensor(M + 1, N)  # a guard row behind the product
+    c.upload(np.full((M + 1, N), 7.0, np.float16))
+    A.gemm_f16(ctx, ctx.from_numpy(a), ctx.from_numpy(b), c.view(M, N))
+    got = c.numpy()
+    check(got[:M], a, b)
+    assert np.all(got[M] == 7.0)
