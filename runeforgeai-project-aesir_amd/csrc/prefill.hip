@@ -1056,161 +1056,77 @@ __global__ __launch_bounds__(kWave) void prefill_attention_kernel(const h16 *__r
     }
 }
 
-// The same attention for KV groups of 8 query heads (head_dim 64 or 128) or 4 (head_dim 128), one workgroup per
-// (row, KV head): the G query heads that share a KV head are computed together, so each K/V row
-// is loaded once per workgroup (whole 16-byte row segments) into LDS tiles of 128 positions
-// instead of once per head and lane. Per tile: thread (head h, slot u) scores positions u,
-// u + 256/G, ... (dot8 over the head dims in the same order as above), the G heads' f32 online
-// softmax runs over their 256/G-thread groups, and thread (h, dim pair) accumulates P V from LDS.
-constexpr int kAttTile = 128;
-template <int HD, int G>
-__global__ __launch_bounds__(kPThreads) void prefill_attention_tile_kernel(
-    const h16 *__restrict__ Q, const h16 *__restrict__ kc, const h16 *__restrict__ vc, h16 *__restrict__ out,
-    int64_t dim, int64_t kvd, int64_t p0, int64_t max_seq, float scale) {
-    constexpr int TPH = kPThreads / G;        // threads per head (32 or 64)
-    constexpr int NP = kAttTile / TPH;         // positions per thread per tile
-    constexpr int NDP = HD / 2 / TPH;          // dim pairs per thread
-    constexpr int KR = HD + 8;                 // padded K row (halves)
-    constexpr int CH = HD / 8;                 // 16-byte chunks per row
-    static_assert(NP >= 1 && NDP >= 1 && TPH <= kWave, "shape");
-    __shared__ __align__(16) h16 ks[kAttTile][KR];
-    __shared__ __align__(16) h16 vs[kAttTile][HD];
-    __shared__ float ps[G][kAttTile];
-    const int tid = threadIdx.x, h = tid / TPH, u = tid % TPH;
-    const int64_t r = blockIdx.x, g = blockIdx.y;
-    const int64_t pos = p0 + r;
-    const int64_t S = pos + 1 < max_seq ? pos + 1 : max_seq;
-    const int64_t head = g * G + h;
-    u32x4 qr[CH];
-    {
-        const h16 *q = Q + r * dim + head * HD;
-#pragma unroll
-        for (int c = 0; c < CH; c++) qr[c] = ld16(q + 8 * c);
-    }
-    const h16 *Kg = kc + g * HD, *Vg = vc + g * HD;
-    float m = -INFINITY, l = 0.0f, acc[NDP][2];
-#pragma unroll
-    for (int j = 0; j < NDP; j++) acc[j][0] = acc[j][1] = 0.0f;
-    for (int64_t t0 = 0; t0 < S; t0 += kAttTile) {
-        const int n = (int)(S - t0 < kAttTile ? S - t0 : kAttTile);
-        __syncthreads();  // the previous tile's K, V and P are no longer read
-        for (int e = tid; e < kAttTile * CH; e += kPThreads) {
-            const int row = e / CH, c = e % CH;
-            const int64_t p = t0 + (row < n ? row : 0);
-            st16(&ks[row][8 * c], ld16(Kg + p * kvd + 8 * c));
-            st16(&vs[row][8 * c], ld16(Vg + p * kvd + 8 * c));
-        }
-        __syncthreads();
-        float sc[NP];
-        float mt = -INFINITY;
-#pragma unroll
-        for (int j = 0; j < NP; j++) {
-            const int row = u + j * TPH;
-            float d = 0.0f;
-#pragma unroll
-            for (int c = 0; c < CH; c++) d = dot8(ld16(&ks[row][8 * c]), qr[c], d);
-            sc[j] = row < n ? d * scale : -INFINITY;
-            mt = fmaxf(mt, sc[j]);
-        }
-        mt = group_max<TPH>(mt);
-        const float mn = fmaxf(m, mt);
-        float lt = 0.0f;
-#pragma unroll
-        for (int j = 0; j < NP; j++) {
-            const float pr = u + j * TPH < n ? expf(sc[j] - mn) : 0.0f;
-            ps[h][u + j * TPH] = pr;
-            lt += pr;
-        }
-        lt = group_sum<TPH>(lt);
-        const float al = expf(m - mn);  // 0 on the first tile
-        l = l * al + lt;
-        m = mn;
-        __syncthreads();
-#pragma unroll
-        for (int j = 0; j < NDP; j++) {
-            const int dp = 2 * (u + j * TPH);
-            float a0 = acc[j][0] * al, a1 = acc[j][1] * al;
-            for (int t = 0; t < n; t++) {
-                const float pr = ps[h][t];
-                const h16x2 v = *reinterpret_cast<const h16x2 *>(&vs[t][dp]);
-                a0 = fmaf(pr, (float)v.x, a0);
-                a1 = fmaf(pr, (float)v.y, a1);
-            }
-            acc[j][0] = a0;
-            acc[j][1] = a1;
-        }
-    }
-    h16 *o = out + r * dim + head * HD;
-#pragma unroll
-    for (int j = 0; j < NDP; j++) {
-        const int dp = 2 * (u + j * TPH);
-        o[dp] = (h16)(acc[j][0] / l);
-        o[dp + 1] = (h16)(acc[j][1] / l);
-    }
-}
-
-// The same causal attention on the matrix cores, for chunks of many rows (no ring wrap inside the
-// chunk). A 512-thread workgroup owns BQ = 128 / G consecutive rows and one KV head; wave w takes
-// query head g G + w / (BQ / 16) on rows 16 (w % (BQ / 16)) .. + 15 of the block, so the 8 waves
-// share every K/V tile of 64 keys, which the workgroup stages in LDS (the next tile's rows are
-// requested into registers while the current one is used). Per tile and wave:
+// The same causal attention on the matrix cores (no ring wrap inside the chunk: prefill positions
+// never pass the context length). A workgroup owns RB = WV / G blocks of 16 consecutive rows and one
+// KV head; in each of its KS key groups of WV waves, wave w takes query head g G + w / RB on row block
+// w % RB, so the group's waves share every K/V tile of 64 keys, which the group stages in LDS (the
+// next tile's rows are requested into registers while the current one is used). Key group kg takes
+// every KS-th tile. Per tile and wave:
 //   scores  S^T[64 keys][16 queries] = K Q^T on v_mfma_f32_16x16x32_f16 (A = K rows from LDS,
 //           B = the wave's 16 query rows, held in registers): lane l holds query l % 16 and keys
-//           16 t + 4 (l / 16) + i of sub-tile t; keys past a row's position are masked
-//   softmax f32 online softmax per query: the lane's 16 values, then lanes l ^ 16, l ^ 32
-//           (permlane swaps)
+//           16 t + 4 (l / 16) + i of sub-tile t; keys past a row's position are masked (only in the
+//           tiles that hold such a key)
+//   softmax f32 online softmax per query in base 2 (scores times scale log2 e): the lane's 16
+//           values, then lanes l ^ 16, l ^ 32 (permlane swaps)
 //   P V     O[16 queries][16 dims] += P V per 32-key step, A = the probabilities as they sit in
 //           the score registers (slot 4 t + i of lane group q is key 16 t + 4 q + i), split into
 //           two f16 terms (hi = f16(p), lo = f16(p - hi)) so that they keep f32 precision; B = V
 //           read transposed from LDS with ds_read_b64_tr_b16 (V chunk c of row m at slot
 //           c ^ 2 ((m / RPS) & SWM), which spreads the transposed reads over the banks)
-// A tile entirely past a wave's last row is skipped by that wave. Scores and sums are f32, as in
-// prefill_attention_tile_kernel; only the accumulation order differs.
+// A tile entirely past a wave's last row is skipped by that wave. The key groups meet in LDS at the
+// end. With gridDim.z > 1 each z takes a contiguous share of the tiles and leaves (m, l, O) in f32
+// for prefill_attention_merge_kernel: short chunks after a long history, whose row blocks alone
+// leave most of the chip idle. Row blocks are dispatched last first: the last rows see the most
+// keys, so the long workgroups start first and the short ones fill in behind them.
+// Bound: the serial phases of a round (scores, softmax, P V between two barriers) with two waves per
+// SIMD. Measured on MI355X, us per layer: 1024 rows at the Llama-3 shape 52 -> 36 (8-wave workgroups
+// of 32 rows without key groups before, in ascending row order); 37 rows after 500 positions 33 -> 14
+// with the merge (one workgroup per row and KV head, scalar P V before); 128 rows at the TinyLlama
+// shape 7.1 -> 7.4 (too few tiles to split). That per-row kernel is gone with the shapes it served.
 typedef short short4_t __attribute__((ext_vector_type(4)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
 constexpr int kPfBK = 64;            // keys per tile
-constexpr int kPfWaves = 8;
-constexpr int64_t kPfMfmaMinRows = 256;  // chunks from here on use the matrix-core attention
-// Groups of 8 waves splitting a row block's key tiles (head_dim 64; at head_dim 128 the 1024-thread
-// workgroup's 128-VGPR budget spills, so one group).
-constexpr int kPfKeyGroups = 2;
-template <int HD, int G, int KS>
-__global__ __launch_bounds__(KS * kPfWaves * kWave) void prefill_attention_mfma_kernel(
+template <int HD, int G, int WV, int KS>
+__global__ __launch_bounds__(KS *WV *kWave) void prefill_attention_mfma_kernel(
     const h16 *__restrict__ Q, const h16 *__restrict__ kc, const h16 *__restrict__ vc, h16 *__restrict__ out,
-    int64_t n, int64_t dim, int64_t kvd, int64_t p0, float scale) {
-    constexpr int BQ = 16 * kPfWaves / G;  // rows per workgroup
-    constexpr int RBLK = BQ / 16;          // 16-row blocks per head
+    int64_t n, int64_t dim, int64_t kvd, int64_t p0, float scale2, float *__restrict__ part) {
+    constexpr int RB = WV / G;             // 16-row blocks per workgroup
+    constexpr int BQ = 16 * RB;            // rows per workgroup
     constexpr int NJ = HD / 32;            // score k-steps
     constexpr int NT = HD / 16;            // O dim tiles
     constexpr int KR = HD + 8;             // padded K row (halves)
-    constexpr int RB = HD * 2;             // V row bytes
-    constexpr int RPS = 256 / RB;          // V rows per 256 LDS bytes
-    constexpr int SWM = RB / 32 - 1;
+    constexpr int VB = HD * 2;             // V row bytes
+    constexpr int RPS = 256 / VB;          // V rows per 256 LDS bytes
+    constexpr int SWM = VB / 32 - 1;
     constexpr int CH = HD / 8;             // 16-byte chunks per row
-    constexpr int GT = kPfWaves * kWave;   // threads of a key group
+    constexpr int GT = WV * kWave;         // threads of a key group
     constexpr int NLD = kPfBK * CH / GT;   // K (and V) chunks per thread per tile
     constexpr int KB = kPfBK * KR * 2;     // K tile bytes (padded rows)
-    constexpr int TB = KB + kPfBK * RB;    // K + V tile bytes of a key group
-    static_assert(RBLK * G == kPfWaves && NLD >= 1 && NLD * GT == kPfBK * CH, "shape");
-    static_assert(KS == 1 || kPfWaves * kWave * NT * 16 <= KS * TB, "the second group's O fits the tiles' LDS");
+    constexpr int TB = KB + kPfBK * VB;    // K + V tile bytes of a key group
+    static_assert(RB * G == WV && NLD >= 1 && NLD * GT == kPfBK * CH, "shape");
+    static_assert(KS == 1 || KS == 2, "one exchange of the second key group");
+    static_assert(KS == 1 || WV * (kWave * NT * 16 + 32 * 4) <= KS * TB, "the second group's O fits the tiles' LDS");
     __shared__ __align__(16) uint8_t smem[KS * TB];
     const int tid = threadIdx.x, lane = tid & 63;
     const int kg = tid / GT, gt = tid % GT, wave = gt >> 6;  // key group, thread and wave in it
     uint8_t *kbase = smem + kg * TB, *vs = kbase + KB;
     auto ks = [&](int row, int col) -> h16 * { return reinterpret_cast<h16 *>(kbase) + row * KR + col; };
     const int q4 = lane >> 4, c16 = lane & 15;
-    const int64_t g = blockIdx.y;
-    const int64_t rb0 = (int64_t)blockIdx.x * BQ;                 // first row of the workgroup
+    const int64_t g = blockIdx.x;
+    const int64_t rb0 = (int64_t)(gridDim.y - 1 - blockIdx.y) * BQ;  // first row of the workgroup
     const int64_t rlast = (rb0 + BQ < n ? rb0 + BQ : n) - 1;      // last valid row
     const int64_t kend = p0 + rlast + 1;                          // keys of the workgroup
-    const int64_t ntile = (kend + kPfBK - 1) / kPfBK;
-    const int64_t niter = (ntile + KS - 1) / KS;                  // tile rounds (group kg: tiles KS it + kg)
-    const int hw = wave / RBLK;
-    const int64_t r0w = rb0 + 16 * (wave % RBLK);                 // first row of the wave
+    const int ntile = (int)((kend + kPfBK - 1) / kPfBK), Z = gridDim.z, z = blockIdx.z;
+    const int per = (ntile + Z - 1) / Z, tl0 = z * per;
+    const int tl1 = tl0 + per < ntile ? tl0 + per : ntile;
+    const int niter = tl1 > tl0 ? (tl1 - tl0 + KS - 1) / KS : 0;  // tile rounds (group kg: tiles tl0 + KS it + kg)
+    const int hw = wave / RB;
+    const int64_t r0w = rb0 + 16 * (wave % RB);                   // first row of the wave
     const int64_t rmax_w = r0w + 15 < rlast ? r0w + 15 : rlast;   // last valid row of the wave
-    const int64_t head = g * G + hw;
+    const int64_t head = g * G + hw, nq = dim / HD;
     // this lane's query row (rows past the chunk are clamped: computed, never stored)
     const int64_t rq = r0w + c16 < rlast ? r0w + c16 : rlast;
-    const int64_t kq = p0 + rq;  // last key the query sees
+    const int kq = (int)(p0 + rq);  // last key the query sees
     u32x4 qb[NJ];
     {
         const h16 *qp = Q + rq * dim + head * HD + 8 * q4;
@@ -1219,11 +1135,11 @@ __global__ __launch_bounds__(KS * kPfWaves * kWave) void prefill_attention_mfma_
     }
     const h16 *Kg = kc + g * HD, *Vg = vc + g * HD;
     u32x4 kr[NLD], vr[NLD];
-    auto load_tile = [&](int64_t t0) {  // rows past the workgroup's keys re-read its last key
+    auto load_tile = [&](int t0) {  // rows past the workgroup's keys re-read its last key
 #pragma unroll
         for (int i = 0; i < NLD; i++) {
             const int e = gt + i * GT, row = e / CH, c = e % CH;
-            const int64_t p = t0 + row < kend ? t0 + row : kend - 1;
+            const int64_t p = t0 + row < (int)kend ? t0 + row : kend - 1;
             kr[i] = ld16(Kg + p * kvd + 8 * c);
             vr[i] = ld16(Vg + p * kvd + 8 * c);
         }
@@ -1233,25 +1149,26 @@ __global__ __launch_bounds__(KS * kPfWaves * kWave) void prefill_attention_mfma_
         const int c = 2 * nt + ((lane & 3) >> 1);
         const int sl = c ^ (2 * ((m / RPS) & SWM));
         return __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-                                             (__attribute__((address_space(3))) short4_t *)(vs + m * RB + 16 * sl + 8 * (lane & 1))));
+                                             (__attribute__((address_space(3))) short4_t *)(vs + m * VB + 16 * sl + 8 * (lane & 1))));
     };
     float m_run = -INFINITY, l_run = 0.0f;  // query c16 (the same in the four lane groups)
     f32x4 o[NT];
 #pragma unroll
     for (int t = 0; t < NT; t++) o[t] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-    load_tile((int64_t)kg * kPfBK);
-    for (int64_t it = 0; it < niter; it++) {
-        const int64_t t0 = (it * KS + kg) * kPfBK;  // past kend: a surplus round of this group
+    if (niter > 0) load_tile((tl0 + kg) * kPfBK);
+    for (int it = 0; it < niter; it++) {
+        const int tile = tl0 + it * KS + kg, t0 = tile * kPfBK;
         __syncthreads();  // the previous tiles are no longer read
 #pragma unroll
         for (int i = 0; i < NLD; i++) {
             const int e = gt + i * GT, row = e / CH, c = e % CH;
             st16(ks(row, 8 * c), kr[i]);
-            st16(vs + row * RB + 16 * (c ^ (2 * ((row / RPS) & SWM))), vr[i]);
+            st16(vs + row * VB + 16 * (c ^ (2 * ((row / RPS) & SWM))), vr[i]);
         }
         __syncthreads();
         if (it + 1 < niter) load_tile(t0 + KS * kPfBK);
-        if (t0 > p0 + rmax_w) continue;  // every key of the tile is past this wave's rows
+        // a surplus round of this group, or every key of the tile past this wave's rows
+        if (tile >= tl1 || t0 > (int)(p0 + rmax_w)) continue;
         f32x4 st[4];
 #pragma unroll
         for (int t = 0; t < 4; t++) {
@@ -1260,51 +1177,64 @@ __global__ __launch_bounds__(KS * kPfWaves * kWave) void prefill_attention_mfma_
             for (int j = 0; j < NJ; j++) st[t] = mfma16x16x32(ld16(ks(16 * t + c16, 32 * j + 8 * q4)), qb[j], st[t]);
         }
         float sv[4][4], mx = -INFINITY;
+        if (t0 + kPfBK - 1 <= (int)(p0 + r0w)) {  // every row of the wave sees the whole tile
 #pragma unroll
-        for (int t = 0; t < 4; t++)
+            for (int t = 0; t < 4; t++)
 #pragma unroll
-            for (int i = 0; i < 4; i++) {
-                const int64_t key = t0 + 16 * t + 4 * q4 + i;
-                sv[t][i] = key <= kq ? st[t][i] * scale : -INFINITY;
-                mx = fmaxf(mx, sv[t][i]);
-            }
+                for (int i = 0; i < 4; i++) {
+                    sv[t][i] = st[t][i] * scale2;
+                    mx = fmaxf(mx, sv[t][i]);
+                }
+        } else {
+#pragma unroll
+            for (int t = 0; t < 4; t++)
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    sv[t][i] = t0 + 16 * t + 4 * q4 + i <= kq ? st[t][i] * scale2 : -INFINITY;
+                    mx = fmaxf(mx, sv[t][i]);
+                }
+        }
         mx = swap_pair_max<32>(swap_pair_max<16>(mx));
-        // the tile holds a key the query sees (t0 <= p0 + rq for every row of the wave but
-        // clamped rows past the chunk, which are never stored), so mx is finite
-        const float mn = fmaxf(m_run, mx);
-        const float al = expf(m_run - mn);   // 0 on the group's first tile
+        const bool grows = mx > m_run;
+        if (__builtin_amdgcn_ballot_w64(grows) != 0) {  // some query's maximum moves: rescale l and O
+            const float mn = fmaxf(m_run, mx);
+            const float al = grows ? __builtin_amdgcn_exp2f(m_run - mn) : 1.0f;  // 0 on the query's first keys
+            l_run *= al;
+            m_run = mn;
+            // O rows of this lane are queries 4 q4 + i, whose factor sits in lane 4 q4 + i
+            float alr[4];
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+                alr[i] = __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute(4 * (4 * q4 + i), __builtin_bit_cast(int, al)));
+#pragma unroll
+            for (int nt = 0; nt < NT; nt++)
+#pragma unroll
+                for (int i = 0; i < 4; i++) o[nt][i] *= alr[i];
+        }
+        // a query without a key in this tile and before it has m_run = -inf: every p is then 0
+        const float mref = m_run == -INFINITY ? 0.0f : m_run;
         float ps = 0.0f;
         u32x4 ph[2], pl[2];  // k-steps: keys of sub-tiles 2 kk and 2 kk + 1
 #pragma unroll
-        for (int kk = 0; kk < 2; kk++) {
-            h16 hi[8], lo[8];
+        for (int kk = 0; kk < 2; kk++)
 #pragma unroll
             for (int t = 0; t < 2; t++)
 #pragma unroll
-                for (int i = 0; i < 4; i++) {
-                    const float p = expf(sv[2 * kk + t][i] - mn);  // 0 where masked
-                    ps += p;
-                    hi[4 * t + i] = (h16)p;
-                    lo[4 * t + i] = (h16)(p - (float)hi[4 * t + i]);
+                for (int i = 0; i < 4; i += 2) {
+                    const f32x2 p = {__builtin_amdgcn_exp2f(sv[2 * kk + t][i] - mref),
+                                     __builtin_amdgcn_exp2f(sv[2 * kk + t][i + 1] - mref)};  // 0 where masked
+                    ps += p.x;
+                    ps += p.y;
+                    const h16x2 hi = __builtin_convertvector(p, h16x2);
+                    const f32x2 r = {p.x - (float)hi.x, p.y - (float)hi.y};
+                    ph[kk][2 * t + i / 2] = h2_bits(hi);
+                    pl[kk][2 * t + i / 2] = h2_bits(__builtin_convertvector(r, h16x2));
                 }
-            ph[kk] = u32x4{h2_bits(h16x2{hi[0], hi[1]}), h2_bits(h16x2{hi[2], hi[3]}), h2_bits(h16x2{hi[4], hi[5]}),
-                           h2_bits(h16x2{hi[6], hi[7]})};
-            pl[kk] = u32x4{h2_bits(h16x2{lo[0], lo[1]}), h2_bits(h16x2{lo[2], lo[3]}), h2_bits(h16x2{lo[4], lo[5]}),
-                           h2_bits(h16x2{lo[6], lo[7]})};
-        }
         ps = swap_pair_sum<16>(ps, ps);
         ps = swap_pair_sum<32>(ps, ps);
-        l_run = l_run * al + ps;
-        m_run = mn;
-        // O rows of this lane are queries 4 q4 + i, whose factor sits in lane 4 q4 + i
-        float alr[4];
+        l_run += ps;
 #pragma unroll
-        for (int i = 0; i < 4; i++)
-            alr[i] = __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute(4 * (4 * q4 + i), __builtin_bit_cast(int, al)));
-#pragma unroll
-        for (int nt = 0; nt < NT; nt++) {
-#pragma unroll
-            for (int i = 0; i < 4; i++) o[nt][i] *= alr[i];
+        for (int nt = 0; nt < NT; nt++)
 #pragma unroll
             for (int kk = 0; kk < 2; kk++) {
                 const u32x2 v0 = read_vt(nt, 32 * kk), v1 = read_vt(nt, 32 * kk + 16);
@@ -1312,15 +1242,18 @@ __global__ __launch_bounds__(KS * kPfWaves * kWave) void prefill_attention_mfma_
                 o[nt] = mfma16x16x32(ph[kk], vb, o[nt]);
                 o[nt] = mfma16x16x32(pl[kk], vb, o[nt]);
             }
-        }
     }
+    auto spread = [&](float v, float(&r)[4]) {  // r[i]: v of query 4 q4 + i
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+            r[i] = __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute(4 * (4 * q4 + i), __builtin_bit_cast(int, v)));
+    };
     if constexpr (KS == 2) {
         // group 1 hands (m, l, O) to the group-0 wave of the same rows and head through the tiles'
-        // LDS: w = exp(m_g - max m) per query, l = sum w l_g, O = sum w O_g
+        // LDS: w = 2^(m_g - max m) per query, l = sum w l_g, O = sum w O_g
         __syncthreads();  // every tile read is done
         f32x4 *ox = reinterpret_cast<f32x4 *>(smem);           // [wave][nt][lane]
-        float *mx1 = reinterpret_cast<float *>(smem + kPfWaves * kWave * NT * 16);  // [wave][m: 16, l: 16]
-        static_assert(kPfWaves * (kWave * NT * 16 + 32 * 4) <= KS * TB, "exchange fits");
+        float *mx1 = reinterpret_cast<float *>(smem + WV * kWave * NT * 16);  // [wave][m: 16, l: 16]
         if (kg == 1) {
 #pragma unroll
             for (int nt = 0; nt < NT; nt++) ox[(wave * NT + nt) * kWave + lane] = o[nt];
@@ -1332,15 +1265,13 @@ __global__ __launch_bounds__(KS * kPfWaves * kWave) void prefill_attention_mfma_
         __syncthreads();
         if (kg == 1) return;
         const float m1 = mx1[wave * 32 + c16], l1 = mx1[wave * 32 + 16 + c16];
-        const float M = fmaxf(m_run, m1);   // m_run finite: group 0 holds tile 0
-        const float e0 = expf(m_run - M), e1 = expf(m1 - M);  // e1 = 0 for a group without tiles
+        const float M = fmaxf(m_run, m1), mref = M == -INFINITY ? 0.0f : M;
+        const float e0 = __builtin_amdgcn_exp2f(m_run - mref), e1 = __builtin_amdgcn_exp2f(m1 - mref);  // 0 for a group without keys
         l_run = l_run * e0 + l1 * e1;
+        m_run = M;
         float e0r[4], e1r[4];
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            e0r[i] = __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute(4 * (4 * q4 + i), __builtin_bit_cast(int, e0)));
-            e1r[i] = __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute(4 * (4 * q4 + i), __builtin_bit_cast(int, e1)));
-        }
+        spread(e0, e0r);
+        spread(e1, e1r);
 #pragma unroll
         for (int nt = 0; nt < NT; nt++) {
             const f32x4 b = ox[(wave * NT + nt) * kWave + lane];
@@ -1348,10 +1279,22 @@ __global__ __launch_bounds__(KS * kPfWaves * kWave) void prefill_attention_mfma_
             for (int i = 0; i < 4; i++) o[nt][i] = o[nt][i] * e0r[i] + b[i] * e1r[i];
         }
     }
-    float lr[4];
+    if (Z > 1) {  // partial z: O [Z][n][nq][HD], then (m, l) [Z][n][nq][2]
+        float *ml = part + (int64_t)Z * n * nq * HD;
+        if (q4 == 0 && r0w + c16 <= rlast)
+            *reinterpret_cast<float2 *>(ml + ((z * n + r0w + c16) * nq + head) * 2) = float2{m_run, l_run};
 #pragma unroll
-    for (int i = 0; i < 4; i++)
-        lr[i] = __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute(4 * (4 * q4 + i), __builtin_bit_cast(int, l_run)));
+        for (int i = 0; i < 4; i++) {
+            const int64_t r = r0w + 4 * q4 + i;
+            if (r > rlast) continue;
+            float *orow = part + ((z * n + r) * nq + head) * HD + c16;
+#pragma unroll
+            for (int nt = 0; nt < NT; nt++) orow[16 * nt] = o[nt][i];
+        }
+        return;
+    }
+    float lr[4];
+    spread(l_run, lr);
 #pragma unroll
     for (int i = 0; i < 4; i++) {
         const int64_t r = r0w + 4 * q4 + i;
@@ -1362,17 +1305,66 @@ __global__ __launch_bounds__(KS * kPfWaves * kWave) void prefill_attention_mfma_
     }
 }
 
+// out = f16(sum_z w_z O_z / sum_z w_z l_z), w_z = 2^(m_z - max m): one thread per 4 dims of a row's
+// head. A part without keys has m = -inf: its w is 0 and its O finite (0). The first part always
+// holds key 0, so max m is finite.
+__global__ __launch_bounds__(kPThreads) void prefill_attention_merge_kernel(const float *__restrict__ part, int Z,
+                                                                            int64_t n, int64_t nq, int hd,
+                                                                            h16 *__restrict__ out) {
+    const int64_t i = ((int64_t)blockIdx.x * kPThreads + threadIdx.x) * 4;  // element of [n][nq][hd]
+    const int64_t total = n * nq * hd;
+    if (i >= total) return;
+    const int64_t rh = i / hd;
+    const float *ml = part + Z * total;
+    float M = -INFINITY;
+    for (int z = 0; z < Z; z++) M = fmaxf(M, ml[(z * n * nq + rh) * 2]);
+    float L = 0.0f;
+    f32x4 o = {0.0f, 0.0f, 0.0f, 0.0f};
+    for (int z = 0; z < Z; z++) {
+        const float2 p = *reinterpret_cast<const float2 *>(ml + (z * n * nq + rh) * 2);
+        const float w = __builtin_amdgcn_exp2f(p.x - M);
+        const f32x4 v = *reinterpret_cast<const f32x4 *>(part + z * total + i);
+        L = fmaf(w, p.y, L);
+#pragma unroll
+        for (int e = 0; e < 4; e++) o[e] = fmaf(w, v[e], o[e]);
+    }
+#pragma unroll
+    for (int e = 0; e < 4; e++) out[i + e] = (h16)(o[e] / L);
+}
+
+// Shares of the key tiles over grid.z: enough that the workgroups reach about two per CU, each with
+// at least one tile per key group, at most 16.
+static int64_t pf_key_splits(int64_t wgs, int64_t tiles, int64_t key_groups) {
+    int64_t z = 256 / wgs;
+    if (z > tiles / key_groups) z = tiles / key_groups;
+    return z < 1 ? 1 : z > 16 ? 16 : z;
+}
+
 // Launches prefill_attention_mfma_kernel for the shapes it is instantiated for;
-// AESIR_ERR_UNSUPPORTED otherwise (the caller takes the tile kernels).
-static int32_t launch_prefill_attention_mfma(hipStream_t s, int64_t hd, int64_t G, const h16 *Q, const h16 *kc,
+// AESIR_ERR_UNSUPPORTED otherwise (the caller takes the per-row kernel).
+static int32_t launch_prefill_attention_mfma(aesir_ctx *ctx, int64_t hd, int64_t G, const h16 *Q, const h16 *kc,
                                              const h16 *vc, h16 *out, int64_t n, int64_t dim, int64_t kvd, int64_t p0,
                                              int64_t nkv, float scale) {
+    hipStream_t s = ctx->stream;
+    if (p0 + n >= ((int64_t)1 << 31) - kPfBK) return AESIR_ERR_UNSUPPORTED;
+    const float scale2 = (float)((double)scale * 1.4426950408889634);  // log2 e
 #define AESIR_PF_MMA(HDV, GV)                                                                                   \
     if (hd == HDV && G == GV) {                                                                                \
-        constexpr int BQ = 16 * kPfWaves / GV, KS = HDV == 64 ? kPfKeyGroups : 1;                              \
-        hipLaunchKernelGGL((prefill_attention_mfma_kernel<HDV, GV, KS>), dim3((unsigned)((n + BQ - 1) / BQ), (unsigned)nkv), \
-                           dim3(KS * kPfWaves * kWave), 0, s, Q, kc, vc, out, n, dim, kvd, p0, scale);         \
+        constexpr int WV = GV > 4 ? GV : 4, KS = HDV == 128 && GV == 8 ? 1 : 2; /* (1024 threads spill there) */ \
+        const int64_t nrb = (n + 16 * (WV / GV) - 1) / (16 * (WV / GV)), wgs = nrb * nkv;                      \
+        if (nrb > 65535) return AESIR_ERR_UNSUPPORTED;                                                         \
+        int64_t Z = pf_key_splits(wgs, (p0 + n + kPfBK - 1) / kPfBK, KS);                                      \
+        while (Z > 1 && Z * n * dim / HDV * (HDV + 2) > ctx->scratch.attn_part_floats) Z--;                    \
+        hipLaunchKernelGGL((prefill_attention_mfma_kernel<HDV, GV, WV, KS>),                                   \
+                           dim3((unsigned)nkv, (unsigned)nrb, (unsigned)Z), dim3(KS * WV * kWave), 0, s, Q, kc, \
+                           vc, out, n, dim, kvd, p0, scale2, ctx->scratch.attn_part);                          \
         AESIR_LAUNCH_CHECK("prefill_attention_mfma_kernel");                                                   \
+        if (Z > 1) {                                                                                           \
+            hipLaunchKernelGGL(prefill_attention_merge_kernel, dim3((unsigned)((n * dim / 4 + kPThreads - 1) / kPThreads)), \
+                               dim3(kPThreads), 0, s, (const float *)ctx->scratch.attn_part, (int)Z, n, dim / HDV, \
+                               (int)HDV, out);                                                                 \
+            AESIR_LAUNCH_CHECK("prefill_attention_merge_kernel");                                              \
+        }                                                                                                      \
         return AESIR_OK;                                                                                       \
     }
     AESIR_PF_MMA(64, 8)
@@ -1548,24 +1540,11 @@ static int32_t prefill_chunk(aesir_model *m, const int64_t *tokens_host, int64_t
             AESIR_LAUNCH_CHECK("qkv_post_rows_kernel");
         }
         const int64_t G = c.n_heads / c.n_kv_heads;
-        const dim3 tgrid((unsigned)n, (unsigned)c.n_kv_heads);
-        bool att_done = false;
-        if (n >= kPfMfmaMinRows && p0 + n <= c.ctx_len) {  // long chunk without ring wrap: matrix cores
-            const int32_t rc = launch_prefill_attention_mfma(s, hd, G, Q, kc, vc, ATT, n, d, kvd, p0, c.n_kv_heads,
-                                                             m->attn_scale);
-            if (rc == AESIR_OK) att_done = true;
-            else if (rc != AESIR_ERR_UNSUPPORTED) return rc;
-        }
-        if (!att_done) {
-#define AESIR_PF_ATT(HDV, GV)                                                                                      \
-    if (hd == HDV && G == GV)                                                                                     \
-        hipLaunchKernelGGL((prefill_attention_tile_kernel<HDV, GV>), tgrid, dim3(kPThreads), 0, s, Q, kc, vc, ATT, d, \
-                           kvd, p0, c.ctx_len, m->attn_scale);                                                   \
-    else
-            AESIR_PF_ATT(64, 8)
-            AESIR_PF_ATT(128, 8)
-            AESIR_PF_ATT(128, 4)
-#undef AESIR_PF_ATT
+        int32_t arc = AESIR_ERR_UNSUPPORTED;
+        if (p0 + n <= c.ctx_len)  // no ring wrap inside the chunk: matrix cores
+            arc = launch_prefill_attention_mfma(m->ctx, hd, G, Q, kc, vc, ATT, n, d, kvd, p0, c.n_kv_heads, m->attn_scale);
+        if (arc != AESIR_OK && arc != AESIR_ERR_UNSUPPORTED) return arc;
+        if (arc == AESIR_ERR_UNSUPPORTED) {
             if (hd % 8 == 0)  // rows of K are then 16-byte aligned (kvd and the cache base are)
                 hipLaunchKernelGGL(prefill_attention_kernel<true>, dim3((unsigned)n, (unsigned)c.n_heads), dim3(kWave), 0,
                                    s, Q, kc, vc, ATT, d, kvd, hd, c.n_heads / c.n_kv_heads, p0, c.ctx_len, m->attn_scale);
