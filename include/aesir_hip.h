@@ -207,12 +207,12 @@ int32_t aesir_gemm_q8_0(aesir_ctx *ctx, const void *A, int64_t a_rows, int64_t a
  * rounding; Q4_K, Q5_K, Q2_K) and w = f16(f16(d * sc) * q) (Q6_K with q - 32, Q3_K with its signed
  * q) (the reference's K-quant gemms read synthetic block layouts that no GGUF file holds). Raises
  * "gemm_q4_0: matrix dimensions must be positive", "...: inner dimension must be a multiple of
- * 32" (256 for the K-quants), "...: output matrix shape mismatch". Takes free well space for the
- * duration of the call: with a_rows < 16 and a_cols a multiple of 128 (at most 28672), or with
- * a_rows > 64 and a_cols a multiple of 128, the blocks are repacked into the library's tiled
- * planes (about the size of the blocks) for the decode GEMV per row or the matrix-core GEMM that
- * dequantizes in registers; otherwise an f16 copy of the weights (2 bytes per weight) for the F16
- * GEMM. */
+ * 32" (256 for the K-quants), "...: output matrix shape mismatch". Up to 64 rows of A with
+ * a_cols a multiple of 128 (A 16-byte, blocks 2-byte aligned) the blocks are multiplied as they lie.
+ * Other calls take free well space for their duration: with a_rows > 64 and a_cols a multiple of 128
+ * the blocks are repacked into the library's tiled planes (about the size of the blocks) for the
+ * matrix-core GEMM that dequantizes in registers; otherwise an f16 copy of the weights (2 bytes per
+ * weight) is made for the F16 GEMM. */
 int32_t aesir_gemm_quant(aesir_ctx *ctx, const void *A, int64_t a_rows, int64_t a_cols, const void *blocks,
                          int32_t ggml_type, int64_t b_rows, void *C, int64_t c_rows, int64_t c_cols);
 /* Q8_0 block matvec with f32 activations and f32 output: y[n] = sum_k x[k] * d*q. Rows of

@@ -213,6 +213,9 @@ int32_t aesir_gemm_q8_0(aesir_ctx *ctx, const void *A, int64_t a_rows, int64_t a
     if (a_cols % 32 != 0) return fail(AESIR_ERR_SHAPE, "gemm_q8_0: inner dimension must be a multiple of 32");
     if (c_rows != a_rows || c_cols != b_rows) return fail(AESIR_ERR_SHAPE, "gemm_q8_0: output matrix shape mismatch");
     if (!A || !blocks || !C) return fail(AESIR_ERR_INVALID, "gemm_q8_0: null tensor pointer");
+    // more rows than one: the blocks meet up to 64 rows per read (the GEMV reads them once per row)
+    if (a_rows >= 2 && gemm_raw_ok(A, a_cols, blocks, AESIR_GGML_Q8_0, b_rows))
+        return launch_gemm_raw(ctx, A, a_rows, a_cols, blocks, AESIR_GGML_Q8_0, b_rows, C);
     return launch_gemm_q8_0(ctx->stream, A, a_rows, a_cols, blocks, b_rows, C);
 }
 
@@ -244,20 +247,19 @@ int32_t aesir_gemm_quant(aesir_ctx *ctx, const void *A, int64_t a_rows, int64_t 
         return fail(AESIR_ERR_SHAPE, "%s: inner dimension must be a multiple of %lld", nm, (long long)blk);
     if (c_rows != a_rows || c_cols != b_rows) return fail(AESIR_ERR_SHAPE, "%s: output matrix shape mismatch", nm);
     if (!A || !blocks || !C) return fail(AESIR_ERR_INVALID, "%s: null tensor pointer", nm);
-    // Fewer than 16 rows of A on whole 128-weight segments of a repacked type: the blocks are
-    // repacked into the tiled planes and each row runs the decode GEMV; more than 64 rows on whole
-    // 128-weight segments: the same planes on the wide-tile matrix-core GEMM, which dequantizes
-    // them in registers. Otherwise the blocks are dequantized to f16 (the same values) for the F16
-    // GEMM, on the matrix cores from 2 rows. Both take free well space for this call, released after enqueueing (later work on the
-    // stream runs after these kernels).
-    // Both repacked-plane routes read A with 16-byte loads (the GEMV stages x with them, the wide
-    // kernel copies A into LDS with them): an A that is not 16-byte aligned (an offset view) takes
-    // the dequantize-then-F16 route, which checks its own alignment.
+    // Up to 64 rows of A on whole 128-weight segments: the short-chunk GEMM reads the blocks as they lie.
+    if (a_rows <= kSkinnyMaxRows && gemm_raw_ok(A, a_cols, blocks, ggml_type, b_rows))
+        return launch_gemm_raw(ctx, A, a_rows, a_cols, blocks, ggml_type, b_rows, C);
+    // More rows on whole 128-weight segments of a repacked type: the blocks are repacked into the
+    // tiled planes for the wide-tile matrix-core GEMM, which dequantizes them in registers (it copies A
+    // into LDS 16 bytes at a time; the repack reads whole 2-byte units). Otherwise, and for an A or
+    // blocks that are not so aligned, the blocks are dequantized to f16 (the same values) for the F16
+    // GEMM, on the matrix cores from 2 rows. Both take free well space for this call, released after
+    // enqueueing (later work on the stream runs after these kernels).
     const int64_t K = a_cols, N = b_rows, mark = ctx->well_offset;
     int32_t rc = AESIR_OK;
-    const bool a16 = ((uintptr_t)A & 15) == 0;
-    const bool wide = a16 && qf_type(ggml_type) && K % 128 == 0 && gemm_qf_wide_ok(a_rows, K, N);
-    if ((a16 && a_rows < 16 && qf_type(ggml_type) && qf_gemv_ok(K)) || wide) {
+    if (((uintptr_t)A & 15) == 0 && ((uintptr_t)blocks & 1) == 0 && qf_type(ggml_type) && K % 128 == 0 &&
+        gemm_qf_wide_ok(a_rows, K, N)) {
         QFMat w;
         w.type = ggml_type;
         void *planes[4] = {nullptr, nullptr, nullptr, nullptr};
@@ -270,9 +272,7 @@ int32_t aesir_gemm_quant(aesir_ctx *ctx, const void *A, int64_t a_rows, int64_t 
         w.s0 = planes[2];
         w.s1 = planes[3];
         if (rc == AESIR_OK) rc = launch_qf_repack(ctx->stream, ggml_type, blocks, N, K, w, 1);
-        if (wide && rc == AESIR_OK) rc = launch_gemm_qf_mfma(ctx, A, a_rows, K, w, N, C);
-        for (int64_t r = 0; !wide && r < a_rows && rc == AESIR_OK; r++)
-            rc = launch_qf_gemv_store(ctx->stream, w, N, K, (const uint16_t *)A + r * K, (uint16_t *)C + r * N);
+        if (rc == AESIR_OK) rc = launch_gemm_qf_mfma(ctx, A, a_rows, K, w, N, C);
     } else {
         void *wf = nullptr;
         rc = well_alloc_bytes(ctx, mul_checked(N, K, 2), &wf);

@@ -35,7 +35,7 @@ int32_t launch_gemm_f16_mfma(aesir_ctx *ctx, const void *A, int64_t M, int64_t K
 //        value q + 4, hmask bit included);
 //   hb   Q6_K: 4 bytes per record, the high 2 bits of the record's weights; Q5_0 / Q5_1 / Q5_K:
 //        4 bytes per record pair, the fifth bits of both records in one word (bit layout in
-//        quant.hip, qf_hb_pos);
+//        qf_tile.hpp, qf_hb_off);
 //   s0   Q4_0 / Q5_0: f16 d per 32 weights; Q4_1 / Q5_1: f16 d | f16 m << 16 per 32 weights;
 //        Q4_K / Q5_K: (scale, min) bytes per 32 weights, 6-bit values unpacked; Q6_K / Q3_K: int8
 //        scale per 16 weights; Q2_K: GGML's scale | min << 4 byte per 16 weights;
@@ -141,12 +141,19 @@ int32_t launch_qf_gemm_wide(hipStream_t s, int epi, int nt, const void *A, int64
 // Whether launch_gemm_qf_mfma takes an M x K by N x K product (more than 64 rows, K % 128 == 0,
 // 32-bit byte ranges), and that product stored as f16 C [M][N] (context stream and partials).
 bool gemm_qf_wide_ok(int64_t M, int64_t K, int64_t N);
+// C = f16(A W^T) for W as packed GGUF blocks (any block type of launch_gguf_dequant, K % 128 == 0, A
+// 16-byte and blocks 2-byte aligned) on the short-chunk GEMM, 64 rows at a time.
+bool gemm_raw_ok(const void *A, int64_t K, const void *blocks, int32_t type, int64_t N);
+int32_t launch_gemm_raw(aesir_ctx *ctx, const void *A, int64_t M, int64_t K, const void *blocks, int32_t type, int64_t N,
+                        void *C);
 int32_t launch_gemm_qf_mfma(aesir_ctx *ctx, const void *A, int64_t M, int64_t K, const QFMat &w, int64_t N, void *C);
 // Short-chunk GEMM (skinny.hip) of 1 to 64 activation rows on a matrix of any type, K % 128 == 0.
 // A weight matrix of N rows: f16 [N][K] (type F16: w), int8 quants [N][K] and f16 block scales
-// [N][K / 32] (Q8_0: w, s), 16-byte aligned, or the tiled planes of a repacked type (qf).
+// [N][K / 32] (Q8_0: w, s), 16-byte aligned, the tiled planes of a repacked type (qf), or the packed
+// GGUF blocks of a type (raw: w, 2-byte aligned).
 struct SkinnyMat {
     int32_t type = 0;
+    bool raw = false;
     const void *w = nullptr, *s = nullptr;
     QFMat qf;
 };
@@ -155,13 +162,15 @@ struct SkinnyPlan {
     int nw = 0;  // waves per workgroup; 0: the shape is not taken
     int64_t splits = 1;
 };
-SkinnyPlan skinny_plan(int64_t M, int64_t K, int64_t N, int32_t type, bool may_split);
+// kSplitFree: the caller's next kernel sums the partials anyway; kSplitPaid: a sum launch of its own.
+enum SkinnySplit : int { kSplitNone, kSplitFree, kSplitPaid };
+SkinnyPlan skinny_plan(int64_t M, int64_t K, int64_t N, int32_t type, SkinnySplit split, bool raw = false);
 // C = epilogue epi (GemmEpi) of A W^T, or with splits > 1 the f32 partials part[z][M][ldp] (columns
 // 0 .. N - 1 of rows of ldp).
 int32_t launch_gemm_skinny(hipStream_t s, int epi, const SkinnyMat &w, const void *A, int64_t M, int64_t K, int64_t N,
                            void *C, int64_t ldc, float *part, int64_t ldp, const SkinnyPlan &p);
-// y[n] = f16(sum_k x[k] w[n, k]) for one row of x (the per-op GEMV of a repacked matrix).
-int32_t launch_qf_gemv_store(hipStream_t s, const QFMat &w, int64_t N, int64_t K, const void *x, void *y);
+int32_t launch_gemm_skinny_raw(hipStream_t s, int epi, const SkinnyMat &w, const void *A, int64_t M, int64_t K, int64_t N,
+                               void *C, int64_t ldc, float *part, int64_t ldp, const SkinnyPlan &p);
 // Decode-step GEMVs of repacked matrices with the fused epilogues (see the F16 launchers).
 int32_t launch_qf_gemv_residual(hipStream_t s, const QFMat &w, int64_t N, int64_t K, const void *x_in, void *x);
 int32_t launch_qf_gate_up_swiglu(hipStream_t s, const void *x, const void *norm_w, float eps, const QFMat &w,

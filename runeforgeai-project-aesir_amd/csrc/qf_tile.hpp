@@ -63,11 +63,6 @@ __host__ __device__ __forceinline__ int qf_hb_off(int f) { return ((f & 1) << 1)
 // The 5-bit types keep a record pair's fifth bits in one word: the even record's at the low bit
 // of each Q6_K field position, the odd record's one above, so that shifting the word right by
 // the record's parity turns it into a Q6_K word whose fields hold only their low bit.
-// Bit position of the high 2 bits of record weight i.
-__host__ __device__ __forceinline__ int qf_hb_pos(int i) {
-    const int a = i & ~2, f = (a & 1) | (((a >> 2) & 1) << 1) | (((a >> 3) & 1) << 2);
-    return qf_hb_off(f) + 16 * ((i >> 1) & 1);
-}
 
 // ------------------------------------------------------------------ weight arithmetic
 

@@ -4,7 +4,7 @@
 #include "device.hpp"
 #include "kernels.hpp"
 #include "mfma_gemm.hpp"
-#include "skinny.hpp"
+#include "skinny_launch.hpp"
 
 namespace aesir {
 
@@ -18,12 +18,15 @@ namespace aesir {
 // 25.7, 24.1 / 15.6, 6.8 / 5.0 (f16 always takes 4: its own bytes outweigh the activations').
 constexpr int64_t kSkinnyWgTarget = 256;
 
-SkinnyPlan skinny_plan(int64_t M, int64_t K, int64_t N, int32_t type, bool may_split) {
+SkinnyPlan skinny_plan(int64_t M, int64_t K, int64_t N, int32_t type, SkinnySplit split, bool raw) {
     const int64_t lim = (int64_t)1 << 31;
     if (M < 1 || M > kSkinnyMaxRows || K % kSeg != 0 || K * M >= lim || N < 1 || N >= lim / 2) return {};
-    if (qf_type(type) && (K % gguf_block_elems(type) != 0 || mul_checked(qf_rows_alloc(N), K) >= lim)) return {};
+    if (!raw && qf_type(type) && (K % gguf_block_elems(type) != 0 || mul_checked(qf_rows_alloc(N), K) >= lim)) return {};
+    if (raw && K % gguf_block_elems(type) != 0) return {};
     SkinnyPlan p;
     const int64_t t8 = (N + 127) / 128;
+    // a sum launch costs more than it gains once 4-wave workgroups alone reach most CUs
+    const bool may_split = split == kSplitFree || (split == kSplitPaid && (N + 63) / 64 < kSkinnyWgTarget * 5 / 8);
     p.nw = type != AESIR_GGML_F16 && t8 * (may_split ? 8 : 1) >= kSkinnyWgTarget * 3 / 4 ? 8 : 4;
     if (may_split) {
         const int64_t tiles = (N + 16 * p.nw - 1) / (16 * p.nw), most = K / (2 * kSeg);
@@ -35,41 +38,16 @@ SkinnyPlan skinny_plan(int64_t M, int64_t K, int64_t N, int32_t type, bool may_s
     return p;
 }
 
-template <int T, int MT, int NW>
-static int32_t launch_t(hipStream_t s, int epi, const SkinnyMat &w, const void *A, int64_t M, int64_t K, int64_t N, void *C,
-                        int64_t ldc, float *part, int64_t ldp, int64_t splits) {
-    constexpr int SG = 2, lds = 2 * SG * MT * 4096;
-    static_assert(lds <= 64 * 1024, "within the default LDS limit");
-    const dim3 grid((unsigned)((N + 16 * NW - 1) / (16 * NW)), (unsigned)splits);
-    hipLaunchKernelGGL((gemm_skinny_kernel<T, MT, 1, NW, SG, 2>), grid, dim3(NW * kWave), lds, s, (const h16 *)A, (int)M,
-                       (int)K, w, (int)N, epi, (h16 *)C, ldc, part, ldp);
-    AESIR_LAUNCH_CHECK("gemm_skinny_kernel");
-    return AESIR_OK;
-}
-
-template <int T>
-static int32_t launch_m(hipStream_t s, int epi, const SkinnyMat &w, const void *A, int64_t M, int64_t K, int64_t N, void *C,
-                        int64_t ldc, float *part, int64_t ldp, const SkinnyPlan &p) {
-#define AESIR_SK(MTV)                                                                                       \
-    return p.nw == 8 ? launch_t<T, MTV, 8>(s, epi, w, A, M, K, N, C, ldc, part, ldp, p.splits)              \
-                     : launch_t<T, MTV, 4>(s, epi, w, A, M, K, N, C, ldc, part, ldp, p.splits)
-    switch ((M + 15) / 16) {
-        case 1: AESIR_SK(1);
-        case 2: AESIR_SK(2);
-        case 3: AESIR_SK(3);
-        default: AESIR_SK(4);
-    }
-#undef AESIR_SK
-}
-
 int32_t launch_gemm_skinny(hipStream_t s, int epi, const SkinnyMat &w, const void *A, int64_t M, int64_t K, int64_t N,
                            void *C, int64_t ldc, float *part, int64_t ldp, const SkinnyPlan &p) {
     if (!p.nw || M < 1 || M > kSkinnyMaxRows || K % kSeg != 0 || p.splits < 1 || p.splits > K / kSeg ||
-        (p.splits > 1 && !part) || (epi == kEpiSwiglu && (N & 1)) || w.qf.row0 % 16 != 0)
+        (p.splits > 1 && !part) || (epi == kEpiSwiglu && (N & 1)) || w.qf.row0 % 16 != 0 ||
+        (w.raw && ((uintptr_t)w.w & 1)))
         return fail(AESIR_ERR_INVALID, "gemm_skinny: unsupported arguments");
     if (((uintptr_t)A & 15) || ((uintptr_t)part & 15)) return fail(AESIR_ERR_INVALID, "gemm_skinny: operand is not 16-byte aligned");
     int32_t rc = AESIR_OK;
-    if (w.type == AESIR_GGML_F16) rc = launch_m<AESIR_GGML_F16>(s, epi, w, A, M, K, N, C, ldc, part, ldp, p);
+    if (w.raw) rc = launch_gemm_skinny_raw(s, epi, w, A, M, K, N, C, ldc, part, ldp, p);
+    else if (w.type == AESIR_GGML_F16) rc = launch_m<AESIR_GGML_F16>(s, epi, w, A, M, K, N, C, ldc, part, ldp, p);
     else if (w.type == AESIR_GGML_Q8_0) rc = launch_m<AESIR_GGML_Q8_0>(s, epi, w, A, M, K, N, C, ldc, part, ldp, p);
     else if (qf_type(w.type))
         qf_switch(w.type, [&](auto t) { rc = launch_m<decltype(t)::value>(s, epi, w, A, M, K, N, C, ldc, part, ldp, p); });

@@ -4,13 +4,16 @@
 
 #include "mfma_gemm.hpp"
 #include "qf_tile.hpp"
+#include "raw_tile.hpp"
 
 namespace aesir {
 
 // One lane's share of a 16-row x 128-k weight tile: row lane % 16, k = 32 (lane / 16) .. + 31.
+// T: f16 rows, Q8_0 planes, a repacked type's planes, or (kRawType + GGML type) packed GGUF blocks.
+constexpr int kRawType = 256;
 template <int T>
 struct SkTile {
-    QTile<T> q;
+    std::conditional_t<(T >= kRawType), RawTile<T % kRawType>, QTile<T % kRawType>> q;
 };
 template <>
 struct SkTile<AESIR_GGML_F16> {
@@ -20,6 +23,10 @@ template <>
 struct SkTile<AESIR_GGML_Q8_0> {
     u32x4 v[2];
     h16 d;
+};
+template <>
+struct SkTile<kRawType + AESIR_GGML_Q8_0> {
+    RawTile<AESIR_GGML_Q8_0> q;
 };
 // The 8 k values of A operand j in lane group g of a segment are granule sk_granule(g, j) (k
 // 8 granule .. + 7): 32 consecutive weights per lane for the repacked tiles (their layout) and for
@@ -60,7 +67,8 @@ __global__ __launch_bounds__(NW *kWave) void gemm_skinny_kernel(const h16 *__res
     constexpr int STAGE = SG * MT * 4096;
     constexpr int RECS = SG * MT * 128;            // 16-element activation records of a step
     constexpr int XL = (RECS + NT - 1) / NT;       // records per thread
-    constexpr bool QF = T != AESIR_GGML_F16 && T != AESIR_GGML_Q8_0;
+    constexpr bool RAW = T >= kRawType, QF = T != AESIR_GGML_F16 && T != AESIR_GGML_Q8_0 && !RAW;
+    constexpr int TR = T % kRawType;
     static_assert(SG <= 2, "the store swizzle covers 16 records per row");
     extern __shared__ __align__(16) uint8_t lds[];  // two stages
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -122,6 +130,7 @@ __global__ __launch_bounds__(NW *kWave) void gemm_skinny_kernel(const h16 *__res
     QfRsrc rs;
     if constexpr (QF) rs = qf_rsrc(w.qf, T, w.qf.row0 + (int64_t)nblk * 16, K);
     const int sbr = K >> 8, s1v = c * es1;
+    const uint8_t *wr[NB];  // packed blocks of the lane's row
     const h16 *wf[NB];
     const int8_t *wq[NB];
     const h16 *wd[NB];
@@ -132,6 +141,7 @@ __global__ __launch_bounds__(NW *kWave) void gemm_skinny_kernel(const h16 *__res
         pb[b] = (int)(w.qf.row0 >> 4) + blk;
         const int row = blk * 16 + c < N ? blk * 16 + c : N - 1;
         if constexpr (T == AESIR_GGML_F16) wf[b] = (const h16 *)w.w + (int64_t)row * K + 8 * g;
+        if constexpr (RAW) wr[b] = (const uint8_t *)w.w + (int64_t)row * (K / (raw_super(TR) ? 256 : 32)) * raw_block_bytes(TR);
         if constexpr (T == AESIR_GGML_Q8_0) {
             wq[b] = (const int8_t *)w.w + (int64_t)row * K + 32 * g;
             wd[b] = (const h16 *)w.s + (int64_t)row * (K / 32) + g;
@@ -152,6 +162,8 @@ __global__ __launch_bounds__(NW *kWave) void gemm_skinny_kernel(const h16 *__res
                     t.v[0] = ld16(wq[b] + sg * 128);
                     t.v[1] = ld16(wq[b] + sg * 128 + 16);
                     t.d = wd[b][sg * 4];
+                } else if constexpr (RAW) {
+                    raw_load<TR>(t.q, wr[b] + (raw_super(TR) ? sg >> 1 : 4 * sg + g) * raw_block_bytes(TR), sg & 1, g);
                 } else {
                     t.q = qf_tile_load<T>(rs, pb[b] * nseg + sg, lane, s1v, (pb[b] * sbr + (sg >> 1)) * 16 * es1);
                 }
@@ -201,6 +213,8 @@ __global__ __launch_bounds__(NW *kWave) void gemm_skinny_kernel(const h16 *__res
                         a[b][2 * h] = u32x4{o[0], o[1], o[2], o[3]};
                         a[b][2 * h + 1] = u32x4{o[4], o[5], o[6], o[7]};
                     }
+                } else if constexpr (RAW) {
+                    raw_tile_a<TR>(t.q, (first + u) & 1, g, a[b]);
                 } else {
                     qf_tile_a<T>(t.q, kr, a[b]);
                 }

@@ -1,4 +1,5 @@
-"""The short-chunk GEMM (1 to 64 activation rows, skinny.hip) at the edges of its tiles.
+"""The short-chunk GEMM (1 to 64 activation rows) at the edges of its tiles, on f16 rows and on packed
+GGUF blocks of every type, and the repacked route above 64 rows on the same blocks.
 
 Rows on both sides of the 16-row activation tiles, weight rows that end inside a 16-row block, a
 workgroup (64 or 128 rows) or a group of 4, one and an odd number of 128-wide K segments, and K splits.
@@ -7,6 +8,8 @@ order over at most 2^14 terms in f32, taken generously) where cancellation leave
 """
 import numpy as np
 import pytest
+
+from quant_tools import expected_f16, make_tensor
 
 pytestmark = pytest.mark.gpu
 
@@ -55,4 +58,33 @@ def test_f16_edges(A, ctx, M, K, N):
     A.gemm_f16(ctx, ctx.from_numpy(a), ctx.from_numpy(b), c.view(M, N))
     got = c.numpy()
     check(got[:M], a, b)
+    assert np.all(got[M] == 7.0)
+
+
+TYPES = {"q4_0": 2, "q4_1": 3, "q5_0": 6, "q5_1": 7, "q8_0": 8, "q2_k": 10, "q3_k": 11, "q4_k": 12, "q5_k": 13,
+         "q6_k": 14}
+
+
+@pytest.mark.parametrize("kind", list(TYPES))
+@pytest.mark.parametrize("M,K,N", [(1, 256, 17), (2, 512, 66), (17, 768, 130), (33, 4096, 70), (64, 1280, 4099),
+                                   (70, 768, 50)])
+@pytest.mark.parametrize("offset", [0, 2])
+def test_packed_blocks(A, ctx, oracle, kind, M, K, N, offset):
+    """Blocks at the start of an allocation and 2 bytes into it (the loads' smallest alignment)."""
+    if kind == "q8_0":
+        d = (0.5 + RNG.random((N, K // 32))) * 0.02 / 73.6
+        t = A.Q8_0Tensor.from_parts(d.astype(np.float16), RNG.integers(-127, 128, (N, K)).astype(np.int8))
+        w = t.dequantize()
+    else:
+        t = make_tensor(A, TYPES[kind], N, K, RNG, 0.02)
+        w = expected_f16(oracle, TYPES[kind], t)
+    raw = np.concatenate([np.zeros(offset, np.uint8), t.blocks.reshape(-1)])
+    raw = np.concatenate([raw, np.zeros(len(raw) % 2, np.uint8)])
+    buf = ctx.from_numpy(raw.view(np.float16))
+    a = RNG.standard_normal((M, K)).astype(np.float16)
+    c = ctx.tensor(M + 1, N)
+    c.upload(np.full((M + 1, N), 7.0, np.float16))
+    A.gemm_quant(ctx, ctx.from_numpy(a), buf.ptr + offset, TYPES[kind], N, c.view(M, N))
+    got = c.numpy()
+    check(got[:M], a, w)
     assert np.all(got[M] == 7.0)
