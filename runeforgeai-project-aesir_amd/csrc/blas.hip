@@ -4,10 +4,9 @@
 // flop per weight byte, three times MI355X's ridge), which is where a library tile sized for that
 // regime pays off; the hand-written wide-tile kernel stays for the short chunks, where the weight
 // stream bounds it. The product is plain: D = A W^T with A [M][K] row-major f16 activations, W
-// [N][K] row-major f16 weights, f32 accumulation and one rounding of each output, to f16 or to
-// f32 for a row kernel that applies the rounding of the epilogue itself. Every epilogue of the
-// prefill (SwiGLU, residual add, RMSNorm) stays a hand-written row kernel, so the rounding
-// points are the fused kernels' own.
+// [N][K] row-major f16 weights, f32 accumulation and one rounding of each output to f16, which is
+// the first rounding of every epilogue. The epilogues of the prefill (SwiGLU, residual add, RMSNorm)
+// stay hand-written row kernels, so the rounding points are the fused kernels' own.
 //
 // In hipBLASLt's column-major terms D^T [N][M] = op(W) A^T with op = transpose on W stored as
 // K x N (leading dimension K), A^T as K x M (leading dimension K) and D^T as N x M (leading
@@ -26,7 +25,6 @@ namespace {
 
 struct BlasPlan {
     int64_t M = 0, N = 0, K = 0;
-    bool f32_out = false;
     bool ok = false;
     hipblasLtMatmulDesc_t desc = nullptr;
     hipblasLtMatrixLayout_t la = nullptr, lb = nullptr, ld = nullptr;
@@ -52,14 +50,13 @@ void destroy_plan(BlasPlan &p) {
 // Builds the descriptors and picks the algorithm for one shape; p.ok stays false when the library
 // offers none within the workspace.
 void make_plan(hipblasLtHandle_t h, BlasPlan &p, size_t ws_bytes) {
-    const hipDataType dt = p.f32_out ? HIP_R_32F : HIP_R_16F;
     const hipblasOperation_t ta = HIPBLAS_OP_T, tb = HIPBLAS_OP_N;
     if (hipblasLtMatmulDescCreate(&p.desc, HIPBLAS_COMPUTE_32F, HIP_R_32F) != HIPBLAS_STATUS_SUCCESS ||
         hipblasLtMatmulDescSetAttribute(p.desc, HIPBLASLT_MATMUL_DESC_TRANSA, &ta, sizeof(ta)) != HIPBLAS_STATUS_SUCCESS ||
         hipblasLtMatmulDescSetAttribute(p.desc, HIPBLASLT_MATMUL_DESC_TRANSB, &tb, sizeof(tb)) != HIPBLAS_STATUS_SUCCESS ||
         hipblasLtMatrixLayoutCreate(&p.la, HIP_R_16F, p.K, p.N, p.K) != HIPBLAS_STATUS_SUCCESS ||
         hipblasLtMatrixLayoutCreate(&p.lb, HIP_R_16F, p.K, p.M, p.K) != HIPBLAS_STATUS_SUCCESS ||
-        hipblasLtMatrixLayoutCreate(&p.ld, dt, p.N, p.M, p.N) != HIPBLAS_STATUS_SUCCESS)
+        hipblasLtMatrixLayoutCreate(&p.ld, HIP_R_16F, p.N, p.M, p.N) != HIPBLAS_STATUS_SUCCESS)
         return;
     hipblasLtMatmulPreference_t pref = nullptr;
     if (hipblasLtMatmulPreferenceCreate(&pref) != HIPBLAS_STATUS_SUCCESS) return;
@@ -81,7 +78,7 @@ void make_plan(hipblasLtHandle_t h, BlasPlan &p, size_t ws_bytes) {
 }  // namespace
 
 int32_t blas_gemm_nt(aesir_ctx *ctx, hipStream_t s, const void *A, int64_t M, int64_t K, const void *W, int64_t N,
-                     void *D, bool f32_out, void *ws, int64_t ws_bytes) {
+                     void *D, void *ws, int64_t ws_bytes) {
     if (M <= 0 || N <= 0 || K <= 0) return fail(AESIR_ERR_INVALID, "blas_gemm_nt: empty shape");
     if (!ctx->blas) {
         auto *st = new BlasState;
@@ -94,7 +91,7 @@ int32_t blas_gemm_nt(aesir_ctx *ctx, hipStream_t s, const void *A, int64_t M, in
     auto *st = static_cast<BlasState *>(ctx->blas);
     BlasPlan *plan = nullptr;
     for (BlasPlan &p : st->plans)
-        if (p.M == M && p.N == N && p.K == K && p.f32_out == f32_out) plan = &p;
+        if (p.M == M && p.N == N && p.K == K) plan = &p;
     if (!plan) {
         // every distinct chunk length brings its shapes: keep the most recent kMaxPlans
         if (st->plans.size() >= kMaxPlans) {
@@ -102,7 +99,7 @@ int32_t blas_gemm_nt(aesir_ctx *ctx, hipStream_t s, const void *A, int64_t M, in
             st->plans.erase(st->plans.begin());
         }
         BlasPlan p;
-        p.M = M, p.N = N, p.K = K, p.f32_out = f32_out;
+        p.M = M, p.N = N, p.K = K;
         make_plan(st->handle, p, (size_t)ws_bytes);
         st->plans.push_back(p);
         plan = &st->plans.back();
