@@ -85,7 +85,9 @@ static int32_t attn_args_for_call(const void *query, int64_t query_rows, const v
     a.seq_len = seq_len;
     a.state = nullptr;
     a.max_seq = seq_len;
-    int64_t max_split = attention_split_count(head_dim, seq_len);
+    const bool aligned = keys_cols % 8 == 0 && values_cols % 8 == 0 &&
+                         (((uintptr_t)query | (uintptr_t)keys | (uintptr_t)values) & 15) == 0;
+    int64_t max_split = attention_split_count(head_dim, seq_len, aligned);
     while (max_split > 1 && attention_partial_floats(nq, head_dim, max_split) > part_cap) max_split >>= 1;
     if (attention_partial_floats(nq, head_dim, max_split) > part_cap)
         return fail(AESIR_ERR_UNSUPPORTED, "flash_attention_gqa: %lld heads x %lld dims exceed the %s of %lld floats",

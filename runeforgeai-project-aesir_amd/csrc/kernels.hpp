@@ -258,8 +258,8 @@ struct AttnArgs {
 // LDS-tiled kernel otherwise), then the merge (one workgroup per query head).
 int32_t launch_attention_decode(hipStream_t s, const AttnArgs &a);
 int64_t attention_partial_floats(int64_t nq, int64_t hd, int64_t max_split);
-// Split count for a KV view of up to max_positions rows.
-int64_t attention_split_count(int64_t hd, int64_t max_positions);
+// Split count for a KV view of up to max_positions rows (aligned: q and all rows on 16 bytes).
+int64_t attention_split_count(int64_t hd, int64_t max_positions, bool aligned = true);
 
 // ------------------------------------------------------------------ elementwise (basic.hip)
 int32_t launch_rmsnorm(hipStream_t s, void *T, int64_t rows, int64_t cols, const void *w, float eps);
