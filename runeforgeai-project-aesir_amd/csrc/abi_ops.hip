@@ -200,8 +200,7 @@ int32_t aesir_argmax_f16(aesir_ctx *ctx, const void *logits, int64_t n, int64_t 
     if (!logits) return fail(AESIR_ERR_INVALID, "argmax: null logits");
     if (n > 2147483647) return fail(AESIR_ERR_UNSUPPORTED, "argmax: more than 2^31-1 logits");
     AESIR_TRY(launch_argmax(ctx->stream, logits, n, ctx->scratch.argmax_part, ctx->scratch.argmax_part_entries,
-                            ctx->scratch.result));
-    AESIR_HIP_TRY(hipMemcpyAsync(ctx->pinned_i64, ctx->scratch.result, sizeof(int64_t), hipMemcpyDeviceToHost, ctx->stream));
+                            ctx->pinned_i64));  // the last kernel writes the index to host memory
     AESIR_HIP_TRY(hipStreamSynchronize(ctx->stream));
     *index = ctx->pinned_i64[0];
     return AESIR_OK;

@@ -171,6 +171,14 @@ int32_t launch_kv_append(hipStream_t s, void *kc, void *vc, const void *k, const
     return AESIR_OK;
 }
 
+__global__ void set_state_kernel(DecodeState v, DecodeState *dst) { *dst = v; }
+
+int32_t launch_set_state(hipStream_t s, const DecodeState &v, DecodeState *dst) {
+    hipLaunchKernelGGL(set_state_kernel, dim3(1), dim3(1), 0, s, v, dst);
+    AESIR_LAUNCH_CHECK("set_state_kernel");
+    return AESIR_OK;
+}
+
 // ------------------------------------------------------------------ seeded init
 // Counter-based normal: element i of stream (seed, stream) from two SplitMix64-mixer outputs
 // (the RuneRNG mixer of sampler.mojo:34-37) and Box-Muller in f64, rounded to f32 then f16.

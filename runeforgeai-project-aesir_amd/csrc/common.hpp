@@ -144,7 +144,6 @@ struct CtxScratch {
     int64_t attn_part_floats = 0;
     void *argmax_part = nullptr;    // argmax partials
     int64_t argmax_part_entries = 0;
-    int64_t *result = nullptr;      // device int64 results
 };
 
 }  // namespace aesir

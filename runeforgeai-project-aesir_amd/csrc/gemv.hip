@@ -273,7 +273,7 @@ __global__ __launch_bounds__(kThreads) void gemv_fixed_kernel(const h16 *__restr
     epi.template apply<ROWS>(n0, m, N, RowSums<ROWS>{red}, tid, pre);
 }
 
-// Final argmax over ordered partials (one workgroup). Writes *result and/or the decode state:
+// Final argmax over ordered partials (one workgroup). Writes *result (device or pinned host memory) and/or the decode state:
 // next_token, and in autoregressive mode token <- next, pos += 1, step += 1, ring[step] = next.
 // Partial g is the first maximum of an index range below partial g + 1's, so the answer is the
 // smallest index among the partials holding the largest value, whatever order they are visited
@@ -694,7 +694,7 @@ int32_t launch_argmax_finish(hipStream_t s, const void *partials, int64_t count,
 
 int32_t launch_lm_head_argmax(hipStream_t s, const LmHeadArgs &a) {
     AESIR_TRY(launch_lm_head(s, a));
-    return launch_argmax_finish(s, a.partials, lm_head_groups(a.vocab), a.state, a.ring, nullptr);
+    return launch_argmax_finish(s, a.partials, lm_head_groups(a.vocab), a.state, a.ring, a.host_next);
 }
 
 // ------------------------------------------------------------------ standalone argmax

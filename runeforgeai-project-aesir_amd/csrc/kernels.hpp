@@ -18,6 +18,9 @@ struct DecodeState {
     int64_t pad[2];
 };
 
+// *dst = v, in stream order (the values travel as the launch's arguments).
+int32_t launch_set_state(hipStream_t s, const DecodeState &v, DecodeState *dst);
+
 // ------------------------------------------------------------------ GEMV / GEMM (gemv.hip)
 
 // C[m, n] = f16(sum_k A[m,k] B[n,k]) for M rows of A (decode GEMV per row; f32 accumulation).
@@ -226,6 +229,7 @@ struct LmHeadArgs {
     int64_t *ring;  // token ring (autoregressive loop), may be null
     const void *w_scale;  // Q8_0 lm_head scales (w is then int8), or null
     QFMat wq;             // Q4_0 / Q4_K / Q6_K lm_head (w and w_scale unused)
+    int64_t *host_next = nullptr;  // pinned host word that receives the greedy token too
 };
 int32_t launch_lm_head_argmax(hipStream_t s, const LmHeadArgs &a);
 int32_t launch_lm_head(hipStream_t s, const LmHeadArgs &a);

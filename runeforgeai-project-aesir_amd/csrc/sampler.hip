@@ -1241,8 +1241,8 @@ struct SamplerWork {
     uint32_t *marks = nullptr; // bits of the running sum at the start of every batch of chunks, then the total
     int64_t *lists = nullptr;  // context tokens then suppress ids
     int64_t *lists_host = nullptr;       // pinned staging of the lists (hipHostMalloc), reused per call
-    hipEvent_t lists_copied = nullptr;   // the last copy out of lists_host
-    int64_t *result = nullptr;
+    bool in_flight = false;              // a call ended before its final wait: lists_host may still be read
+    int64_t *result = nullptr;           // the context's pinned words: (token, whether a random number was used)
     uint32_t *sel_hist = nullptr;  // top-k selection: 3 digit histograms of kSelBins
     uint32_t *sel_cnt = nullptr;   // per-workgroup counts below / equal to the threshold key
     uint64_t *sel_cand = nullptr;  // the selected (key, index) values, kSeqTile
@@ -1255,12 +1255,11 @@ struct SamplerWork {
 static void free_work(SamplerWork *w) {
     void *ps[] = {w->counts, w->mask,  w->vals,  w->keys,      w->keys_out, w->idx,   w->idx_out,
                   w->hdr,    w->cmax,  w->terms, w->csum,      w->heads,    w->subk,  w->slow_list,
-                  w->marks,  w->lists, w->result, w->gpv,      w->gpi,      w->sort_tmp,
+                  w->marks,  w->lists, w->gpv,   w->gpi,       w->sort_tmp,
                   w->sel_hist, w->sel_cnt, w->sel_cand};
     for (void *p : ps)
         if (p) (void)hipFree(p);
     if (w->lists_host) (void)hipHostFree(w->lists_host);
-    if (w->lists_copied) (void)hipEventDestroy(w->lists_copied);
     *w = SamplerWork{};
 }
 
@@ -1277,17 +1276,12 @@ static int32_t ensure_work(aesir_ctx *ctx, int64_t V, int64_t n_lists) {
     if (V > w->cap_v) {
         AESIR_HIP_TRY(hipStreamSynchronize(ctx->stream));
         const int64_t keep_lists = w->cap_ctx;
-        int64_t *old_lists = w->lists, *old_result = w->result, *old_host = w->lists_host;
-        hipEvent_t old_event = w->lists_copied;
+        int64_t *old_lists = w->lists, *old_host = w->lists_host;
         w->lists = nullptr;
         w->lists_host = nullptr;
-        w->lists_copied = nullptr;
-        w->result = nullptr;
         free_work(w);
         w->lists = old_lists;
         w->lists_host = old_host;
-        w->lists_copied = old_event;
-        w->result = old_result;
         w->cap_ctx = keep_lists;
         AESIR_HIP_TRY(hipMalloc((void **)&w->counts, (size_t)V * 4));
         AESIR_HIP_TRY(hipMalloc((void **)&w->mask, (size_t)V));
@@ -1327,8 +1321,7 @@ static int32_t ensure_work(aesir_ctx *ctx, int64_t V, int64_t n_lists) {
         AESIR_HIP_TRY(hipHostMalloc((void **)&w->lists_host, (size_t)cap * 8, hipHostMallocDefault));
         w->cap_ctx = cap;
     }
-    if (!w->lists_copied) AESIR_HIP_TRY(hipEventCreateWithFlags(&w->lists_copied, hipEventDisableTiming));
-    if (!w->result) AESIR_HIP_TRY(hipMalloc((void **)&w->result, 16));
+    w->result = ctx->pinned_i64;
     if (!w->gpv) AESIR_HIP_TRY(hipMalloc((void **)&w->gpv, kGreedyParts * sizeof(float)));
     if (!w->gpi) AESIR_HIP_TRY(hipMalloc((void **)&w->gpi, kGreedyParts * sizeof(int64_t)));
     return AESIR_OK;
@@ -1384,20 +1377,20 @@ int32_t aesir_sample_token(aesir_ctx *ctx, const void *logits, int64_t vocab, co
     const bool greedy = cfg->temperature <= 0.0f || cfg->top_k == 1;  // sampler.mojo:235
     if (greedy && n_suppress == 0) {  // the greedy branch reads no penalty state: argmax of the logits
         AESIR_TRY(launch_greedy(s, (const h16 *)logits, vocab, nullptr, w));
-        AESIR_HIP_TRY(hipMemcpyAsync(ctx->pinned_i64, w->result, 16, hipMemcpyDeviceToHost, s));
         AESIR_HIP_TRY(hipStreamSynchronize(s));
-        *token = ctx->pinned_i64[0];
+        *token = w->result[0];  // written by the last kernel straight to host memory
         return AESIR_OK;
     }
     if (n_lists > 0) {
         // through the pinned staging buffer (an asynchronous copy; a pageable source would be
-        // staged synchronously by the runtime), once the previous call's copy out of it is done
-        AESIR_HIP_TRY(hipEventSynchronize(w->lists_copied));
+        // staged synchronously by the runtime); a call waits for its kernels before it returns, so
+        // only one that failed midway can have left a copy out of it
+        if (w->in_flight) AESIR_HIP_TRY(hipStreamSynchronize(s));
         if (n_context > 0) std::memcpy(w->lists_host, context, (size_t)n_context * 8);
         if (n_suppress > 0) std::memcpy(w->lists_host + n_context, suppress, (size_t)n_suppress * 8);
         AESIR_HIP_TRY(hipMemcpyAsync(w->lists, w->lists_host, (size_t)n_lists * 8, hipMemcpyHostToDevice, s));
-        AESIR_HIP_TRY(hipEventRecord(w->lists_copied, s));
     }
+    w->in_flight = true;
     const unsigned g = (unsigned)((vocab + kSThreads - 1) / kSThreads < 4096 ? (vocab + kSThreads - 1) / kSThreads : 4096);
     hipLaunchKernelGGL(sampler_clear_kernel, dim3(g), dim3(kSThreads), 0, s, w->counts, w->mask, vocab, w->sel_hist,
                        3 * kSelBins);
@@ -1501,12 +1494,10 @@ int32_t aesir_sample_token(aesir_ctx *ctx, const void *logits, int64_t vocab, co
         }
         st = peek;
     }
-    int64_t res[2];
-    AESIR_HIP_TRY(hipMemcpyAsync(ctx->pinned_i64, w->result, 16, hipMemcpyDeviceToHost, s));
     AESIR_HIP_TRY(hipStreamSynchronize(s));
-    std::memcpy(res, ctx->pinned_i64, 16);
-    *token = res[0];
-    if (res[1]) *rng_state = st;  // the draw consumed RuneRNG.next_float32
+    w->in_flight = false;
+    *token = w->result[0];
+    if (w->result[1]) *rng_state = st;  // the draw consumed RuneRNG.next_float32
     return AESIR_OK;
 }
 
