@@ -8,8 +8,8 @@
 //             (descending logit key, index). Equal logits (-0 == +0) keep index order, which is the
 //             order the reference's stable insertion sort (:92-104) produces; every later stage of
 //             the stack sees an already sorted prefix, so one sort serves all of them. With
-//             top_k <= 4096 only that prefix is found: a radix select of the k-th key, an
-//             index-order compaction and a sort of the k selected pairs (same order, no full sort)
+//             top_k <= 4096 only that prefix is found: a radix select of the k-th key's top bits, a
+//             gather of the keys not above them and a sort of those (same order, no full sort)
 //   tail      top_k <= 4096: one workgroup makes the truncations and the draw, the running sums
 //             of apply_top_p, apply_min_p and the draw in one lane in candidate order (f32
 //             addition is not associative; the sums must follow the reference's order to choose
@@ -58,15 +58,13 @@ struct SampleParams {
     float u;        // RuneRNG.next_float32 for the draw
 };
 
-// Clears the context histogram and suppress flags, and the top-k selection's key histograms.
-__global__ void sampler_clear_kernel(int32_t *__restrict__ counts, uint8_t *__restrict__ mask, int64_t V,
-                                     uint32_t *__restrict__ hist, int nhist) {
+// Clears the context histogram and suppress flags.
+__global__ void sampler_clear_kernel(int32_t *__restrict__ counts, uint8_t *__restrict__ mask, int64_t V) {
     const int64_t t0 = (int64_t)blockIdx.x * kSThreads + threadIdx.x, step = (int64_t)gridDim.x * kSThreads;
     for (int64_t i = t0; i < V; i += step) {
         counts[i] = 0;
         mask[i] = 0;
     }
-    for (int64_t i = t0; i < nhist; i += step) hist[i] = 0;
 }
 
 // Occurrence counts of the context tokens and the suppress flags (ids outside the vocabulary
@@ -86,45 +84,30 @@ __global__ void sampler_mark_kernel(const int64_t *__restrict__ ctx, int64_t n_c
     }
 }
 
-__global__ void sampler_prepare_kernel(const h16 *__restrict__ logits, int64_t V, const int32_t *__restrict__ counts,
-                                       const uint8_t *__restrict__ mask, SampleParams p, float *__restrict__ vals,
-                                       uint32_t *__restrict__ keys, int32_t *__restrict__ idx) {
-    for (int64_t i = (int64_t)blockIdx.x * kSThreads + threadIdx.x; i < V; i += (int64_t)gridDim.x * kSThreads) {
-        float v = sanitize_logit((float)logits[i]);
-        if (mask[i]) v = -1e9f;
-        const int32_t c = counts[i];
-        if (p.apply_rep && c > 0) v = v < 0.0f ? v * p.repetition_penalty : v / p.repetition_penalty;
-        if (p.apply_freq && c > 0) {
-            const float freq_loss = (float)c * p.frequency_penalty;
-            v -= (freq_loss + p.presence_penalty);
-        }
-        if (p.apply_temp) v *= p.inv_temp;
-        vals[i] = v;
-        if (p.sort) {
-            keys[i] = desc_key(v);
-            idx[i] = (int32_t)i;
-        }
-    }
-}
-
 // ------------------------------------------------------------------ top-k selection
 //
 // With top_k <= kSeqTile only the first top_k candidates of the stable descending sort are ever
 // read, so instead of sorting the vocabulary the stages find them exactly:
-//   1. the k-th smallest radix key T (ascending key order is the sort's order) by a radix select,
-//      three histogram passes over the key's digits (bits 21-31, 10-20, 0-9); pass p counts the
-//      keys that match the digits already fixed, each workgroup deriving those digits from the
-//      earlier passes' histograms (a scan of 2048 bins per pass)
-//   2. per workgroup, the counts of keys below T and equal to T; then the compaction, in index
-//      order: every key below T, and the lowest-index keys equal to T that complete top_k (the
-//      stable sort keeps equal keys in index order)
-//   3. one workgroup sorts the top_k (key, index) pairs as 64-bit values in LDS (bitonic); the
-//      pairs are distinct, so any correct sort gives the stable sort's order
+//   1. the top 22 bits of the k-th smallest radix key (ascending key order is the sort's order) by a
+//      radix select, two histogram passes over the key's digits (bits 21-31 within the prepare
+//      kernel, 10-20); each later workgroup derives the fixed digits from the histograms (a scan of
+//      2048 bins per digit)
+//   2. a gather, in no order, of every (key, index) whose top 22 bits are not above those: fewer than
+//      top_k below them, and those that share them (logits are f16, so distinct ones differ in these
+//      bits even after a temperature scale: in practice only ties share them)
+//   3. one workgroup sorts what was gathered as 64-bit values in LDS (bitonic) and keeps the first
+//      top_k; the pairs are distinct, so any correct sort gives the stable sort's order. Where more
+//      share the 22 bits than LDS holds (large ties), it finds the last digit and the lowest-index
+//      ties itself by scanning the keys (about 60 us more at 128256 logits that are all equal)
+// Three launches where the digit passes, a count and an ordered compaction took five. Measured on
+// MI355X, 128256 logits, 256 context tokens, top-k 40 with top-p, us per blocking call: 75 -> 43 (with the
+// token lists read by the prepare kernel); 1000 logits 57-74 -> 36; top-k 1000 79-85 -> 64.
 constexpr int kSelBins = 2048;
 constexpr int kSelPer = 4;                              // keys per thread of the selection passes
 constexpr int kSelBlock = kSThreads * kSelPer;          // keys per workgroup
-constexpr int kSelShift[3] = {21, 10, 0};
-constexpr uint32_t kSelMask[3] = {0x7FFu, 0x7FFu, 0x3FFu};
+constexpr int kSelShift[2] = {21, 10};
+constexpr uint32_t kSelLow = 0x3FFu;  // the bits below both digits
+constexpr int kSelCtrs = 4;           // after the two histograms: gathered below / sharing, keys below, the shared bits
 
 struct SelState {
     uint32_t prefix;  // digits fixed so far
@@ -179,156 +162,202 @@ __device__ SelState sel_state(const uint32_t *__restrict__ hist, int np, uint32_
     return st;
 }
 
-__device__ __forceinline__ bool sel_match(uint32_t key, const SelState &st, int np) {
-    return np == 0 || (key >> kSelShift[np - 1]) == (st.prefix >> kSelShift[np - 1]);
+// Values (and radix keys) of kSelBlock consecutive entries per workgroup. LISTS: the context counts
+// and suppress flags of the workgroup's range come from a scan of the token lists into LDS (lists of up
+// to kListScanMax tokens: every workgroup reads them all, from L2), else from the arrays that
+// sampler_mark_kernel filled. HIST: also the first digit's key histogram of the top-k selection
+// (hist, zero on entry), while workgroup 0 clears its second histogram and counters.
+// As separate clear, mark, prepare and histogram launches these took 2.3 + 1.9 + 2.9 + 3.9 us at 128256
+// logits and 256 context tokens plus three launch boundaries.
+constexpr int64_t kListScanMax = 8192;
+template <bool LISTS, bool HIST>
+__global__ __launch_bounds__(kSThreads) void sampler_prepare_kernel(
+    const h16 *__restrict__ logits, int64_t V, const int32_t *__restrict__ counts, const uint8_t *__restrict__ mask,
+    const int64_t *__restrict__ lists, int n_ctx, int n_sup, SampleParams p, float *__restrict__ vals,
+    uint32_t *__restrict__ keys, int32_t *__restrict__ idx, uint32_t *__restrict__ hist) {
+    __shared__ int32_t lc[LISTS ? kSelBlock : 1];    // occurrences of the range's tokens
+    __shared__ uint32_t lm[LISTS ? kSelBlock : 1];   // suppressed
+    __shared__ uint32_t lh[HIST ? kSelBins : 1];
+    const int tid = threadIdx.x;
+    const int64_t base = (int64_t)blockIdx.x * kSelBlock;
+    if constexpr (LISTS)
+        for (int i = tid; i < kSelBlock; i += kSThreads) {
+            lc[i] = 0;
+            lm[i] = 0;
+        }
+    if constexpr (HIST) {
+        for (int i = tid; i < kSelBins; i += kSThreads) lh[i] = 0;
+        if (blockIdx.x == 0)
+            for (int i = tid; i < kSelBins + kSelCtrs; i += kSThreads) hist[kSelBins + i] = 0;
+    }
+    if constexpr (LISTS || HIST) __syncthreads();
+    if constexpr (LISTS) {
+        // (ids outside the vocabulary never match a candidate in the reference: they match no range)
+        for (int i = tid; i < n_ctx + n_sup; i += kSThreads) {
+            const int64_t t = lists[i];
+            if (t < base || t >= base + kSelBlock) continue;
+            if (i < n_ctx) atomicAdd(&lc[t - base], 1);
+            else lm[t - base] = 1;
+        }
+        __syncthreads();
+    }
+#pragma unroll
+    for (int j = 0; j < kSelPer; j++) {
+        const int e = j * kSThreads + tid;
+        const int64_t i = base + e;
+        if (i >= V) break;
+        float v = sanitize_logit((float)logits[i]);
+        if (LISTS ? lm[LISTS ? e : 0] != 0 : mask[i] != 0) v = -1e9f;
+        const int32_t c = LISTS ? lc[LISTS ? e : 0] : counts[i];
+        if (p.apply_rep && c > 0) v = v < 0.0f ? v * p.repetition_penalty : v / p.repetition_penalty;
+        if (p.apply_freq && c > 0) {
+            const float freq_loss = (float)c * p.frequency_penalty;
+            v -= (freq_loss + p.presence_penalty);
+        }
+        if (p.apply_temp) v *= p.inv_temp;
+        vals[i] = v;
+        if (p.sort) {
+            const uint32_t key = desc_key(v);
+            keys[i] = key;
+            if constexpr (HIST) atomicAdd(&lh[key >> kSelShift[0]], 1u);
+            else idx[i] = (int32_t)i;
+        }
+    }
+    if constexpr (HIST) {
+        __syncthreads();
+        for (int b = tid; b < kSelBins; b += kSThreads)
+            if (lh[b]) atomicAdd(&hist[b], lh[b]);
+    }
 }
 
-template <int NP>
+// Histogram of the second digit over the keys that match the first.
 __global__ __launch_bounds__(kSThreads) void sampler_select_hist_kernel(const uint32_t *__restrict__ keys, int64_t V,
                                                                         uint32_t *__restrict__ hist, uint32_t k) {
     __shared__ uint32_t lh[kSelBins];
     __shared__ uint32_t sh[8];
     const int tid = threadIdx.x;
+    const int64_t base = (int64_t)blockIdx.x * kSelBlock;
+    uint32_t kv[kSelPer];
+#pragma unroll
+    for (int j = 0; j < kSelPer; j++) {
+        const int64_t i = base + j * kSThreads + tid;
+        kv[j] = keys[i < V ? i : V - 1];
+    }
     for (int b = tid; b < kSelBins; b += kSThreads) lh[b] = 0;
-    const SelState st = sel_state(hist, NP, k, sh);
-    __syncthreads();  // lh is clear (sel_state synchronizes only when NP > 0)
-    const int64_t base = (int64_t)blockIdx.x * kSelBlock;
+    const SelState st = sel_state(hist, 1, k, sh);  // synchronizes: lh is clear
 #pragma unroll
-    for (int j = 0; j < kSelPer; j++) {
-        const int64_t i = base + j * kSThreads + tid;
-        if (i < V) {
-            const uint32_t key = keys[i];
-            if (sel_match(key, st, NP)) atomicAdd(&lh[(key >> kSelShift[NP]) & kSelMask[NP]], 1u);
-        }
-    }
+    for (int j = 0; j < kSelPer; j++)
+        if (base + j * kSThreads + tid < V && kv[j] >> kSelShift[0] == st.prefix >> kSelShift[0])
+            atomicAdd(&lh[(kv[j] >> kSelShift[1]) & (kSelBins - 1)], 1u);
     __syncthreads();
-    uint32_t *gh = hist + NP * kSelBins;
     for (int b = tid; b < kSelBins; b += kSThreads)
-        if (lh[b]) atomicAdd(&gh[b], lh[b]);
+        if (lh[b]) atomicAdd(&hist[kSelBins + b], lh[b]);
 }
 
-// Per workgroup of kSelBlock keys: how many are below T and how many equal it.
-__global__ __launch_bounds__(kSThreads) void sampler_select_count_kernel(const uint32_t *__restrict__ keys, int64_t V,
-                                                                         const uint32_t *__restrict__ hist, uint32_t k,
-                                                                         uint32_t *__restrict__ cnt) {
+// Every (key, index) with top bits below the k-th key's, in cand[0, below), and those sharing them behind
+// (as many as fit kSeqTile); ctr: how many of each were met, `below` and the shared bits.
+__global__ __launch_bounds__(kSThreads) void sampler_select_gather_kernel(const uint32_t *__restrict__ keys, int64_t V,
+                                                                          const uint32_t *__restrict__ hist, uint32_t k,
+                                                                          uint32_t *__restrict__ ctr,
+                                                                          uint64_t *__restrict__ cand) {
     __shared__ uint32_t sh[8];
-    __shared__ uint32_t red[2][kSThreads / 64];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const SelState st = sel_state(hist, 3, k, sh);
-    const uint32_t T = st.prefix;
+    const int tid = threadIdx.x, lane = tid & 63;
     const int64_t base = (int64_t)blockIdx.x * kSelBlock;
-    uint32_t lt = 0, eq = 0;
+    uint32_t kv[kSelPer];
 #pragma unroll
     for (int j = 0; j < kSelPer; j++) {
         const int64_t i = base + j * kSThreads + tid;
-        if (i < V) {
-            const uint32_t key = keys[i];
-            lt += key < T;
-            eq += key == T;
-        }
+        kv[j] = keys[i < V ? i : V - 1];
     }
-    for (int o = 32; o > 0; o >>= 1) {
-        lt += __shfl_xor(lt, o);
-        eq += __shfl_xor(eq, o);
+    const SelState st = sel_state(hist, 2, k, sh);
+    const uint32_t top = st.prefix >> kSelShift[1];
+    if (blockIdx.x == 0 && tid == 0) {
+        ctr[2] = st.lt;
+        ctr[3] = top;
     }
-    if (lane == 0) {
-        red[0][wave] = lt;
-        red[1][wave] = eq;
-    }
-    __syncthreads();
-    if (tid == 0) {
-        uint32_t a = 0, b = 0;
-        for (int w = 0; w < kSThreads / 64; w++) {
-            a += red[0][w];
-            b += red[1][w];
-        }
-        cnt[2 * blockIdx.x] = a;
-        cnt[2 * blockIdx.x + 1] = b;
-    }
-}
-
-// The compaction: key-below-T entries at their index-order rank among them, the first
-// `rank` equal-key entries (in index order) after them; 64-bit (key, index) values.
-__global__ __launch_bounds__(kSThreads) void sampler_select_compact_kernel(const uint32_t *__restrict__ keys, int64_t V,
-                                                                           const uint32_t *__restrict__ hist, uint32_t k,
-                                                                           const uint32_t *__restrict__ cnt,
-                                                                           uint64_t *__restrict__ cand) {
-    __shared__ uint32_t sh[8];
-    __shared__ uint32_t wl[kSThreads / 64], we[kSThreads / 64];
-    __shared__ uint32_t pre_s[2];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const SelState st = sel_state(hist, 3, k, sh);
-    const uint32_t T = st.prefix, need = st.rank, total_lt = st.lt;
-    // keys below T and equal to T in the workgroups before this one
-    {
-        uint32_t a = 0, b = 0;
-        for (int w = tid; w < (int)blockIdx.x; w += kSThreads) {
-            a += cnt[2 * w];
-            b += cnt[2 * w + 1];
-        }
-        for (int o = 32; o > 0; o >>= 1) {
-            a += __shfl_xor(a, o);
-            b += __shfl_xor(b, o);
-        }
-        if (lane == 0) {
-            wl[wave] = a;
-            we[wave] = b;
-        }
-        __syncthreads();
-        if (tid == 0) {
-            uint32_t x = 0, y = 0;
-            for (int w = 0; w < kSThreads / 64; w++) {
-                x += wl[w];
-                y += we[w];
-            }
-            pre_s[0] = x;
-            pre_s[1] = y;
-        }
-        __syncthreads();
-    }
-    uint32_t run_lt = pre_s[0], run_eq = pre_s[1];
-    const int64_t base = (int64_t)blockIdx.x * kSelBlock;
-    for (int j = 0; j < kSelPer; j++) {  // index order: pass j covers keys base + j * 256 + [0, 256)
+#pragma unroll
+    for (int j = 0; j < kSelPer; j++) {
         const int64_t i = base + j * kSThreads + tid;
-        const uint32_t key = i < V ? keys[i] : 0xFFFFFFFFu;
-        const bool is_lt = i < V && key < T, is_eq = i < V && key == T;
-        const uint64_t bl = __ballot(is_lt), be = __ballot(is_eq);
-        const uint32_t rl = (uint32_t)__popcll(bl & ((1ull << lane) - 1ull));
-        const uint32_t re = (uint32_t)__popcll(be & ((1ull << lane) - 1ull));
-        __syncthreads();  // wl / we of the previous pass have been read
-        if (lane == 0) {
-            wl[wave] = (uint32_t)__popcll(bl);
-            we[wave] = (uint32_t)__popcll(be);
-        }
-        __syncthreads();
-        uint32_t ol = run_lt, oe = run_eq;
-        for (int w = 0; w < wave; w++) {
-            ol += wl[w];
-            oe += we[w];
-        }
-        // the slots stay below k by construction (total_lt + need = k); the bounds are checked anyway
-        if (is_lt && ol + rl < k) cand[ol + rl] = ((uint64_t)key << 32) | (uint64_t)i;
-        if (is_eq && oe + re < need && total_lt + oe + re < k)
-            cand[total_lt + oe + re] = ((uint64_t)key << 32) | (uint64_t)i;
-        for (int w = 0; w < kSThreads / 64; w++) {
-            run_lt += wl[w];
-            run_eq += we[w];
-        }
+        const uint32_t t = kv[j] >> kSelShift[1];
+        const bool in = i < V;
+        const uint64_t below = __ballot(in && t < top), same = __ballot(in && t == top);
+        uint32_t at = 0;  // lane 0: the wave's first slot among the keys below; lane 1: among the sharing ones
+        if (lane == 0 && below) at = atomicAdd(&ctr[0], (uint32_t)__popcll(below));
+        if (lane == 1 && same) at = atomicAdd(&ctr[1], (uint32_t)__popcll(same));
+        const uint32_t a = __shfl(at, 0), b = __shfl(at, 1);
+        const uint64_t before = (1ull << lane) - 1ull;
+        uint32_t slot = kSeqTile;
+        if (in && t < top) slot = a + (uint32_t)__popcll(below & before);
+        if (in && t == top) slot = st.lt + b + (uint32_t)__popcll(same & before);
+        if (slot < kSeqTile) cand[slot] = ((uint64_t)kv[j] << 32) | (uint64_t)i;
     }
 }
 
-// Sorts the k <= kSeqTile selected (key, index) values (bitonic, in LDS) and writes the indices.
+// Sorts the gathered (key, index) values (bitonic, in LDS), writes the first k indices and clears the
+// first digit's histogram for the next call.
 constexpr int kSelSortThreads = 1024;
-__global__ __launch_bounds__(kSelSortThreads) void sampler_select_sort_kernel(const uint64_t *__restrict__ cand,
-                                                                              int k, int32_t *__restrict__ order) {
+__global__ __launch_bounds__(kSelSortThreads) void sampler_select_sort_kernel(const uint32_t *__restrict__ keys, int64_t V,
+                                                                              uint32_t *__restrict__ hist,
+                                                                              const uint64_t *__restrict__ cand, int k,
+                                                                              int32_t *__restrict__ order) {
     __shared__ uint64_t v[kSeqTile];
+    __shared__ uint32_t lh[kSelLow + 1], wc[kSelSortThreads / 64], sh[4];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const uint32_t *ctr = hist + 2 * kSelBins;
+    const int lt = (int)ctr[2];
+    int total = lt + (int)(ctr[1] < (uint32_t)(kSeqTile + 1) ? ctr[1] : kSeqTile + 1);
+    const uint32_t top = ctr[3];
+    for (int i = tid; i < kSelBins; i += kSelSortThreads) hist[i] = 0;
+    const bool all = total <= kSeqTile;
+    for (int i = tid; i < (all ? total : lt); i += kSelSortThreads) v[i] = cand[i];
+    if (!all) {  // the k - lt first (key, index) among those sharing the bits, found by scanning the keys
+        static_assert(kSelSortThreads == (int)kSelLow + 1, "one bin per thread");
+        lh[tid] = 0;
+        __syncthreads();
+        for (int64_t i = tid; i < V; i += kSelSortThreads)
+            if (keys[i] >> kSelShift[1] == top) atomicAdd(&lh[keys[i] & kSelLow], 1u);
+        __syncthreads();
+        const uint32_t mine = lh[tid], need = (uint32_t)(k - lt);
+        for (int o = 1; o < kSelSortThreads; o <<= 1) {  // inclusive sums
+            const uint32_t t = tid >= o ? lh[tid - o] : 0u;
+            __syncthreads();
+            lh[tid] += t;
+            __syncthreads();
+        }
+        if (lh[tid] >= need && lh[tid] - mine < need) {
+            sh[0] = (uint32_t)tid;          // the last digit of the k-th key
+            sh[1] = lh[tid] - mine;         // keys with a smaller one
+            sh[2] = 0;
+        }
+        __syncthreads();
+        const uint32_t T = (top << kSelShift[1]) | sh[0], less = sh[1];
+        uint32_t met = 0;  // keys equal to T so far, in index order
+        for (int64_t b0 = 0; b0 < V; b0 += kSelSortThreads) {
+            const int64_t i = b0 + tid;
+            const uint32_t key = i < V ? keys[i] : 0xFFFFFFFFu;
+            const bool in = i < V && key >> kSelShift[1] == top;
+            if (in && key < T) v[lt + atomicAdd(&sh[2], 1u)] = ((uint64_t)key << 32) | (uint64_t)i;
+            const uint64_t eq = __ballot(in && key == T);
+            if (lane == 0) wc[wave] = (uint32_t)__popcll(eq);
+            __syncthreads();
+            uint32_t r = met;
+            for (int w = 0; w < kSelSortThreads / 64; w++) {
+                if (w < wave) r += wc[w];
+                met += wc[w];
+            }
+            r += (uint32_t)__popcll(eq & ((1ull << lane) - 1ull));
+            if (in && key == T && r < need - less) v[lt + less + r] = ((uint64_t)key << 32) | (uint64_t)i;
+            __syncthreads();
+        }
+        total = k;
+    }
     int m = 1;
-    while (m < k) m <<= 1;
-    for (int i = threadIdx.x; i < m; i += kSelSortThreads) v[i] = i < k ? cand[i] : ~0ull;
+    while (m < total) m <<= 1;
+    for (int i = total + tid; i < m; i += kSelSortThreads) v[i] = ~0ull;
     __syncthreads();
     for (int size = 2; size <= m; size <<= 1) {
         for (int stride = size >> 1; stride > 0; stride >>= 1) {
-            for (int i = threadIdx.x; i < m; i += kSelSortThreads) {
+            for (int i = tid; i < m; i += kSelSortThreads) {
                 const int j = i ^ stride;
                 if (j > i) {
                     const bool up = (i & size) == 0;
@@ -342,7 +371,7 @@ __global__ __launch_bounds__(kSelSortThreads) void sampler_select_sort_kernel(co
             __syncthreads();
         }
     }
-    for (int i = threadIdx.x; i < k; i += kSelSortThreads) order[i] = (int32_t)(v[i] & 0xFFFFFFFFull);
+    for (int i = tid; i < k; i += kSelSortThreads) order[i] = (int32_t)(v[i] & 0xFFFFFFFFull);
 }
 
 // Greedy branch (:241-261): best = 0, max = value of index 0, strict '>' ascending; values are
@@ -1243,8 +1272,7 @@ struct SamplerWork {
     int64_t *lists_host = nullptr;       // pinned staging of the lists (hipHostMalloc), reused per call
     bool in_flight = false;              // a call ended before its final wait: lists_host may still be read
     int64_t *result = nullptr;           // the context's pinned words: (token, whether a random number was used)
-    uint32_t *sel_hist = nullptr;  // top-k selection: 3 digit histograms of kSelBins
-    uint32_t *sel_cnt = nullptr;   // per-workgroup counts below / equal to the threshold key
+    uint32_t *sel_hist = nullptr;  // top-k selection: 2 digit histograms of kSelBins (the first kept zero between calls), kSelCtrs counters
     uint64_t *sel_cand = nullptr;  // the selected (key, index) values, kSeqTile
     float *gpv = nullptr;      // the greedy branch's per-workgroup best values
     int64_t *gpi = nullptr;    // and their indices
@@ -1256,7 +1284,7 @@ static void free_work(SamplerWork *w) {
     void *ps[] = {w->counts, w->mask,  w->vals,  w->keys,      w->keys_out, w->idx,   w->idx_out,
                   w->hdr,    w->cmax,  w->terms, w->csum,      w->heads,    w->subk,  w->slow_list,
                   w->marks,  w->lists, w->gpv,   w->gpi,       w->sort_tmp,
-                  w->sel_hist, w->sel_cnt, w->sel_cand};
+                  w->sel_hist, w->sel_cand};
     for (void *p : ps)
         if (p) (void)hipFree(p);
     if (w->lists_host) (void)hipHostFree(w->lists_host);
@@ -1299,8 +1327,8 @@ static int32_t ensure_work(aesir_ctx *ctx, int64_t V, int64_t n_lists) {
         AESIR_HIP_TRY(hipMalloc((void **)&w->heads, (size_t)nbat * 64 * 4));
         AESIR_HIP_TRY(hipMalloc((void **)&w->subk, (size_t)nch * kSubWords * 4));
         AESIR_HIP_TRY(hipMalloc((void **)&w->slow_list, (size_t)kSlowListMax * 4));
-        AESIR_HIP_TRY(hipMalloc((void **)&w->sel_hist, (size_t)3 * kSelBins * 4));
-        AESIR_HIP_TRY(hipMalloc((void **)&w->sel_cnt, (size_t)2 * ((V + kSelBlock - 1) / kSelBlock) * 4));
+        AESIR_HIP_TRY(hipMalloc((void **)&w->sel_hist, (size_t)(2 * kSelBins + kSelCtrs) * 4));
+        w->in_flight = true;  // its first histogram is not zero yet
         AESIR_HIP_TRY(hipMalloc((void **)&w->sel_cand, (size_t)kSeqTile * 8));
         AESIR_HIP_TRY(hipMalloc((void **)&w->marks, (size_t)(nbat + 1) * 4));
         size_t bytes = 0;
@@ -1381,21 +1409,23 @@ int32_t aesir_sample_token(aesir_ctx *ctx, const void *logits, int64_t vocab, co
         *token = w->result[0];  // written by the last kernel straight to host memory
         return AESIR_OK;
     }
+    if (w->in_flight) {  // a call that failed midway may still read lists_host and leaves the histogram as it was
+        AESIR_HIP_TRY(hipStreamSynchronize(s));
+        AESIR_HIP_TRY(hipMemsetAsync(w->sel_hist, 0, kSelBins * 4, s));
+    }
+    w->in_flight = true;
     if (n_lists > 0) {
-        // through the pinned staging buffer (an asynchronous copy; a pageable source would be
-        // staged synchronously by the runtime); a call waits for its kernels before it returns, so
-        // only one that failed midway can have left a copy out of it
-        if (w->in_flight) AESIR_HIP_TRY(hipStreamSynchronize(s));
+        // through the pinned staging buffer (an asynchronous copy; a pageable source would be staged
+        // synchronously by the runtime); a call waits for its kernels before it returns
         if (n_context > 0) std::memcpy(w->lists_host, context, (size_t)n_context * 8);
         if (n_suppress > 0) std::memcpy(w->lists_host + n_context, suppress, (size_t)n_suppress * 8);
         AESIR_HIP_TRY(hipMemcpyAsync(w->lists, w->lists_host, (size_t)n_lists * 8, hipMemcpyHostToDevice, s));
     }
-    w->in_flight = true;
-    const unsigned g = (unsigned)((vocab + kSThreads - 1) / kSThreads < 4096 ? (vocab + kSThreads - 1) / kSThreads : 4096);
-    hipLaunchKernelGGL(sampler_clear_kernel, dim3(g), dim3(kSThreads), 0, s, w->counts, w->mask, vocab, w->sel_hist,
-                       3 * kSelBins);
-    AESIR_LAUNCH_CHECK("sampler_clear_kernel");
-    if (n_lists > 0) {
+    const bool scan = !greedy && n_lists <= kListScanMax;  // the prepare kernel reads the lists itself
+    if (!scan) {
+        const unsigned g = (unsigned)((vocab + kSThreads - 1) / kSThreads < 4096 ? (vocab + kSThreads - 1) / kSThreads : 4096);
+        hipLaunchKernelGGL(sampler_clear_kernel, dim3(g), dim3(kSThreads), 0, s, w->counts, w->mask, vocab);
+        AESIR_LAUNCH_CHECK("sampler_clear_kernel");
         const unsigned gl = (unsigned)((n_lists + kSThreads - 1) / kSThreads < 4096 ? (n_lists + kSThreads - 1) / kSThreads : 4096);
         hipLaunchKernelGGL(sampler_mark_kernel, dim3(gl), dim3(kSThreads), 0, s, w->lists, n_context,
                            w->lists + n_context, n_suppress, w->counts, w->mask, vocab);
@@ -1422,25 +1452,27 @@ int32_t aesir_sample_token(aesir_ctx *ctx, const void *logits, int64_t vocab, co
         p.sort = k_on || p_on || m_on;
         uint64_t peek = st;
         p.u = (float)(rune_next(&peek) & 0xFFFFFFULL) / 16777216.0f;
-        hipLaunchKernelGGL(sampler_prepare_kernel, dim3(g), dim3(kSThreads), 0, s, (const h16 *)logits, vocab,
-                           w->counts, w->mask, p, w->vals, w->keys, w->idx);
-        AESIR_LAUNCH_CHECK("sampler_prepare_kernel");
         const bool select_k = k_on && cfg->top_k <= kSeqTile;
+        const unsigned nb = (unsigned)((vocab + kSelBlock - 1) / kSelBlock);
+#define AESIR_PREPARE(LV, HV)                                                                                      \
+    hipLaunchKernelGGL((sampler_prepare_kernel<LV, HV>), dim3(nb), dim3(kSThreads), 0, s, (const h16 *)logits, vocab, \
+                       w->counts, w->mask, w->lists, (int)(scan ? n_context : 0), (int)(scan ? n_suppress : 0), p, w->vals, \
+                       w->keys, w->idx, w->sel_hist)
+        if (scan && select_k) AESIR_PREPARE(true, true);
+        else if (scan) AESIR_PREPARE(true, false);
+        else if (select_k) AESIR_PREPARE(false, true);
+        else AESIR_PREPARE(false, false);
+#undef AESIR_PREPARE
+        AESIR_LAUNCH_CHECK("sampler_prepare_kernel");
         if (select_k) {  // the first top_k of the stable sort, found without sorting the vocabulary
-            const unsigned nb = (unsigned)((vocab + kSelBlock - 1) / kSelBlock);
             const uint32_t k = (uint32_t)cfg->top_k;
-            hipLaunchKernelGGL(sampler_select_hist_kernel<0>, dim3(nb), dim3(kSThreads), 0, s, w->keys, vocab, w->sel_hist, k);
-            hipLaunchKernelGGL(sampler_select_hist_kernel<1>, dim3(nb), dim3(kSThreads), 0, s, w->keys, vocab, w->sel_hist, k);
-            hipLaunchKernelGGL(sampler_select_hist_kernel<2>, dim3(nb), dim3(kSThreads), 0, s, w->keys, vocab, w->sel_hist, k);
+            hipLaunchKernelGGL(sampler_select_hist_kernel, dim3(nb), dim3(kSThreads), 0, s, w->keys, vocab, w->sel_hist, k);
             AESIR_LAUNCH_CHECK("sampler_select_hist_kernel");
-            hipLaunchKernelGGL(sampler_select_count_kernel, dim3(nb), dim3(kSThreads), 0, s, w->keys, vocab, w->sel_hist, k,
-                               w->sel_cnt);
-            AESIR_LAUNCH_CHECK("sampler_select_count_kernel");
-            hipLaunchKernelGGL(sampler_select_compact_kernel, dim3(nb), dim3(kSThreads), 0, s, w->keys, vocab,
-                               w->sel_hist, k, w->sel_cnt, w->sel_cand);
-            AESIR_LAUNCH_CHECK("sampler_select_compact_kernel");
-            hipLaunchKernelGGL(sampler_select_sort_kernel, dim3(1), dim3(kSelSortThreads), 0, s, w->sel_cand, (int)k,
-                               w->idx_out);
+            hipLaunchKernelGGL(sampler_select_gather_kernel, dim3(nb), dim3(kSThreads), 0, s, w->keys, vocab, w->sel_hist, k,
+                               w->sel_hist + 2 * kSelBins, w->sel_cand);
+            AESIR_LAUNCH_CHECK("sampler_select_gather_kernel");
+            hipLaunchKernelGGL(sampler_select_sort_kernel, dim3(1), dim3(kSelSortThreads), 0, s, w->keys, vocab, w->sel_hist,
+                               w->sel_cand, (int)k, w->idx_out);
             AESIR_LAUNCH_CHECK("sampler_select_sort_kernel");
         } else if (p.sort) {
             size_t bytes = w->sort_tmp_bytes;

@@ -1,0 +1,37 @@
+"""The sampler's top-k selection and token lists where their route changes: more ties at the k-th logit
+than the sorting workgroup holds (constant logits, three levels), exactly as many candidates as top_k
+leaves, token lists on both sides of the length that the prepare kernel scans itself, ids outside the
+vocabulary, vocabularies around a workgroup's 1024 entries. Token and RuneRNG state equal the oracle's
+(exact: both sides run the reference's f32 sums in the reference's order)."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def A():
+    import aesir_hip
+
+    return aesir_hip
+
+
+@pytest.mark.parametrize("vocab,levels,top_k,n_context,n_suppress", [
+    (128256, 1, 40, 0, 0), (128256, 1, 4096, 5, 0), (128256, 3, 1000, 300, 2), (60000, 2, 3000, 8192, 0),
+    (60000, 200, 64, 8190, 3), (1023, 1, 1000, 10, 0), (1024, 60, 1023, 0, 1), (1025, 60, 40, 2000, 10),
+    (4097, 1, 4096, 1, 1), (2, 1, 1, 0, 0),
+])
+def test_selection(A, oracle, vocab, levels, top_k, n_context, n_suppress):
+    rng = np.random.default_rng(vocab + top_k + n_context)
+    cfg = dict(temperature=0.8, top_k=top_k, top_p=0.97, repetition_penalty=1.2)
+    g_rng = A.RuneRNG(99)
+    o_state = oracle.rune_rng_state(99)
+    with A.Context(64 << 20) as ctx:
+        for d in range(4):
+            logits = (rng.integers(0, levels, vocab) * 0.5 + 1.0).astype(np.float16)
+            context = rng.integers(-3, vocab + 3, n_context).tolist()
+            suppress = rng.integers(0, vocab + 1, n_suppress).tolist()
+            got = A.sample_token(ctx, ctx.from_numpy(logits.reshape(1, -1)), A.SamplerConfig(**cfg), g_rng, context, suppress)
+            want, o_state = oracle.sample_token_f16(logits, oracle.SamplerConfig(**cfg), o_state, context, suppress)
+            assert got == want, d
+            assert g_rng.state == o_state, d
