@@ -562,4 +562,12 @@ __device__ __forceinline__ void qf_perm_rec(const u32x4 (&x)[2], u32x4 (&o)[2]) 
     }
 }
 
+// qf_perm_rec's inverse: a record's operands 2 h and 2 h + 1 of qf_tile_a to its 16 weights in order.
+__device__ __forceinline__ void qf_unperm_rec(const u32x4 &p, const u32x4 &q, u32x4 (&o)[2]) {
+    o[0] = u32x4{__builtin_amdgcn_perm(p.y, p.x, 0x05040100u), __builtin_amdgcn_perm(p.y, p.x, 0x07060302u),
+                 __builtin_amdgcn_perm(q.y, q.x, 0x05040100u), __builtin_amdgcn_perm(q.y, q.x, 0x07060302u)};
+    o[1] = u32x4{__builtin_amdgcn_perm(p.w, p.z, 0x05040100u), __builtin_amdgcn_perm(p.w, p.z, 0x07060302u),
+                 __builtin_amdgcn_perm(q.w, q.z, 0x05040100u), __builtin_amdgcn_perm(q.w, q.z, 0x07060302u)};
+}
+
 }  // namespace aesir
