@@ -13,7 +13,7 @@
 //   tail      top_k <= 4096: one workgroup makes the truncations and the draw, the running sums
 //             of apply_top_p, apply_min_p and the draw in one lane in candidate order (f32
 //             addition is not associative; the sums must follow the reference's order to choose
-//             the same cut and token), the next LDS tile of exps computed by the other waves
+//             the same cut and token), in the workgroup that sorted the selection
 //   chunked   longer candidate lists: each running sum (top-p's sum and cut, min-p's sum, the
 //             final draw's sum and walk) is a terms pass and a records pass over the whole device
 //             and one wave that reproduces the sequential f32 sum bit for bit, with one integer
@@ -35,8 +35,7 @@
 namespace aesir {
 
 constexpr int kSThreads = 256;
-constexpr int kTailThreads = 256;
-constexpr int kSeqTile = 4096;  // terms per LDS tile of the tail (two tiles); its candidate limit
+constexpr int kSeqTile = 4096;  // candidates that the selecting workgroup holds in LDS
 
 __device__ __forceinline__ float sanitize_logit(float v) { return (isnan(v) || isinf(v)) ? -1e9f : v; }
 __device__ __forceinline__ float exp_f32(float x) { return (float)exp((double)x); }
@@ -52,7 +51,6 @@ __device__ __forceinline__ uint32_t desc_key(float v) {
 struct SampleParams {
     float repetition_penalty, frequency_penalty, presence_penalty, inv_temp;
     int apply_rep, apply_freq, apply_temp, sort;
-    int64_t top_k;  // > 0: truncate to top_k after the sort
     float top_p;    // < 1: nucleus
     float min_p;    // in (0, 1): min-p
     float u;        // RuneRNG.next_float32 for the draw
@@ -95,13 +93,14 @@ __global__ void sampler_mark_kernel(const int64_t *__restrict__ ctx, int64_t n_c
 //   2. a gather, in no order, of every (key, index) whose top 22 bits are not above those: fewer than
 //      top_k below them, and those that share them (logits are f16, so distinct ones differ in these
 //      bits even after a temperature scale: in practice only ties share them)
-//   3. one workgroup sorts what was gathered as 64-bit values in LDS (bitonic) and keeps the first
-//      top_k; the pairs are distinct, so any correct sort gives the stable sort's order. Where more
+//   3. one workgroup sorts what was gathered as 64-bit values in LDS and keeps the first top_k;
+//      the pairs are distinct, so any correct sort gives the stable sort's order. Where more
 //      share the 22 bits than LDS holds (large ties), it finds the last digit and the lowest-index
 //      ties itself by scanning the keys (about 60 us more at 128256 logits that are all equal)
-// Three launches where the digit passes, a count and an ordered compaction took five. Measured on
-// MI355X, 128256 logits, 256 context tokens, top-k 40 with top-p, us per blocking call: 75 -> 43 (with the
-// token lists read by the prepare kernel); 1000 logits 57-74 -> 36; top-k 1000 79-85 -> 64.
+//   4. the same workgroup makes the truncations and the draw (sampler_select_draw_kernel)
+// Three launches where three digit passes, a count, an ordered compaction, a sort and a tail took seven.
+// Measured on MI355X, 128256 logits, 256 context tokens, top-k 40 with top-p, us per blocking call:
+// 75 -> 37.5 (with the token lists read by the prepare kernel).
 constexpr int kSelBins = 2048;
 constexpr int kSelPer = 4;                              // keys per thread of the selection passes
 constexpr int kSelBlock = kSThreads * kSelPer;          // keys per workgroup
@@ -293,87 +292,6 @@ __global__ __launch_bounds__(kSThreads) void sampler_select_gather_kernel(const 
     }
 }
 
-// Sorts the gathered (key, index) values (bitonic, in LDS), writes the first k indices and clears the
-// first digit's histogram for the next call.
-constexpr int kSelSortThreads = 1024;
-__global__ __launch_bounds__(kSelSortThreads) void sampler_select_sort_kernel(const uint32_t *__restrict__ keys, int64_t V,
-                                                                              uint32_t *__restrict__ hist,
-                                                                              const uint64_t *__restrict__ cand, int k,
-                                                                              int32_t *__restrict__ order) {
-    __shared__ uint64_t v[kSeqTile];
-    __shared__ uint32_t lh[kSelLow + 1], wc[kSelSortThreads / 64], sh[4];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const uint32_t *ctr = hist + 2 * kSelBins;
-    const int lt = (int)ctr[2];
-    int total = lt + (int)(ctr[1] < (uint32_t)(kSeqTile + 1) ? ctr[1] : kSeqTile + 1);
-    const uint32_t top = ctr[3];
-    for (int i = tid; i < kSelBins; i += kSelSortThreads) hist[i] = 0;
-    const bool all = total <= kSeqTile;
-    for (int i = tid; i < (all ? total : lt); i += kSelSortThreads) v[i] = cand[i];
-    if (!all) {  // the k - lt first (key, index) among those sharing the bits, found by scanning the keys
-        static_assert(kSelSortThreads == (int)kSelLow + 1, "one bin per thread");
-        lh[tid] = 0;
-        __syncthreads();
-        for (int64_t i = tid; i < V; i += kSelSortThreads)
-            if (keys[i] >> kSelShift[1] == top) atomicAdd(&lh[keys[i] & kSelLow], 1u);
-        __syncthreads();
-        const uint32_t mine = lh[tid], need = (uint32_t)(k - lt);
-        for (int o = 1; o < kSelSortThreads; o <<= 1) {  // inclusive sums
-            const uint32_t t = tid >= o ? lh[tid - o] : 0u;
-            __syncthreads();
-            lh[tid] += t;
-            __syncthreads();
-        }
-        if (lh[tid] >= need && lh[tid] - mine < need) {
-            sh[0] = (uint32_t)tid;          // the last digit of the k-th key
-            sh[1] = lh[tid] - mine;         // keys with a smaller one
-            sh[2] = 0;
-        }
-        __syncthreads();
-        const uint32_t T = (top << kSelShift[1]) | sh[0], less = sh[1];
-        uint32_t met = 0;  // keys equal to T so far, in index order
-        for (int64_t b0 = 0; b0 < V; b0 += kSelSortThreads) {
-            const int64_t i = b0 + tid;
-            const uint32_t key = i < V ? keys[i] : 0xFFFFFFFFu;
-            const bool in = i < V && key >> kSelShift[1] == top;
-            if (in && key < T) v[lt + atomicAdd(&sh[2], 1u)] = ((uint64_t)key << 32) | (uint64_t)i;
-            const uint64_t eq = __ballot(in && key == T);
-            if (lane == 0) wc[wave] = (uint32_t)__popcll(eq);
-            __syncthreads();
-            uint32_t r = met;
-            for (int w = 0; w < kSelSortThreads / 64; w++) {
-                if (w < wave) r += wc[w];
-                met += wc[w];
-            }
-            r += (uint32_t)__popcll(eq & ((1ull << lane) - 1ull));
-            if (in && key == T && r < need - less) v[lt + less + r] = ((uint64_t)key << 32) | (uint64_t)i;
-            __syncthreads();
-        }
-        total = k;
-    }
-    int m = 1;
-    while (m < total) m <<= 1;
-    for (int i = total + tid; i < m; i += kSelSortThreads) v[i] = ~0ull;
-    __syncthreads();
-    for (int size = 2; size <= m; size <<= 1) {
-        for (int stride = size >> 1; stride > 0; stride >>= 1) {
-            for (int i = tid; i < m; i += kSelSortThreads) {
-                const int j = i ^ stride;
-                if (j > i) {
-                    const bool up = (i & size) == 0;
-                    const uint64_t a = v[i], b = v[j];
-                    if ((a > b) == up) {
-                        v[i] = b;
-                        v[j] = a;
-                    }
-                }
-            }
-            __syncthreads();
-        }
-    }
-    for (int i = tid; i < k; i += kSelSortThreads) order[i] = (int32_t)(v[i] & 0xFFFFFFFFull);
-}
-
 // Greedy branch (:241-261): best = 0, max = value of index 0, strict '>' ascending; values are
 // sanitized and suppressed ones are -1e9. Equivalent to the lowest index of the maximum, which two
 // launches find: kGreedyParts workgroups take strided ranges of the logits (each thread sees its
@@ -446,12 +364,6 @@ __global__ __launch_bounds__(kGreedyThreads) void sampler_greedy_finish_kernel(c
     }
 }
 
-// Truncations and the draw over at most kSeqTile candidates (top_k <= kSeqTile), in one
-// workgroup: value i is vals[order ? order[i] : i]. The running f32 sums of apply_top_p and
-// apply_min_p are evaluated in candidate order by lane 0 of wave 0 (f32 addition is not
-// associative, so the order fixes the cut). The terms come from two LDS tiles: while lane 0 adds
-// one tile, waves 1-3 compute the next tile's terms into the other. Longer candidate lists take
-// the chunked stages below.
 constexpr int kSeqBlock = 32;   // terms per block of lane 0's adds
 
 // Lane 0's adds over one tile, acc += buf[e] for e in [0, cnt), 32 terms per block with the next
@@ -509,55 +421,6 @@ __device__ __forceinline__ float chain_tile(const float *buf, int cnt, float acc
     return acc;
 }
 
-// acc_i = acc_{i-1} + term(i) in f32 over i in [0, m), m >= 1, in index order. Returns the first
-// i with target <= acc_i (m when none) under kHit, else m; the running sum where the chain
-// stopped goes to total (every thread). Enter and leave with the workgroup converged;
-// tile0/tile1 and n_sh/f_sh are free on entry.
-template <bool kHit, class Term>
-__device__ __forceinline__ int64_t ordered_chain(float *tile0, float *tile1, int64_t m, Term term, float target,
-                                                 float &total, int64_t *n_sh, float *f_sh) {
-    const int tid = threadIdx.x;
-    const int64_t nt = (m + kSeqTile - 1) / kSeqTile;
-    auto tile_cnt = [&](int64_t k) -> int {
-        const int64_t r = m - k * kSeqTile;
-        return (int)(r < kSeqTile ? r : kSeqTile);
-    };
-    {
-        const int c = tile_cnt(0);
-        for (int e = tid; e < c; e += kTailThreads) tile0[e] = term((int64_t)e);
-    }
-    __syncthreads();
-    float acc = 0.0f;
-    int64_t hit = m;
-    for (int64_t k = 0; k < nt; k++) {
-        float *cur = (k & 1) ? tile1 : tile0;
-        float *nxt = (k & 1) ? tile0 : tile1;
-        if (tid < 64) {
-            if (tid == 0) {
-                int he;
-                acc = chain_tile<kHit>(cur, tile_cnt(k), acc, target, he);
-                // two slots: the others read slot k&1 between barriers k and k+1, lane 0 writes
-                // slot (k+1)&1 only after barrier k
-                if (kHit) n_sh[k & 1] = he >= 0 ? k * kSeqTile + he : m;
-            }
-        } else if (k + 1 < nt) {
-            const int64_t base = (k + 1) * kSeqTile;
-            const int c = tile_cnt(k + 1);
-            for (int e = tid - 64; e < c; e += kTailThreads - 64) nxt[e] = term(base + e);
-        }
-        __syncthreads();
-        if (kHit) {
-            hit = n_sh[k & 1];
-            if (hit < m) break;
-        }
-    }
-    if (tid == 0) *f_sh = acc;
-    __syncthreads();
-    total = *f_sh;
-    __syncthreads();
-    return hit;
-}
-
 // Device-side state of the chunked stages: the candidate count as the truncations leave it, the
 // count of chunks a records pass lists as likely slow, the last sum pass's total and min-p's first
 // failing index.
@@ -568,90 +431,182 @@ struct DrawHdr {
     int64_t kept;
 };
 
-__global__ __launch_bounds__(kTailThreads) void sampler_tail_kernel(const float *__restrict__ vals,
-                                                                    const int32_t *__restrict__ order, int64_t V,
-                                                                    SampleParams p, int64_t *out) {
-    __shared__ __align__(16) float tile[2][kSeqTile];
-    __shared__ float red[kTailThreads];
-    __shared__ int64_t n_sh[2];
-    __shared__ float f_sh;
-    const int tid = threadIdx.x;
-    auto val = [&](int64_t i) -> float { return vals[order ? order[i] : i]; };
-    int64_t n = V;
-    if (p.top_k > 0 && p.top_k < n) n = p.top_k;  // apply_top_k (:107-116)
+// Sorts the gathered (key, index) values in LDS, keeps the first k, and makes the truncations and the
+// draw over them; clears the first digit's histogram for the next call. Up to kRankMax values are
+// sorted by rank (each thread counts the values below its own, one barrier), more by a bitonic sort.
+// The tail is in the same workgroup because the sorted candidates are in its LDS already and a launch
+// costs as much as the tail itself. Bound by latency (one workgroup). Measured on MI355X, 128256 logits, top-k 40
+// with top-p: 43.1 -> 37.5 us per blocking call (bitonic sort of 64 values and a 256-thread tail launch before).
+constexpr int kSelSortThreads = 1024;
+constexpr int kRankMax = 256;
+__global__ __launch_bounds__(kSelSortThreads) void sampler_select_draw_kernel(const uint32_t *__restrict__ keys, int64_t V,
+                                                                              uint32_t *__restrict__ hist,
+                                                                              const uint64_t *__restrict__ cand, int k,
+                                                                              const float *__restrict__ vals,
+                                                                              SampleParams p, int64_t *out) {
+    __shared__ __align__(16) uint64_t v[kSeqTile];
+    __shared__ int32_t order[kSeqTile];
+    __shared__ uint32_t lh[kSelLow + 1], wc[kSelSortThreads / 64], sh[4];
+    __shared__ float f_sh[1 + kSelSortThreads / 64];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const uint32_t *ctr = hist + 2 * kSelBins;
+    const int lt = (int)ctr[2];
+    int total = lt + (int)(ctr[1] < (uint32_t)(kSeqTile + 1) ? ctr[1] : kSeqTile + 1);
+    const uint32_t top = ctr[3];
+    for (int i = tid; i < kSelBins; i += kSelSortThreads) hist[i] = 0;
+    const bool all = total <= kSeqTile;
+    for (int i = tid; i < (all ? total : lt); i += kSelSortThreads) v[i] = cand[i];
+    if (!all) {  // the k - lt first (key, index) among those sharing the bits, found by scanning the keys
+        static_assert(kSelSortThreads == (int)kSelLow + 1, "one bin per thread");
+        lh[tid] = 0;
+        __syncthreads();
+        for (int64_t i = tid; i < V; i += kSelSortThreads)
+            if (keys[i] >> kSelShift[1] == top) atomicAdd(&lh[keys[i] & kSelLow], 1u);
+        __syncthreads();
+        const uint32_t mine = lh[tid], need = (uint32_t)(k - lt);
+        for (int o = 1; o < kSelSortThreads; o <<= 1) {  // inclusive sums
+            const uint32_t t = tid >= o ? lh[tid - o] : 0u;
+            __syncthreads();
+            lh[tid] += t;
+            __syncthreads();
+        }
+        if (lh[tid] >= need && lh[tid] - mine < need) {
+            sh[0] = (uint32_t)tid;          // the last digit of the k-th key
+            sh[1] = lh[tid] - mine;         // keys with a smaller one
+            sh[2] = 0;
+        }
+        __syncthreads();
+        const uint32_t T = (top << kSelShift[1]) | sh[0], less = sh[1];
+        uint32_t met = 0;  // keys equal to T so far, in index order
+        for (int64_t b0 = 0; b0 < V; b0 += kSelSortThreads) {
+            const int64_t i = b0 + tid;
+            const uint32_t key = i < V ? keys[i] : 0xFFFFFFFFu;
+            const bool in = i < V && key >> kSelShift[1] == top;
+            if (in && key < T) v[lt + atomicAdd(&sh[2], 1u)] = ((uint64_t)key << 32) | (uint64_t)i;
+            const uint64_t eq = __ballot(in && key == T);
+            if (lane == 0) wc[wave] = (uint32_t)__popcll(eq);
+            __syncthreads();
+            uint32_t r = met;
+            for (int w = 0; w < kSelSortThreads / 64; w++) {
+                if (w < wave) r += wc[w];
+                met += wc[w];
+            }
+            r += (uint32_t)__popcll(eq & ((1ull << lane) - 1ull));
+            if (in && key == T && r < need - less) v[lt + less + r] = ((uint64_t)key << 32) | (uint64_t)i;
+            __syncthreads();
+        }
+        total = k;
+    }
+    if (total <= kRankMax) {
+        __syncthreads();
+        if (tid < total) {
+            const uint64_t mine = v[tid];
+            int r = 0;
+#pragma unroll 8
+            for (int j = 0; j < total; j++) r += v[j] < mine;  // (distinct values: distinct ranks)
+            if (r < k) order[r] = (int32_t)(mine & 0xFFFFFFFFull);
+        }
+    } else {
+        int m = 1;
+        while (m < total) m <<= 1;
+        for (int i = total + tid; i < m; i += kSelSortThreads) v[i] = ~0ull;
+        __syncthreads();
+        for (int size = 2; size <= m; size <<= 1) {
+            for (int stride = size >> 1; stride > 0; stride >>= 1) {
+                for (int i = tid; i < m; i += kSelSortThreads) {
+                    const int j = i ^ stride;
+                    if (j > i) {
+                        const bool up = (i & size) == 0;
+                        const uint64_t a = v[i], b = v[j];
+                        if ((a > b) == up) {
+                            v[i] = b;
+                            v[j] = a;
+                        }
+                    }
+                }
+                __syncthreads();
+            }
+        }
+        for (int i = tid; i < k; i += kSelSortThreads) order[i] = (int32_t)(v[i] & 0xFFFFFFFFull);
+    }
+    __syncthreads();
 
+    // Truncations and the draw over the k candidates. The running f32 sums of apply_top_p, apply_min_p
+    // and the draw are evaluated in candidate order by lane 0 (f32 addition is not associative, so the
+    // order fixes the cut) over terms in LDS. The values and terms take v's place.
+    float *val = reinterpret_cast<float *>(v), *term = val + kSeqTile;
+    for (int i = tid; i < k; i += kSelSortThreads) val[i] = vals[order[i]];
+    __syncthreads();
+    int n = k;
+    const float x0 = val[0];
+    auto exps = [&](float mx) {
+        for (int e = tid; e < n; e += kSelSortThreads) term[e] = exp_f32(val[e] - mx);
+        __syncthreads();
+    };
+    auto sum_terms = [&]() -> float {
+        if (tid == 0) {
+            int he;
+            f_sh[0] = chain_tile<false>(term, n, 0.0f, 0.0f, he);
+        }
+        __syncthreads();
+        return f_sh[0];
+    };
+    auto block_reduce = [&](float x, auto op) -> float {
+        for (int o = 32; o > 0; o >>= 1) x = op(x, __shfl_xor(x, o));
+        if (lane == 0) f_sh[1 + wave] = x;
+        __syncthreads();
+        x = f_sh[1];
+        for (int w = 1; w < kSelSortThreads / 64; w++) x = op(x, f_sh[1 + w]);
+        return x;
+    };
     if (p.top_p < 1.0f && n > 1) {  // apply_top_p (:119-147): exps relative to the first (largest) logit
-        const float mx = val(0);
-        float sum, stop;
-        ordered_chain<false>(tile[0], tile[1], n, [&](int64_t i) { return exp_f32(val(i) - mx); }, 0.0f, sum, n_sh,
-                             &f_sh);
-        const int64_t cut = ordered_chain<true>(
-            tile[0], tile[1], n,
-            [&](int64_t i) {
-                const float e = exp_f32(val(i) - mx);
-                return sum > 0.0f ? e / sum : e;
-            },
-            p.top_p, stop, n_sh, &f_sh);
-        n = cut < n ? cut + 1 : n;
+        exps(x0);
+        const float sum = sum_terms();
+        for (int e = tid; e < n; e += kSelSortThreads) term[e] = sum > 0.0f ? term[e] / sum : term[e];
+        __syncthreads();
+        if (tid == 0) {
+            int he;
+            chain_tile<true>(term, n, 0.0f, p.top_p, he);
+            sh[3] = (uint32_t)(he >= 0 ? he + 1 : n);
+        }
+        __syncthreads();
+        n = (int)sh[3];
     }
     if (p.min_p > 0.0f && p.min_p < 1.0f && n > 1) {  // apply_min_p (:166-194)
-        const float mx = val(0);
-        float sum;
-        ordered_chain<false>(tile[0], tile[1], n, [&](int64_t i) { return exp_f32(val(i) - mx); }, 0.0f, sum, n_sh,
-                             &f_sh);
-        const float e0 = exp_f32(0.0f);  // the first candidate's exp (val(0) - mx = 0)
+        exps(x0);
+        const float sum = sum_terms();
+        const float e0 = exp_f32(0.0f);  // the first candidate's exp (x_0 - x_0 = 0)
         const float p0 = sum > 0.0f ? e0 / sum : e0;
         const float threshold = p.min_p * p0;
         // kept = the first index whose probability falls below the threshold (each test is
-        // independent of the others, so the tile is searched in parallel)
-        int64_t kept = n;
-        for (int64_t t0 = 0; t0 < n && kept == n; t0 += kSeqTile) {
-            const int cnt = (int)(n - t0 < kSeqTile ? n - t0 : kSeqTile);
-            for (int e = tid; e < cnt; e += kTailThreads) tile[0][e] = exp_f32(val(t0 + e) - mx);
-            __syncthreads();
-            int first = cnt;
-            for (int e = tid; e < cnt; e += kTailThreads) {
-                const float pr = sum > 0.0f ? tile[0][e] / sum : tile[0][e];
-                if (!(pr >= threshold)) {
-                    first = e;
-                    break;
-                }
+        // independent of the others, so the terms are searched in parallel)
+        int first = n;
+        for (int e = tid; e < n; e += kSelSortThreads) {
+            const float pr = sum > 0.0f ? term[e] / sum : term[e];
+            if (!(pr >= threshold)) {
+                first = e;
+                break;
             }
-            red[tid] = (float)first;  // exact: indices < 2^24
-            __syncthreads();
-            for (int st = kTailThreads / 2; st > 0; st >>= 1) {
-                if (tid < st) red[tid] = fminf(red[tid], red[tid + st]);
-                __syncthreads();
-            }
-            if ((int)red[0] < cnt) kept = t0 + (int)red[0];
-            __syncthreads();
         }
+        const int kept = (int)block_reduce((float)first, [](float a, float b) { return fminf(a, b); });
         n = kept > 0 ? kept : n;
+        __syncthreads();  // every thread has read f_sh and the terms
     }
-    // At most kSeqTile candidates: the final draw (:284-305) here, its exps in one LDS tile and
-    // both running sums (sum_e, then the inverse-CDF walk) in lane 0 in candidate order.
+    // the final draw (:284-305)
     float mx = -INFINITY;
-    for (int64_t i = tid; i < n; i += kTailThreads) mx = fmaxf(mx, val(i));
-    red[tid] = mx;
-    __syncthreads();
-    for (int st = kTailThreads / 2; st > 0; st >>= 1) {
-        if (tid < st) red[tid] = fmaxf(red[tid], red[tid + st]);
-        __syncthreads();
-    }
-    mx = red[0];
-    for (int e = tid; e < (int)n; e += kTailThreads) tile[0][e] = exp_f32(val(e) - mx);
-    __syncthreads();
+    for (int i = tid; i < n; i += kSelSortThreads) mx = fmaxf(mx, val[i]);
+    mx = block_reduce(mx, [](float a, float b) { return fmaxf(a, b); });
+    exps(mx);
     if (tid == 0) {
         int he;
-        const float sum_e = chain_tile<false>(tile[0], (int)n, 0.0f, 0.0f, he);
+        const float sum_e = chain_tile<false>(term, n, 0.0f, 0.0f, he);
         if (sum_e <= 0.0f) {  // a NaN sum goes on to the walk, as in the reference
-            out[0] = order ? order[0] : 0;
+            out[0] = order[0];
             out[1] = 0;
         } else {
             const float r = p.u * sum_e;
-            chain_tile<true>(tile[0], (int)n, 0.0f, r, he);
-            const int64_t pick = he >= 0 ? he : n - 1;
-            out[0] = order ? order[pick] : pick;
+            chain_tile<true>(term, n, 0.0f, r, he);
+            out[0] = order[he >= 0 ? he : n - 1];
             out[1] = 1;
         }
     }
@@ -1443,7 +1398,6 @@ int32_t aesir_sample_token(aesir_ctx *ctx, const void *logits, int64_t vocab, co
         p.apply_freq = !(cfg->frequency_penalty == 0.0f && cfg->presence_penalty == 0.0f) && n_context > 0;
         p.apply_temp = cfg->temperature > 0.0f && cfg->temperature != 1.0f;
         p.inv_temp = 1.0f / cfg->temperature;
-        p.top_k = cfg->top_k;
         p.top_p = cfg->top_p;
         p.min_p = cfg->min_p;
         const bool k_on = cfg->top_k > 0 && cfg->top_k < vocab;
@@ -1471,21 +1425,16 @@ int32_t aesir_sample_token(aesir_ctx *ctx, const void *logits, int64_t vocab, co
             hipLaunchKernelGGL(sampler_select_gather_kernel, dim3(nb), dim3(kSThreads), 0, s, w->keys, vocab, w->sel_hist, k,
                                w->sel_hist + 2 * kSelBins, w->sel_cand);
             AESIR_LAUNCH_CHECK("sampler_select_gather_kernel");
-            hipLaunchKernelGGL(sampler_select_sort_kernel, dim3(1), dim3(kSelSortThreads), 0, s, w->keys, vocab, w->sel_hist,
-                               w->sel_cand, (int)k, w->idx_out);
-            AESIR_LAUNCH_CHECK("sampler_select_sort_kernel");
+            hipLaunchKernelGGL(sampler_select_draw_kernel, dim3(1), dim3(kSelSortThreads), 0, s, w->keys, vocab, w->sel_hist,
+                               w->sel_cand, (int)k, w->vals, p, w->result);
+            AESIR_LAUNCH_CHECK("sampler_select_draw_kernel");
         } else if (p.sort) {
             size_t bytes = w->sort_tmp_bytes;
             AESIR_HIP_TRY(rocprim::radix_sort_pairs(w->sort_tmp, bytes, w->keys, w->keys_out, w->idx, w->idx_out,
                                                     (unsigned)vocab, 0, 32, s));
         }
         const int32_t *order = p.sort ? (const int32_t *)w->idx_out : nullptr;
-        if (select_k) {
-            // at most one LDS tile of candidates: truncations and the draw in one workgroup
-            hipLaunchKernelGGL(sampler_tail_kernel, dim3(1), dim3(kTailThreads), 0, s, w->vals, order, vocab, p,
-                               w->result);
-            AESIR_LAUNCH_CHECK("sampler_tail_kernel");
-        } else {
+        if (!select_k) {
             // the chunked stages over hdr->n candidates (chunks past the count exit at once): each
             // running sum is a terms pass, a records pass and a walk
             const unsigned nch = (unsigned)((vocab + kDrawChunk - 1) / kDrawChunk);

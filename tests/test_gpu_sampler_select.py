@@ -35,3 +35,22 @@ def test_selection(A, oracle, vocab, levels, top_k, n_context, n_suppress):
             want, o_state = oracle.sample_token_f16(logits, oracle.SamplerConfig(**cfg), o_state, context, suppress)
             assert got == want, d
             assert g_rng.state == o_state, d
+
+
+@pytest.mark.parametrize("top_p,min_p", [(0.9, 0.0), (1.0, 0.02), (0.97, 0.1), (1.0, 0.0), (1e-6, 0.0), (1.0, 0.999)])
+@pytest.mark.parametrize("top_k", [2, 63, 255, 256, 257, 1025, 4096])
+def test_truncations_of_the_selection(A, oracle, top_k, top_p, min_p):
+    """Both sorts of the selecting workgroup (by rank up to 256 gathered candidates, bitonic above) with
+    each truncation behind them; infinities and NaN among the logits are sanitized first."""
+    rng = np.random.default_rng(top_k)
+    cfg = dict(temperature=0.7, top_k=top_k, top_p=top_p, min_p=min_p)
+    g_rng = A.RuneRNG(5)
+    o_state = oracle.rune_rng_state(5)
+    with A.Context(64 << 20) as ctx:
+        for d in range(3):
+            logits = (rng.standard_normal(9000) * (0.3, 2.5, 8.0)[d]).astype(np.float16)
+            logits[rng.integers(0, 9000, 4)] = [np.inf, -np.inf, np.nan, -0.0]
+            got = A.sample_token(ctx, ctx.from_numpy(logits.reshape(1, -1)), A.SamplerConfig(**cfg), g_rng, [], [])
+            want, o_state = oracle.sample_token_f16(logits, oracle.SamplerConfig(**cfg), o_state, [], [])
+            assert got == want, d
+            assert g_rng.state == o_state, d
