@@ -283,8 +283,12 @@ __device__ __forceinline__ int split_count(int64_t S, int64_t max_split) {
     return (int)((rounds + per - 1) / per);
 }
 
-template <int HD, int GH>
-__global__ __launch_bounds__(kAThreads) void attn_fast_kernel(AttnArgs a) {
+// NG > 1 (short views, one split): NG groups of 256 threads share the workgroup; group q takes
+// rounds q, q + NG, ... of the view (every group runs the same number of loop iterations, the
+// surplus ones masked), and the groups' (m, l, acc) are combined in LDS before the output is
+// written, so no merge launch follows.
+template <int HD, int GH, int NG>
+__global__ __launch_bounds__(kAThreads * NG) void attn_fast_kernel(AttnArgs a) {
     constexpr int TPP = HD / 16;              // score threads per K row (16 dims each)
     constexpr int RPP = kAThreads / TPP;      // K rows per score pass
     constexpr int NSP = kRound / RPP;         // score passes per round (2 for HD 128, 1 for HD 64)
@@ -294,12 +298,20 @@ __global__ __launch_bounds__(kAThreads) void attn_fast_kernel(AttnArgs a) {
     constexpr int PVS = kAThreads / kItems;   // PV position groups (1, 2, 4 or 8)
     constexpr int NPOS = kRound / PVS;        // positions per thread per round in the PV pass
     static_assert(NSP * RPP == kRound && NVL * kAThreads == kRound * VCH && kItems * PVS == kAThreads, "shape");
-    __shared__ __align__(16) float sc[GH][kRound];  // scores, then probabilities
-    __shared__ __align__(16) h16 vs[kRound][HD];
-    __shared__ float alpha[GH], mrun[GH], lrun[GH];
-    __shared__ float2 pvx[PVS > 1 ? PVS - 1 : 1][kItems];
+    __shared__ __align__(16) float scs[NG][GH][kRound];  // scores, then probabilities
+    __shared__ __align__(16) h16 vss[NG][kRound][HD];
+    __shared__ float alphas[NG][GH], mruns[NG][GH], lruns[NG][GH];
+    __shared__ float2 pvxs[NG][PVS > 1 ? PVS - 1 : 1][kItems];
+    __shared__ float2 gacc[NG > 1 ? NG - 1 : 1][kItems];
 
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int tid = threadIdx.x % kAThreads, grp = threadIdx.x / kAThreads;  // thread in its group
+    const int lane = tid & 63, wave = tid >> 6;
+    auto &sc = scs[grp];
+    auto &vs = vss[grp];
+    auto &alpha = alphas[grp];
+    auto &mrun = mruns[grp];
+    auto &lrun = lruns[grp];
+    auto &pvx = pvxs[grp];
     const int64_t G = (int64_t)GH * gridDim.z;  // query heads per KV head (the grid's z is G / GH)
     const int g = blockIdx.y, hg = blockIdx.z;
     const int split = blockIdx.x;
@@ -323,6 +335,8 @@ __global__ __launch_bounds__(kAThreads) void attn_fast_kernel(AttnArgs a) {
 
     // K/V requests of one round (rows past p1 re-read row t0 and are masked)
     auto load_round = [&](int64_t t0, u32x4 (&kr)[NSP][2], u32x4 (&vr)[NVL]) {
+        if constexpr (NG > 1)
+            if (t0 >= p1) t0 = p0;  // a group's surplus round re-reads the first round (masked)
         const int n = (int)(p1 - t0 < kRound ? p1 - t0 : kRound);
 #pragma unroll
         for (int i = 0; i < NSP; i++) {
@@ -337,8 +351,11 @@ __global__ __launch_bounds__(kAThreads) void attn_fast_kernel(AttnArgs a) {
             vr[i] = ld16(Vb + (t0 + (r < n ? r : 0)) * a.v_stride + 8 * c);
         }
     };
+    const int nrounds = (int)((p1 - p0 + kRound - 1) / kRound);
+    const int iters = (nrounds + NG - 1) / NG;  // loop iterations of every group
+    auto round_t0 = [&](int j) { return p0 + (int64_t)kRound * (grp + NG * j); };
     u32x4 kr[NSP][2], vr[NVL], kn[NSP][2], vn[NVL];
-    load_round(p0, kr, vr);
+    load_round(NG > 1 ? round_t0(0) : p0, kr, vr);
     u32x4 qr[GH][2];
     {
         const h16 *qb = reinterpret_cast<const h16 *>(a.q) + head0 * HD + 16 * sc_c;
@@ -353,7 +370,7 @@ __global__ __launch_bounds__(kAThreads) void attn_fast_kernel(AttnArgs a) {
     // One round: scores, V to LDS, online softmax, P V. The caller owns the barrier that lets the
     // next round rewrite sc and vs.
     auto round = [&](int64_t t0, const u32x4 (&kc)[NSP][2], const u32x4 (&vc)[NVL]) {
-        const int n_here = (int)(p1 - t0 < kRound ? p1 - t0 : kRound);
+        const int n_here = NG > 1 && t0 >= p1 ? 0 : (int)(p1 - t0 < kRound ? p1 - t0 : kRound);  // 0: surplus round
 #pragma unroll
         for (int i = 0; i < NSP; i++) {
 #pragma unroll
@@ -371,7 +388,7 @@ __global__ __launch_bounds__(kAThreads) void attn_fast_kernel(AttnArgs a) {
         }
         __syncthreads();
         // online softmax of head `wave` over the round (one position per lane)
-        if (wave < GH) {
+        if (wave < GH && (NG == 1 || n_here > 0)) {
             const float s = lane < n_here ? sc[wave][lane] : -INFINITY;
             const float mn = fmaxf(m_w, wave_max(s));
             const float pr = lane < n_here ? expf(s - mn) : 0.0f;
@@ -383,6 +400,7 @@ __global__ __launch_bounds__(kAThreads) void attn_fast_kernel(AttnArgs a) {
         }
         __syncthreads();
         // P V over this thread's positions of the round (probabilities are 0 beyond n_here)
+        if (NG > 1 && n_here == 0) return;
         const float al = alpha[ph];
         acc0 *= al;
         acc1 *= al;
@@ -399,21 +417,77 @@ __global__ __launch_bounds__(kAThreads) void attn_fast_kernel(AttnArgs a) {
     };
     // Rounds with a successor request it before computing (unconditionally, so the compiler's wait
     // counts stay exact and the successor's loads overlap this round); the last round follows.
-    const int64_t step = (int64_t)nsplit * kRound;
-    int64_t t0 = p0;
-    for (; t0 + step < p1; t0 += step) {
-        load_round(t0 + step, kn, vn);
-        round(t0, kr, vr);
+    if constexpr (NG == 1) {
+        const int64_t step = (int64_t)nsplit * kRound;
+        int64_t t0 = p0;
+        for (; t0 + step < p1; t0 += step) {
+            load_round(t0 + step, kn, vn);
+            round(t0, kr, vr);
 #pragma unroll
-        for (int i = 0; i < NSP; i++) {
-            kr[i][0] = kn[i][0];
-            kr[i][1] = kn[i][1];
+            for (int i = 0; i < NSP; i++) {
+                kr[i][0] = kn[i][0];
+                kr[i][1] = kn[i][1];
+            }
+#pragma unroll
+            for (int i = 0; i < NVL; i++) vr[i] = vn[i];
+            __syncthreads();  // sc and vs are rewritten by the next round
         }
+        round(t0, kr, vr);
+    } else {
+        int j = 0;
+        for (; j + 1 < iters; j++) {
+            load_round(round_t0(j + 1), kn, vn);
+            round(round_t0(j), kr, vr);
 #pragma unroll
-        for (int i = 0; i < NVL; i++) vr[i] = vn[i];
-        __syncthreads();  // sc and vs are rewritten by the next round
+            for (int i = 0; i < NSP; i++) {
+                kr[i][0] = kn[i][0];
+                kr[i][1] = kn[i][1];
+            }
+#pragma unroll
+            for (int i = 0; i < NVL; i++) vr[i] = vn[i];
+            __syncthreads();
+        }
+        round(round_t0(j), kr, vr);
     }
-    round(t0, kr, vr);
+
+    if constexpr (NG > 1) {  // combine the groups (one split: the output is written here)
+        if (wave < GH && lane == 0) {
+            mrun[wave] = m_w;
+            lrun[wave] = l_w;
+        }
+        if (PVS > 1 && pg > 0) pvx[pg - 1][item] = float2{acc0, acc1};
+        __syncthreads();
+        if (pg == 0) {
+#pragma unroll
+            for (int q = 0; q < PVS - 1; q++) {
+                const float2 o = pvx[q][item];
+                acc0 += o.x;
+                acc1 += o.y;
+            }
+            if (grp > 0) gacc[grp - 1][item] = float2{acc0, acc1};
+        }
+        __syncthreads();
+        if (grp == 0 && pg == 0) {
+            float M = mruns[0][ph];
+#pragma unroll
+            for (int q = 1; q < NG; q++) M = fmaxf(M, mruns[q][ph]);  // group 0 always has a round
+            float L = lruns[0][ph] * expf(mruns[0][ph] - M);
+            acc0 *= expf(mruns[0][ph] - M);
+            acc1 *= expf(mruns[0][ph] - M);
+#pragma unroll
+            for (int q = 1; q < NG; q++) {
+                const float e = expf(mruns[q][ph] - M);  // 0 for a group without rounds
+                const float2 o = gacc[q - 1][item];
+                L = fmaf(lruns[q][ph], e, L);
+                acc0 = fmaf(o.x, e, acc0);
+                acc1 = fmaf(o.y, e, acc1);
+            }
+            h16 *out = reinterpret_cast<h16 *>(a.out) + (head0 + ph) * HD + pd;
+            out[0] = (h16)(acc0 / L);
+            out[1] = (h16)(acc1 / L);
+        }
+        return;
+    }
 
     // Write the partial (or the output for one split). With one PV position group and one head
     // per wave (head_dim 128, 4 heads per workgroup), thread t's head is its wave's, whose
@@ -552,18 +626,22 @@ __global__ __launch_bounds__(kAThreads) void attn_fast_merge_kernel(AttnArgs a) 
 
 // ------------------------------------------------------------------ short views
 //
-// One workgroup per query head over a view of at most 512 positions (256 at head_dim 128), one launch and
+// One workgroup per query head over a view of short_view_max(head_dim) positions at most, one launch and
 // one barrier: wave w owns positions PW w .. + PW - 1 and requests all of their K and V rows and the q row
 // at once, so a launch costs one memory round trip. Lane l holds dims 8 (l % CH) .. + 7 of the K and V
 // rows l / CH, + 64 / CH, .. (whole rows per load). Per wave: scores summed over the CH lanes of a row,
 // the wave's own softmax maximum and sum (f32, no exchange with the other waves), P V with the
 // probability already in the row's lanes, and the lanes of one dim chunk summed. The waves' (m, l, O)
-// meet in LDS. Bound by latency (a view is tens of KB). Measured on MI355X, us per launch inside a
-// decode step: head_dim 8, 81 positions 3.1 (5.4 + 2.8 as splits of 64 positions and their merge before);
-// head_dim 64, 8 heads per KV head, 384 positions 5.8 (6.3 with two rounds of 64 positions per group of
-// 256 threads and three barriers a round). The stories260K-shape step at position 80 158 -> 140 us, the
-// TinyLlama one at 440 690 -> 668. Not faster: two lanes per K row (each load then touches 32 lines: 715),
-// waiting for the position first.
+// meet in LDS. Bound by latency (a view is tens of KB). A decode step costs the same at every position,
+// since the rows up to the view's capacity are requested before the position is known (waiting for it
+// first is slower still), so the views it takes are those where that is no more than the position's own
+// share costs elsewhere. Measured on MI355X, us per step of the device loop, this kernel against the others at
+// an early and a late position: 5 layers of head_dim 8 at 512 rows 93 against 106 and 115 (splits of 64
+// positions and their merge); 8 of head_dim 16 140 against 158 and 176; 8 of head_dim 32 176 against 180 and
+// 198; 22 of head_dim 64 (8 heads per KV head) 566 against 578 at 64 rows, but 589 against 578 and 581 at
+// 128, 600 against 579 and 591 at 256 and 634 against 578 and 634 at 448 rows; 4 of head_dim 128 337.5
+// against 339 and 340 at 128 rows, 342 against 339 and 350 at 256. Not faster: two lanes per K row (each
+// load then touches 32 lines).
 template <int HD>
 __global__ __launch_bounds__(1024) void attn_short_kernel(AttnArgs a) {
     constexpr int CH = HD / 8;                       // lanes (16-byte chunks) per row
@@ -670,10 +748,13 @@ static int fast_group(const AttnArgs &a) {
     return G % 4 == 0 ? 4 : G % 2 == 0 ? 2 : 1;
 }
 
-// Views of at most this many positions run as one split (attn_short_kernel).
-static int64_t single_split_max(int64_t hd) {
-    return hd == 8 || hd == 16 || hd == 32 || hd == 64 ? 512 : hd == 128 ? 256 : 0;
-}
+// Views of at most this many positions run on attn_short_kernel (both sides of each line are measured there).
+static int64_t short_view_max(int64_t hd) { return hd == 8 || hd == 16 || hd == 32 ? 512 : hd == 64 ? 64 : hd == 128 ? 128 : 0; }
+
+// Views of at most this many positions run as one split: attn_short_kernel, or (head_dim 64 and 128)
+// one workgroup per head group with groups of 256 threads taking two rounds each at most, and no
+// merge launch.
+static int64_t single_split_max(int64_t hd) { return hd == 64 ? 8 * kRound : hd == 128 ? 4 * kRound : short_view_max(hd); }
 
 // Split count: one split for short views (above); otherwise one 64-position round per split up
 // to 64 splits (more splits cost more in the merge than they gain in parallelism on MI355X;
@@ -701,7 +782,7 @@ int32_t launch_attention_decode(hipStream_t s, const AttnArgs &a) {
         return fail(AESIR_ERR_UNSUPPORTED, "attention: query group x head_dim too large");
     if (a.max_split < 1 || a.max_split > kMaxFastSplit) return fail(AESIR_ERR_INVALID, "attention: bad split count");
     if (a.hd / 2 > kMergeThreads * 64) return fail(AESIR_ERR_UNSUPPORTED, "attention: head_dim too large for the merge");
-    if (a.max_split == 1 && a.max_seq <= single_split_max(a.hd) && a.nq <= 65535 && rows_16(a)) {
+    if (a.max_split == 1 && a.max_seq <= short_view_max(a.hd) && a.nq <= 65535 && rows_16(a)) {
         const int pw = a.hd >= 64 ? 32 : 64;  // positions per wave (attn_short_kernel)
         const dim3 grid((unsigned)a.nq), block((unsigned)((a.max_seq + pw - 1) / pw * kWave));
 #define AESIR_ATTN_SHORT(HDV) \
@@ -715,10 +796,28 @@ int32_t launch_attention_decode(hipStream_t s, const AttnArgs &a) {
         AESIR_LAUNCH_CHECK("attn_short_kernel");
         return AESIR_OK;
     }
+    if (const int gh = fast_group(a); gh && a.max_split == 1) {
+        // one split: NG groups per workgroup (4 for head_dim 64 with one head per workgroup, 2
+        // for head_dim 128 with up to 4, whose registers allow only 2 groups), no merge. One head
+        // per workgroup at head_dim 64 doubles the workgroups of a short view (K/V rows are then
+        // read once per head, from L2): TinyLlama decode 1612 -> 1635 tok/s against 2 heads.
+        const int gs = a.hd == 64 ? 1 : gh;
+        const dim3 grid(1u, (unsigned)a.nkv, (unsigned)(G / gs));
+#define AESIR_ATTN_ONE(HDV, GHV, NGV)                                                          \
+    if (a.hd == HDV && gs == GHV) hipLaunchKernelGGL((attn_fast_kernel<HDV, GHV, NGV>), grid, dim3(kAThreads * NGV), 0, s, a);
+        AESIR_ATTN_ONE(128, 4, 2)
+        AESIR_ATTN_ONE(128, 2, 2)
+        AESIR_ATTN_ONE(128, 1, 2)
+        AESIR_ATTN_ONE(64, 2, 4)
+        AESIR_ATTN_ONE(64, 1, 4)
+#undef AESIR_ATTN_ONE
+        AESIR_LAUNCH_CHECK("attn_fast_kernel (one split)");
+        return AESIR_OK;
+    }
     if (const int gh = fast_group(a)) {
         const dim3 grid((unsigned)a.max_split, (unsigned)a.nkv, (unsigned)(G / gh));
 #define AESIR_ATTN_FAST(HDV, GHV)                                                              \
-    if (a.hd == HDV && gh == GHV) hipLaunchKernelGGL((attn_fast_kernel<HDV, GHV>), grid, dim3(kAThreads), 0, s, a);
+    if (a.hd == HDV && gh == GHV) hipLaunchKernelGGL((attn_fast_kernel<HDV, GHV, 1>), grid, dim3(kAThreads), 0, s, a);
         AESIR_ATTN_FAST(128, 4)
         AESIR_ATTN_FAST(128, 2)
         AESIR_ATTN_FAST(128, 1)
