@@ -273,8 +273,9 @@ __global__ __launch_bounds__(kThreads) void gemv_fixed_kernel(const h16 *__restr
     epi.template apply<ROWS>(n0, m, N, RowSums<ROWS>{red}, tid, pre);
 }
 
-// Final argmax over ordered partials (one workgroup). Writes *result (device or pinned host memory) and/or the decode state:
-// next_token, and in autoregressive mode token <- next, pos += 1, step += 1, ring[step] = next.
+// Final argmax over ordered partials (one workgroup). Writes *result (device or pinned host memory) and/or
+// the decode state: next_token, and in autoregressive mode (whose host reads the ring, so *result is not
+// written) token <- next, pos += 1, step += 1, ring[step] = next.
 // Partial g is the first maximum of an index range below partial g + 1's, so the answer is the
 // smallest index among the partials holding the largest value, whatever order they are visited
 // in: thread t keeps the first maximum of partials t, t + 1024, ... (coalesced loads, 16 in
@@ -319,7 +320,6 @@ __global__ __launch_bounds__(kFinishThreads) void argmax_finish_kernel(const Arg
 #pragma unroll
     for (int w = 1; w < kFinishWaves; w++) bi = min(bi, widx[w]);
     const int64_t idx = (vmax > kArgmaxFloor && bi != INT32_MAX && bi >= 0) ? (int64_t)bi : 0;
-    if (result) *result = idx;
     if (state) {
         state->next_token = idx;
         if (state->advance) {
@@ -327,8 +327,10 @@ __global__ __launch_bounds__(kFinishThreads) void argmax_finish_kernel(const Arg
             state->token = idx;
             state->pos = state->pos + 1;
             state->step = state->step + 1;
+            return;
         }
     }
+    if (result) *result = idx;
 }
 
 // ------------------------------------------------------------------ Q8_0 weights

@@ -229,7 +229,7 @@ struct LmHeadArgs {
     int64_t *ring;  // token ring (autoregressive loop), may be null
     const void *w_scale;  // Q8_0 lm_head scales (w is then int8), or null
     QFMat wq;             // Q4_0 / Q4_K / Q6_K lm_head (w and w_scale unused)
-    int64_t *host_next = nullptr;  // pinned host word that receives the greedy token too
+    int64_t *host_next = nullptr;  // pinned host word that receives the greedy token too, unless the state advances by itself
 };
 int32_t launch_lm_head_argmax(hipStream_t s, const LmHeadArgs &a);
 int32_t launch_lm_head(hipStream_t s, const LmHeadArgs &a);

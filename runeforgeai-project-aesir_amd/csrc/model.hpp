@@ -117,7 +117,7 @@ struct aesir_model {
     int64_t pf_part_floats = 0;
     void *lm_parts = nullptr;
     aesir::DecodeState *state = nullptr;  // device
-    int64_t *next_host = nullptr;         // pinned: the greedy token of the last pass
+    int64_t *next_host = nullptr;         // pinned: the greedy token of the last blocking pass
     int64_t *ring = nullptr;
     int64_t ring_cap = 0;
     const void *rope = nullptr;
