@@ -1130,12 +1130,15 @@ __global__ __launch_bounds__(kWave) void prefill_attention_kernel(const h16 *__r
 //           16 t + 4 (l / 16) + i of sub-tile t; keys past a row's position are masked (only in the
 //           tiles that hold such a key)
 //   softmax f32 online softmax per query in base 2 (scores times scale log2 e): the lane's 16
-//           values, then lanes l ^ 16, l ^ 32 (permlane swaps)
+//           values, then lanes l ^ 16, l ^ 32 (permlane swaps). The running reference is the maximum
+//           rounded up to a whole number, so every rescaling is an exact power of two, and
+//           probabilities carry a factor 2^15 that the division by their sum takes out again
 //   P V     O[16 queries][16 dims] += P V per 32-key step, A = the probabilities as they sit in
 //           the score registers (slot 4 t + i of lane group q is key 16 t + 4 q + i), split into
-//           two f16 terms (hi = f16(p), lo = f16(p - hi)) so that they keep f32 precision; B = V
-//           read transposed from LDS with ds_read_b64_tr_b16 (V chunk c of row m at slot
-//           c ^ 2 ((m / RPS) & SWM), which spreads the transposed reads over the banks)
+//           two f16 terms (hi = f16(p), lo = f16(p - hi)): 22 bits of every probability from 2^-18 of
+//           the largest up, and 2^-40 of the largest below (the factor 2^15 keeps them off f16's
+//           subnormals); B = V read transposed from LDS with ds_read_b64_tr_b16 (V chunk c of row m
+//           at slot c ^ 2 ((m / RPS) & SWM), which spreads the transposed reads over the banks)
 // A tile entirely past a wave's last row is skipped by that wave. The key groups meet in LDS at the
 // end. With gridDim.z > 1 each z takes a contiguous share of the tiles and leaves (m, l, O) in f32
 // for prefill_attention_merge_kernel: short chunks after a long history, whose row blocks alone
@@ -1149,6 +1152,7 @@ __global__ __launch_bounds__(kWave) void prefill_attention_kernel(const h16 *__r
 typedef short short4_t __attribute__((ext_vector_type(4)));
 typedef float f32x2 __attribute__((ext_vector_type(2)));
 constexpr int kPfBK = 64;            // keys per tile
+constexpr float kPfPScale = 15.0f;   // log2 of the probabilities' factor: at most 2^15 in f16
 template <int HD, int G, int WV, int KS>
 __global__ __launch_bounds__(KS *WV *kWave) void prefill_attention_mfma_kernel(
     const h16 *__restrict__ Q, const h16 *__restrict__ kc, const h16 *__restrict__ vc, h16 *__restrict__ out,
@@ -1260,7 +1264,7 @@ __global__ __launch_bounds__(KS *WV *kWave) void prefill_attention_mfma_kernel(
         mx = swap_pair_max<32>(swap_pair_max<16>(mx));
         const bool grows = mx > m_run;
         if (__builtin_amdgcn_ballot_w64(grows) != 0) {  // some query's maximum moves: rescale l and O
-            const float mn = fmaxf(m_run, mx);
+            const float mn = fmaxf(m_run, ceilf(mx));
             const float al = grows ? __builtin_amdgcn_exp2f(m_run - mn) : 1.0f;  // 0 on the query's first keys
             l_run *= al;
             m_run = mn;
@@ -1275,7 +1279,7 @@ __global__ __launch_bounds__(KS *WV *kWave) void prefill_attention_mfma_kernel(
                 for (int i = 0; i < 4; i++) o[nt][i] *= alr[i];
         }
         // a query without a key in this tile and before it has m_run = -inf: every p is then 0
-        const float mref = m_run == -INFINITY ? 0.0f : m_run;
+        const float mref = (m_run == -INFINITY ? 0.0f : m_run) - kPfPScale;
         float ps = 0.0f;
         u32x4 ph[2], pl[2];  // k-steps: keys of sub-tiles 2 kk and 2 kk + 1
 #pragma unroll

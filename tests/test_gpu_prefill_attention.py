@@ -43,3 +43,45 @@ def test_chunk_after_history(A, oracle, dim, heads, kv, first, n):
         m.close()
     want = np.asarray(want, np.float64)
     assert np.all(np.abs(got - want) <= 2e-2 + 1e-2 * np.abs(want))
+
+
+@pytest.mark.parametrize("hd,heads,kv,first,n", [(64, 8, 1, 0, 202), (64, 8, 1, 600, 40), (64, 4, 4, 0, 202),
+                                                 (128, 8, 2, 0, 202), (128, 4, 2, 300, 60), (128, 8, 1, 0, 300)])
+def test_small_probabilities_are_kept(A, hd, heads, kv, first, n):
+    """One key holds nearly all of the last query's weight and has V = 0; every other key holds 2^-26 of it
+    and a large V, so the output is what the small probabilities carry. Everything else of the model is the
+    identity or zero: norms of one-hot rows, RoPE at the pair that does not turn, no feed-forward. A whole
+    position's worth of f32 sums stays far inside 1/64; f16 alone would drop every one of those keys."""
+    dim, total = heads * hd, first + n
+    names = ["attn_q", "attn_k", "attn_v", "attn_output", "ffn_gate", "ffn_up", "ffn_down"]
+    kvd, ffn, vocab = kv * hd, 256, 8
+    shapes = dict(zip(names, [(dim, dim), (kvd, dim), (kvd, dim), (dim, dim), (ffn, dim), (ffn, dim), (dim, ffn)]))
+    w = {"blk.0.%s.weight" % x: np.zeros(s, np.float16) for x, s in shapes.items()}
+    for x in ("blk.0.attn_norm", "blk.0.ffn_norm", "output_norm"):
+        w[x + ".weight"] = np.ones((1, dim), np.float16)
+    emb, head = np.zeros((vocab, dim), np.float16), np.zeros((vocab, dim), np.float16)
+    heavy, light, query = 1, 2, 3
+    for t in (heavy, light, query):
+        emb[t, t] = 1.0
+    unit = np.float16(1.0 / np.sqrt(1.0 / dim + 1e-5))  # a one-hot row after its norm
+    a = np.float16(np.sqrt(26 * np.log(2.0) * np.sqrt(hd)) / unit)
+    w["blk.0.attn_q.weight"][hd - 2::hd, query] = a
+    w["blk.0.attn_k.weight"][hd - 2::hd, heavy] = a
+    w["blk.0.attn_v.weight"][:, light] = 40.0
+    w["blk.0.attn_output.weight"][100, 0] = 1.0
+    head[5, 100] = 1.0
+    w["token_embd.weight"], w["output.weight"] = emb, head
+    prompt = [heavy] + [light] * (total - 2) + [query]
+    with A.Context(256 << 20) as ctx:
+        m = A.Model.create(ctx, A.ModelConfig(dim, 1, heads, kv, ffn, vocab, total + 4, 1e-5, 1e12, 1, -1))
+        m.set_weights(w)
+        if first:
+            m.prefill(prompt[:first])
+        m.prefill(prompt[first:], start_pos=first)
+        got = float(m.logits()[5])
+        m.close()
+    q = float(np.float16(unit * a))
+    small = (total - 2) * np.exp(-q * q / np.sqrt(hd))
+    out = small / (1.0 + small) * float(np.float16(unit * np.float16(40.0)))
+    want = out / np.sqrt((1.0 + out * out) / dim + 1e-5)
+    assert abs(got - want) <= want / 64, (got, want)
