@@ -1139,6 +1139,9 @@ __global__ __launch_bounds__(kWave) void prefill_attention_kernel(const h16 *__r
 //           the largest up, and 2^-40 of the largest below (the factor 2^15 keeps them off f16's
 //           subnormals); B = V read transposed from LDS with ds_read_b64_tr_b16 (V chunk c of row m
 //           at slot c ^ 2 ((m / RPS) & SWM), which spreads the transposed reads over the banks)
+// A masked key's probability is 0, and so is its product with a V that is finite. V elements that are not
+// finite go into LDS as 0 and are added in f32 at the end for the queries that see their key, so that a row of
+// the chunk whose V overflows leaves the rows before it as they are.
 // A tile entirely past a wave's last row is skipped by that wave. The key groups meet in LDS at the
 // end. With gridDim.z > 1 each z takes a contiguous share of the tiles and leaves (m, l, O) in f32
 // for prefill_attention_merge_kernel: short chunks after a long history, whose row blocks alone
@@ -1174,6 +1177,7 @@ __global__ __launch_bounds__(KS *WV *kWave) void prefill_attention_mfma_kernel(
     static_assert(KS == 1 || KS == 2, "one exchange of the second key group");
     static_assert(KS == 1 || WV * (kWave * NT * 16 + 32 * 4) <= KS * TB, "the second group's O fits the tiles' LDS");
     __shared__ __align__(16) uint8_t smem[KS * TB];
+    __shared__ int odd[KS];                // the first tile whose V holds elements that are not finite
     const int tid = threadIdx.x, lane = tid & 63;
     const int kg = tid / GT, gt = tid % GT, wave = gt >> 6;  // key group, thread and wave in it
     uint8_t *kbase = smem + kg * TB, *vs = kbase + KB;
@@ -1222,10 +1226,28 @@ __global__ __launch_bounds__(KS *WV *kWave) void prefill_attention_mfma_kernel(
     f32x4 o[NT];
 #pragma unroll
     for (int t = 0; t < NT; t++) o[t] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    if (gt == 0) odd[kg] = INT_MAX;
     if (niter > 0) load_tile((tl0 + kg) * kPfBK);
     for (int it = 0; it < niter; it++) {
         const int tile = tl0 + it * KS + kg, t0 = tile * kPfBK;
         __syncthreads();  // the previous tiles are no longer read
+        {  // x * 0 + 0 is 0 for every finite x and NaN for the others
+            h16x2 z = {(h16)0.0f, (h16)0.0f};
+#pragma unroll
+            for (int i = 0; i < NLD; i++)
+#pragma unroll
+                for (int w = 0; w < 4; w++) z = __builtin_elementwise_fma(as_h2(vr[i][w]), h16x2{(h16)0.0f, (h16)0.0f}, z);
+            if (h2_bits(z) != 0) {
+                atomicMin(&odd[kg], tile);
+#pragma unroll
+                for (int i = 0; i < NLD; i++)
+#pragma unroll
+                    for (int w = 0; w < 4; w++) {
+                        if ((vr[i][w] & 0x7c00u) == 0x7c00u) vr[i][w] &= 0xffff0000u;
+                        if ((vr[i][w] & 0x7c000000u) == 0x7c000000u) vr[i][w] &= 0xffffu;
+                    }
+            }
+        }
 #pragma unroll
         for (int i = 0; i < NLD; i++) {
             const int e = gt + i * GT, row = e / CH, c = e % CH;
@@ -1315,6 +1337,27 @@ __global__ __launch_bounds__(KS *WV *kWave) void prefill_attention_mfma_kernel(
         for (int i = 0; i < 4; i++)
             r[i] = __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute(4 * (4 * q4 + i), __builtin_bit_cast(int, v)));
     };
+    if (niter > 0 && odd[kg] != INT_MAX) {  // (every write to it lies before the last round's second barrier)
+        const float mref = (m_run == -INFINITY ? 0.0f : m_run) - kPfPScale;
+#pragma unroll 1
+        for (int tile = odd[kg]; tile < tl1; tile += KS)
+#pragma unroll 1
+            for (int key = tile * kPfBK; key < (tile + 1) * kPfBK && key < (int)kend; key++) {
+                float d = 0.0f, pq[4];
+#pragma unroll
+                for (int j = 0; j < NJ; j++) d = dot8(ld16(Kg + key * kvd + 32 * j + 8 * q4), qb[j], d);
+                d = swap_pair_sum<16>(d, d);
+                d = swap_pair_sum<32>(d, d);
+                spread(__builtin_amdgcn_exp2f(d * scale2 - mref), pq);
+#pragma unroll
+                for (int nt = 0; nt < NT; nt++) {
+                    const float v = (float)Vg[key * kvd + 16 * nt + c16];
+#pragma unroll
+                    for (int i = 0; i < 4; i++)
+                        if (v - v != 0.0f && key <= (int)(p0 + r0w) + 4 * q4 + i) o[nt][i] = fmaf(pq[i], v, o[nt][i]);
+                }
+            }
+    }
     if constexpr (KS == 2) {
         // group 1 hands (m, l, O) to the group-0 wave of the same rows and head through the tiles'
         // LDS: w = 2^(m_g - max m) per query, l = sum w l_g, O = sum w O_g

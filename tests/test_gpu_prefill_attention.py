@@ -85,3 +85,46 @@ def test_small_probabilities_are_kept(A, hd, heads, kv, first, n):
     out = small / (1.0 + small) * float(np.float16(unit * np.float16(40.0)))
     want = out / np.sqrt((1.0 + out * out) / dim + 1e-5)
     assert abs(got - want) <= want / 64, (got, want)
+
+
+@pytest.mark.parametrize("hd,heads,kv,first,n,bad_at", [
+    (64, 8, 1, 0, 40, 30), (64, 8, 1, 0, 300, 130), (64, 8, 1, 600, 37, 20), (64, 8, 2, 0, 70, 64), (64, 4, 2, 300, 33, 1),
+    (64, 4, 4, 10, 64, 50), (128, 8, 1, 0, 40, 15), (128, 8, 2, 500, 37, 12), (128, 4, 2, 0, 100, 63), (128, 4, 4, 0, 270, 200),
+    (32, 8, 2, 0, 40, 30),
+])
+def test_a_later_row_does_not_reach_earlier_ones(A, oracle, hd, heads, kv, first, n, bad_at):
+    """A token of the chunk whose K and V overflow to infinity: the rows before it come out as with any other
+    token there, bit for bit (their second-layer K and V are read back by a step at that position)."""
+    total = first + n
+    cfg = oracle.Config(dim=heads * hd, n_layers=2, n_heads=heads, n_kv_heads=kv, ffn=256, vocab=64, ctx_len=total + 4)
+    w = oracle.synthetic_weights(cfg, 4, norm_mean=1.0)
+    bad = 63
+    emb = w["token_embd.weight"]
+    emb[:, 0] = 0.0
+    emb[bad] = 0.0
+    emb[bad, 0] = 1.0
+    for i in range(cfg.n_layers):
+        for t in ("attn_k", "attn_v"):
+            w["blk.%d.%s.weight" % (i, t)][:, 0] = np.float16(60000.0)  # the other tokens have nothing at dim 0 ..
+        for t in ("attn_output", "ffn_down"):
+            w["blk.%d.%s.weight" % (i, t)][0] = 0.0  # .. in any layer
+    prompt = [1 + (5 * i) % 60 for i in range(total)]
+    at = first + bad_at
+    with A.Context(256 << 20) as ctx:
+        m = A.Model.create(ctx, A.ModelConfig(cfg.dim, cfg.n_layers, cfg.n_heads, cfg.n_kv_heads, cfg.ffn, cfg.vocab,
+                                              cfg.ctx_len, cfg.eps, cfg.theta, 1, -1))
+        m.set_weights(w)
+        got = []
+        for tok in (prompt[at], bad):
+            chunk = list(prompt)
+            chunk[at] = tok
+            if first:
+                m.prefill(chunk[:first])
+            m.prefill(chunk[first:], start_pos=first)
+            last = m.logits().astype(np.float32)
+            assert np.isfinite(last).all() == (tok != bad)  # later rows do see it
+            m.forward_pass(prompt[:at + 1], at)
+            got.append(m.logits())
+        m.close()
+    assert np.isfinite(got[0].astype(np.float32)).all()
+    assert np.array_equal(got[0].view(np.uint16), got[1].view(np.uint16))
