@@ -10,9 +10,10 @@
 //
 // In hipBLASLt's column-major terms D^T [N][M] = op(W) A^T with op = transpose on W stored as
 // K x N (leading dimension K), A^T as K x M (leading dimension K) and D^T as N x M (leading
-// dimension N, i.e. row-major [M][N]). The algorithm is the library heuristic's first choice for
-// the shape (deterministic for a given library and device), cached per context with its
-// descriptors.
+// dimension N, i.e. row-major [M][N]). The algorithm is the first of the library heuristic's choices
+// for the shape that it also runs (deterministic for a given library and device), cached per context with
+// its descriptors: for some shapes the first choice, one that splits the sum over a workspace, is refused at
+// the call (internal error; e.g. 256 x 4096 x 14336 and 804 x 2048 x 5632, 100 of 3600 products tried).
 #include <hipblaslt/hipblaslt.h>
 
 #include <vector>
@@ -25,14 +26,13 @@ namespace {
 
 struct BlasPlan {
     int64_t M = 0, N = 0, K = 0;
-    bool ok = false;
     hipblasLtMatmulDesc_t desc = nullptr;
     hipblasLtMatrixLayout_t la = nullptr, lb = nullptr, ld = nullptr;
-    hipblasLtMatmulAlgo_t algo{};
-    size_t ws = 0;
+    std::vector<hipblasLtMatmulHeuristicResult_t> algos;  // not refused yet, in the heuristic's order
 };
 
 constexpr size_t kMaxPlans = 256;
+constexpr int kMaxAlgos = 8;
 
 struct BlasState {
     hipblasLtHandle_t handle = nullptr;
@@ -47,7 +47,7 @@ void destroy_plan(BlasPlan &p) {
     p = BlasPlan{};
 }
 
-// Builds the descriptors and picks the algorithm for one shape; p.ok stays false when the library
+// Builds the descriptors and lists the algorithms for one shape; p.algos stays empty when the library
 // offers none within the workspace.
 void make_plan(hipblasLtHandle_t h, BlasPlan &p, size_t ws_bytes) {
     const hipblasOperation_t ta = HIPBLAS_OP_T, tb = HIPBLAS_OP_N;
@@ -61,18 +61,15 @@ void make_plan(hipblasLtHandle_t h, BlasPlan &p, size_t ws_bytes) {
     hipblasLtMatmulPreference_t pref = nullptr;
     if (hipblasLtMatmulPreferenceCreate(&pref) != HIPBLAS_STATUS_SUCCESS) return;
     const uint64_t wsl = ws_bytes;
-    hipblasLtMatmulHeuristicResult_t res[1];
+    hipblasLtMatmulHeuristicResult_t res[kMaxAlgos];
     int n = 0;
     const bool got = hipblasLtMatmulPreferenceSetAttribute(pref, HIPBLASLT_MATMUL_PREF_MAX_WORKSPACE_BYTES, &wsl,
                                                            sizeof(wsl)) == HIPBLAS_STATUS_SUCCESS &&
-                     hipblasLtMatmulAlgoGetHeuristic(h, p.desc, p.la, p.lb, p.ld, p.ld, pref, 1, res, &n) ==
-                         HIPBLAS_STATUS_SUCCESS &&
-                     n > 0 && res[0].state == HIPBLAS_STATUS_SUCCESS && res[0].workspaceSize <= ws_bytes;
+                     hipblasLtMatmulAlgoGetHeuristic(h, p.desc, p.la, p.lb, p.ld, p.ld, pref, kMaxAlgos, res, &n) ==
+                         HIPBLAS_STATUS_SUCCESS;
     (void)hipblasLtMatmulPreferenceDestroy(pref);
-    if (!got) return;
-    p.algo = res[0].algo;
-    p.ws = res[0].workspaceSize;
-    p.ok = true;
+    for (int i = 0; got && i < n; i++)
+        if (res[i].state == HIPBLAS_STATUS_SUCCESS && res[i].workspaceSize <= ws_bytes) p.algos.push_back(res[i]);
 }
 
 }  // namespace
@@ -104,14 +101,17 @@ int32_t blas_gemm_nt(aesir_ctx *ctx, hipStream_t s, const void *A, int64_t M, in
         st->plans.push_back(p);
         plan = &st->plans.back();
     }
-    if (!plan->ok) return fail(AESIR_ERR_UNSUPPORTED, "hipBLASLt offers no algorithm for %lld x %lld x %lld",
-                               (long long)M, (long long)N, (long long)K);
     const float alpha = 1.0f, beta = 0.0f;
-    if (hipblasLtMatmul(st->handle, plan->desc, &alpha, W, plan->la, A, plan->lb, &beta, D, plan->ld, D, plan->ld,
-                        &plan->algo, plan->ws ? ws : nullptr, plan->ws, s) != HIPBLAS_STATUS_SUCCESS)
-        return fail(AESIR_ERR_HIP, "hipblasLtMatmul failed (%lld x %lld x %lld)", (long long)M, (long long)N,
-                    (long long)K);
-    return AESIR_OK;
+    while (!plan->algos.empty()) {
+        const hipblasLtMatmulHeuristicResult_t &r = plan->algos.front();
+        if (hipblasLtMatmul(st->handle, plan->desc, &alpha, W, plan->la, A, plan->lb, &beta, D, plan->ld, D, plan->ld, &r.algo,
+                            r.workspaceSize ? ws : nullptr, r.workspaceSize, s) == HIPBLAS_STATUS_SUCCESS)
+            return AESIR_OK;
+        plan->algos.erase(plan->algos.begin());
+        (void)hipGetLastError();  // what the refused launch left behind
+    }
+    return fail(AESIR_ERR_UNSUPPORTED, "hipBLASLt offers no algorithm for %lld x %lld x %lld", (long long)M, (long long)N,
+                (long long)K);
 }
 
 void blas_release(aesir_ctx *ctx) {
