@@ -1121,10 +1121,11 @@ __global__ __launch_bounds__(kWave) void prefill_attention_kernel(const h16 *__r
 
 // The same causal attention on the matrix cores (no ring wrap inside the chunk: prefill positions
 // never pass the context length). A workgroup owns RB = WV / G blocks of 16 consecutive rows and one
-// KV head; in each of its KS key groups of WV waves, wave w takes query head g G + w / RB on row block
-// w % RB, so the group's waves share every K/V tile of 64 keys, which the group stages in LDS (the
-// next tile's rows are requested into registers while the current one is used). Key group kg takes
-// every KS-th tile. Per tile and wave:
+// group of G query heads of one KV head (8 query heads at head_dim 128 are two groups: 1024 threads spill);
+// in each of its KS key groups of WV waves, wave w takes query head w / RB of the group on row block
+// w % RB, so the key group's waves share every K/V tile of 64 keys, which they stage in LDS (the next
+// tile's rows are requested into registers while the current one is used). Key group kg takes every
+// KS-th tile. Per tile and wave:
 //   scores  S^T[64 keys][16 queries] = K Q^T on v_mfma_f32_16x16x32_f16 (A = K rows from LDS,
 //           B = the wave's 16 query rows, held in registers): lane l holds query l % 16 and keys
 //           16 t + 4 (l / 16) + i of sub-tile t; keys past a row's position are masked (only in the
@@ -1150,8 +1151,7 @@ __global__ __launch_bounds__(kWave) void prefill_attention_kernel(const h16 *__r
 // Bound: the serial phases of a round (scores, softmax, P V between two barriers) with two waves per
 // SIMD. Measured on MI355X, us per layer: 1024 rows at the Llama-3 shape 52 -> 36 (8-wave workgroups
 // of 32 rows without key groups before, in ascending row order); 37 rows after 500 positions 33 -> 14
-// with the merge (one workgroup per row and KV head, scalar P V before); 128 rows at the TinyLlama
-// shape 7.1 -> 7.4 (too few tiles to split). That per-row kernel is gone with the shapes it served.
+// with the merge (one workgroup per row and KV head, scalar P V before).
 typedef short short4_t __attribute__((ext_vector_type(4)));
 typedef float f32x2 __attribute__((ext_vector_type(2)));
 constexpr int kPfBK = 64;            // keys per tile
@@ -1159,7 +1159,7 @@ constexpr float kPfPScale = 15.0f;   // log2 of the probabilities' factor: at mo
 template <int HD, int G, int WV, int KS>
 __global__ __launch_bounds__(KS *WV *kWave) void prefill_attention_mfma_kernel(
     const h16 *__restrict__ Q, const h16 *__restrict__ kc, const h16 *__restrict__ vc, h16 *__restrict__ out,
-    int64_t n, int64_t dim, int64_t kvd, int64_t p0, float scale2, float *__restrict__ part) {
+    int64_t n, int64_t dim, int64_t kvd, int64_t p0, float scale2, unsigned hsub, float *__restrict__ part) {
     constexpr int RB = WV / G;             // 16-row blocks per workgroup
     constexpr int BQ = 16 * RB;            // rows per workgroup
     constexpr int NJ = HD / 32;            // score k-steps
@@ -1183,7 +1183,7 @@ __global__ __launch_bounds__(KS *WV *kWave) void prefill_attention_mfma_kernel(
     uint8_t *kbase = smem + kg * TB, *vs = kbase + KB;
     auto ks = [&](int row, int col) -> h16 * { return reinterpret_cast<h16 *>(kbase) + row * KR + col; };
     const int q4 = lane >> 4, c16 = lane & 15;
-    const int64_t g = blockIdx.x;
+    const int64_t g = blockIdx.x / hsub;
     const int64_t rb0 = (int64_t)(gridDim.y - 1 - blockIdx.y) * BQ;  // first row of the workgroup
     const int64_t rlast = (rb0 + BQ < n ? rb0 + BQ : n) - 1;      // last valid row
     const int64_t kend = p0 + rlast + 1;                          // keys of the workgroup
@@ -1194,7 +1194,7 @@ __global__ __launch_bounds__(KS *WV *kWave) void prefill_attention_mfma_kernel(
     const int hw = wave / RB;
     const int64_t r0w = rb0 + 16 * (wave % RB);                   // first row of the wave
     const int64_t rmax_w = r0w + 15 < rlast ? r0w + 15 : rlast;   // last valid row of the wave
-    const int64_t head = g * G + hw, nq = dim / HD;
+    const int64_t head = (int64_t)blockIdx.x * G + hw, nq = dim / HD;
     // this lane's query row (rows past the chunk are clamped: computed, never stored)
     const int64_t rq = r0w + c16 < rlast ? r0w + c16 : rlast;
     const int kq = (int)(p0 + rq);  // last key the query sees
@@ -1442,8 +1442,8 @@ __global__ __launch_bounds__(kPThreads) void prefill_attention_merge_kernel(cons
     for (int e = 0; e < 4; e++) out[i + e] = (h16)(o[e] / L);
 }
 
-// Shares of the key tiles over grid.z: enough that the workgroups reach about two per CU, each with
-// at least one tile per key group, at most 16.
+// Shares of the key tiles over grid.z: as many workgroups as CUs, each with at least one tile per key group, at
+// most 16.
 static int64_t pf_key_splits(int64_t wgs, int64_t tiles, int64_t key_groups) {
     int64_t z = 256 / wgs;
     if (z > tiles / key_groups) z = tiles / key_groups;
@@ -1458,33 +1458,43 @@ static int32_t launch_prefill_attention_mfma(aesir_ctx *ctx, int64_t hd, int64_t
     hipStream_t s = ctx->stream;
     if (p0 + n >= ((int64_t)1 << 31) - kPfBK) return AESIR_ERR_UNSUPPORTED;
     const float scale2 = (float)((double)scale * 1.4426950408889634);  // log2 e
-#define AESIR_PF_MMA(HDV, GV)                                                                                   \
-    if (hd == HDV && G == GV) {                                                                                \
-        constexpr int WV = GV > 4 ? GV : 4, KS = HDV == 128 && GV == 8 ? 1 : 2; /* (1024 threads spill there) */ \
-        const int64_t nrb = (n + 16 * (WV / GV) - 1) / (16 * (WV / GV)), wgs = nrb * nkv;                      \
+    const int64_t tiles = (p0 + n + kPfBK - 1) / kPfBK;
+    // Up to two tiles run with one key group: its exchange and twice the threads cost more than the second tile
+    // (22 layers at the TinyLlama shape, us per prefill: 1 row 1096 -> 1078, 33 rows 1255 -> 1222, 64 rows 1379 ->
+    // 1347, 128 rows 1454 -> 1430; the kernel with one workgroup per row that served these before 1078, 1229, 1396,
+    // 1448).
+    const bool one = tiles <= 2;
+#define AESIR_PF_MMA(HDV, GTOT, GV)                                                                             \
+    if (hd == HDV && G == GTOT) {                                                                              \
+        constexpr int WV = GV > 4 ? GV : 4, SUB = GTOT / GV;                                                   \
+        const int64_t nrb = (n + 16 * (WV / GV) - 1) / (16 * (WV / GV)), wgs = nrb * nkv * SUB;                \
         if (nrb > 65535) return AESIR_ERR_UNSUPPORTED;                                                         \
-        int64_t Z = pf_key_splits(wgs, (p0 + n + kPfBK - 1) / kPfBK, KS);                                      \
+        int64_t Z = one ? 1 : pf_key_splits(wgs, tiles, 2);                                                    \
         while (Z > 1 && Z * n * dim / HDV * (HDV + 2) > ctx->scratch.attn_part_floats) Z--;                    \
-        hipLaunchKernelGGL((prefill_attention_mfma_kernel<HDV, GV, WV, KS>),                                   \
-                           dim3((unsigned)nkv, (unsigned)nrb, (unsigned)Z), dim3(KS * WV * kWave), 0, s, Q, kc, \
-                           vc, out, n, dim, kvd, p0, scale2, ctx->scratch.attn_part);                          \
+        const dim3 grid((unsigned)(nkv * SUB), (unsigned)nrb, (unsigned)Z);                                    \
+        float *part = ctx->scratch.attn_part;                                                                  \
+        if (one)                                                                                               \
+            hipLaunchKernelGGL((prefill_attention_mfma_kernel<HDV, GV, WV, 1>), grid, dim3(WV * kWave), 0, s, Q, kc, vc, \
+                               out, n, dim, kvd, p0, scale2, (unsigned)SUB, part);                             \
+        else                                                                                                   \
+            hipLaunchKernelGGL((prefill_attention_mfma_kernel<HDV, GV, WV, 2>), grid, dim3(2 * WV * kWave), 0, s, Q, kc, \
+                               vc, out, n, dim, kvd, p0, scale2, (unsigned)SUB, part);                         \
         AESIR_LAUNCH_CHECK("prefill_attention_mfma_kernel");                                                   \
         if (Z > 1) {                                                                                           \
             hipLaunchKernelGGL(prefill_attention_merge_kernel, dim3((unsigned)((n * dim / 4 + kPThreads - 1) / kPThreads)), \
-                               dim3(kPThreads), 0, s, (const float *)ctx->scratch.attn_part, (int)Z, n, dim / HDV, \
-                               (int)HDV, out);                                                                 \
+                               dim3(kPThreads), 0, s, (const float *)part, (int)Z, n, dim / HDV, (int)HDV, out); \
             AESIR_LAUNCH_CHECK("prefill_attention_merge_kernel");                                              \
         }                                                                                                      \
         return AESIR_OK;                                                                                       \
     }
-    AESIR_PF_MMA(64, 8)
-    AESIR_PF_MMA(64, 4)
-    AESIR_PF_MMA(64, 2)
-    AESIR_PF_MMA(64, 1)
-    AESIR_PF_MMA(128, 8)
-    AESIR_PF_MMA(128, 4)
-    AESIR_PF_MMA(128, 2)
-    AESIR_PF_MMA(128, 1)
+    AESIR_PF_MMA(64, 8, 8)
+    AESIR_PF_MMA(64, 4, 4)
+    AESIR_PF_MMA(64, 2, 2)
+    AESIR_PF_MMA(64, 1, 1)
+    AESIR_PF_MMA(128, 8, 4)
+    AESIR_PF_MMA(128, 4, 4)
+    AESIR_PF_MMA(128, 2, 2)
+    AESIR_PF_MMA(128, 1, 1)
 #undef AESIR_PF_MMA
     return AESIR_ERR_UNSUPPORTED;
 }
