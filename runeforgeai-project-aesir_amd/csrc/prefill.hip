@@ -523,6 +523,25 @@ static int64_t gemm_splits(int64_t M, int64_t K, int64_t N) {
     return s < 1 ? 1 : s;
 }
 
+// Whether an f16 product of M rows goes to the short-chunk GEMM instead of the 32-row kernel above. Measured on
+// MI355X, weights past the MALL, us per product and its sum (prefills of 6 to 22 layers, by their slope):
+//   no K split (gate/up): 11264 x 2048 1-2 us less and 28672 x 4096 9.5 less from 160 workgroups of 64 weight
+//     rows on; 8192 x 4096 6.7 more, 4096 x 2048 2.4 more: the 32-row kernel splits K there.
+//   summed by the next kernel (Q/K/V, O, down): up to 32 rows it gains where the 32-row kernel plans more
+//     than the 8 splits that the fused row kernels are compiled for (3072 x 8192 and 3072 x 3072, 4 us; 2048 x
+//     5632, 1.5); elsewhere it takes 1-3 us more (4096 x 14336, 4096 x 4096, 2048 x 2048, 1024 x 1024). Above
+//     32 rows the 32-row kernel goes over the weights twice: 3 us less from about 9 M weights on (3072 x 3072,
+//     4096 x 4096), 1 more at 2048 x 2048.
+//   a call of its own with a launch for the sum, above 32 rows: 32000 x 2048 37 -> 25-30, 14336 x 4096 29 ->
+//     24-28; 8000 x 512 7.8 -> 8.3 and 6144 x 4096 14.1 -> 16.6 from the MALL, so from half a chip of unsplit
+//     workgroups and 1024 wide on.
+static bool f16_skinny_pays(int64_t M, int64_t K, int64_t N, SkinnySplit split) {
+    const int64_t wgs = (N + 63) / 64;
+    if (split == kSplitNone) return wgs >= 160;
+    if (split == kSplitPaid) return M > kGemmMT && wgs >= 128 && K >= 1024;
+    return M > kGemmMT ? N * K >= 9000000 : gemm_splits(M, K, N) > 8;
+}
+
 // The shape half of prefill_mfma_ok: true when a model of this shape runs every prefill GEMM on
 // the matrix cores (its arena buffers and weights are 256-byte aligned, which covers the rest), so
 // the f16 gate/up products of the fallback need no buffer.
@@ -733,7 +752,9 @@ static int32_t prefill_gemm(aesir_model *m, hipStream_t s, const WMat &w, const 
         }
     }
     if (part_out) *part_out = nullptr;
-    if (const SkinnyPlan sp = skinny_plan(M, K, N, w.type, EPI == kEpiSwiglu ? kSplitNone : kSplitFree); sp.nw)
+    const SkinnySplit split = EPI == kEpiSwiglu ? kSplitNone : kSplitFree;
+    if (const SkinnyPlan sp = skinny_plan(M, K, N, w.type, split);
+        sp.nw && (w.type != AESIR_GGML_F16 || f16_skinny_pays(M, K, N, split)))
         return launch_skinny<EPI>(s, skinny_mat(w), A, M, K, N, C, ldc, m->pf_part, m->pf_part_floats, sp, defer, splits_out);
     if (!qf_type(w.type))
         return launch_mfma<EPI>(s, A, M, K, w.w, N, C, ldc, m->pf_part, m->pf_part_floats, name, defer, splits_out,
@@ -797,9 +818,7 @@ int32_t launch_gemm_raw(aesir_ctx *ctx, const void *A, int64_t M, int64_t K, con
 
 int32_t launch_gemm_f16_mfma(aesir_ctx *ctx, const void *A, int64_t M, int64_t K, const void *B, int64_t N, void *C) {
     if (!mfma_shape_ok(A, M, K, B, N)) return launch_gemm_f16(ctx, A, M, K, B, N, C);
-    // up to 32 rows the 32-row kernel with its sum stays (16 x 4096 x 4096 from the MALL 10.7 us against
-    // 11.5; 64 x 4096 x 14336 32.5 against 29.5)
-    if (const SkinnyPlan sp = skinny_plan(M, K, N, AESIR_GGML_F16, kSplitPaid); sp.nw && M > kGemmMT) {
+    if (const SkinnyPlan sp = skinny_plan(M, K, N, AESIR_GGML_F16, kSplitPaid); sp.nw && f16_skinny_pays(M, K, N, kSplitPaid)) {
         SkinnyMat w;
         w.type = AESIR_GGML_F16;
         w.w = B;
