@@ -208,7 +208,8 @@ int32_t aesir_gemm_q8_0(aesir_ctx *ctx, const void *A, int64_t a_rows, int64_t a
  * q) (the reference's K-quant gemms read synthetic block layouts that no GGUF file holds). Raises
  * "gemm_q4_0: matrix dimensions must be positive", "...: inner dimension must be a multiple of
  * 32" (256 for the K-quants), "...: output matrix shape mismatch". Up to 64 rows of A with
- * a_cols a multiple of 128 (A 16-byte, blocks 2-byte aligned) the blocks are multiplied as they lie.
+ * a_cols a multiple of 128 (A 16-byte, blocks 2-byte aligned) the blocks are multiplied as they lie,
+ * but for short or few rows of Q3_K and Q6_K blocks, which take the copy where the well has room for it.
  * Other calls take free well space for their duration: with a_rows > 64 and a_cols a multiple of 128
  * the blocks are repacked into the library's tiled planes (about the size of the blocks) for the
  * matrix-core GEMM that dequantizes in registers; otherwise an f16 copy of the weights (2 bytes per

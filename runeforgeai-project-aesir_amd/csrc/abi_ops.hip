@@ -206,6 +206,18 @@ int32_t aesir_argmax_f16(aesir_ctx *ctx, const void *logits, int64_t n, int64_t 
     return AESIR_OK;
 }
 
+// Whether the short-chunk GEMM on Q8_0 blocks as they lie (64 rows per pass over the blocks, its K splits summed
+// by a launch of their own) beats the GEMV (a pass per row, blocks kept in the caches of few weight rows).
+// Measured on MI355X, us per call, GEMV / GEMM: 2 rows 4096 x 4096 7.6 / 14.2, 500 x 6144 4.8 / 10.7, 14336 x 4096
+// 30.4 / 26.9; 5 rows 4096 x 4096 17.8 / 14.2, 2048 x 2048 6.8 / 8.3; 12 rows 2048 x 2048 11.0 / 9.0, 1024 x 1024
+// 6.7 / 6.8; 64 rows 4096 x 4096 191 / 18.8, 300 x 2048 9.9 / 9.4, 100 x 1024 4.7 / 7.3. More rows than 64 pay per
+// pass: 65 rows 4096 x 4096 195 / 33, 700 x 512 18 / 12.4, 300 x 2048 10.0 / 17.5; 512 rows 14336 x 4096 5469 / 266,
+// 256 x 512 46 / 55. Without K splits (up to 256 wide) one pass is one launch: 2 rows 100 x 256 4.8 / 3.6.
+static bool q8_rows_pay(int64_t M, int64_t K, int64_t N) {
+    const int64_t passes = (M + kSkinnyMaxRows - 1) / kSkinnyMaxRows;
+    return M >= 2 && (M * N >= 24576 * passes || (K <= 256 && passes == 1));
+}
+
 int32_t aesir_gemm_q8_0(aesir_ctx *ctx, const void *A, int64_t a_rows, int64_t a_cols, const void *blocks,
                         int64_t b_rows, void *C, int64_t c_rows, int64_t c_cols) {
     AESIR_TRY(bind(ctx));
@@ -214,10 +226,22 @@ int32_t aesir_gemm_q8_0(aesir_ctx *ctx, const void *A, int64_t a_rows, int64_t a
     if (a_cols % 32 != 0) return fail(AESIR_ERR_SHAPE, "gemm_q8_0: inner dimension must be a multiple of 32");
     if (c_rows != a_rows || c_cols != b_rows) return fail(AESIR_ERR_SHAPE, "gemm_q8_0: output matrix shape mismatch");
     if (!A || !blocks || !C) return fail(AESIR_ERR_INVALID, "gemm_q8_0: null tensor pointer");
-    // more rows than one: the blocks meet up to 64 rows per read (the GEMV reads them once per row)
-    if (a_rows >= 2 && gemm_raw_ok(A, a_cols, blocks, AESIR_GGML_Q8_0, b_rows))
+    if (q8_rows_pay(a_rows, a_cols, b_rows) && gemm_raw_ok(A, a_cols, blocks, AESIR_GGML_Q8_0, b_rows))
         return launch_gemm_raw(ctx, A, a_rows, a_cols, blocks, AESIR_GGML_Q8_0, b_rows, C);
     return launch_gemm_q8_0(ctx->stream, A, a_rows, a_cols, blocks, b_rows, C);
+}
+
+// Whether up to 64 rows of A multiply the other types' blocks as they lie, or an f16 copy of them. Q3_K and Q6_K
+// blocks (110 and 210 bytes) cost the GEMM most: their loads straddle lines and need the longest unpacking, which
+// short rows and few bytes don't cover. Measured on MI355X, us per call, blocks / copy (Q6_K): 64 rows 8000 x 256
+// 14.6 / 9.6, 4000 x 512 15.4 / 12.0, 500 x 2048 11.7 / 11.0, 2048 x 1024 11.3 / 11.8; 1 row 700 x 512 8.6 / 6.4, 8000
+// x 1024 14.3 / 10.6, 500 x 6144 15.3 / 8.8, 2048 x 5632 15.4 / 20.2 (repacked), 700 x 256 6.2 / 6.5. Of the other
+// types the copy is never faster (Q4_0, 1 row: 4000 x 512 6.6 / 9.2, 2048 x 1024 6.8 / 7.5).
+static bool raw_pays(int32_t type, int64_t M, int64_t K, int64_t N) {
+    if (type != AESIR_GGML_Q3_K && type != AESIR_GGML_Q6_K) return true;
+    const int64_t w = N * K;
+    if (K < 1024) return M <= 16 && w <= (1 << 18);
+    return M == 1 ? K >= 2048 && w >= (4 << 20) : w >= (2 << 20);
 }
 
 int32_t aesir_gemm_quant(aesir_ctx *ctx, const void *A, int64_t a_rows, int64_t a_cols, const void *blocks,
@@ -248,8 +272,11 @@ int32_t aesir_gemm_quant(aesir_ctx *ctx, const void *A, int64_t a_rows, int64_t 
         return fail(AESIR_ERR_SHAPE, "%s: inner dimension must be a multiple of %lld", nm, (long long)blk);
     if (c_rows != a_rows || c_cols != b_rows) return fail(AESIR_ERR_SHAPE, "%s: output matrix shape mismatch", nm);
     if (!A || !blocks || !C) return fail(AESIR_ERR_INVALID, "%s: null tensor pointer", nm);
-    // Up to 64 rows of A on whole 128-weight segments: the short-chunk GEMM reads the blocks as they lie.
-    if (a_rows <= kSkinnyMaxRows && gemm_raw_ok(A, a_cols, blocks, ggml_type, b_rows))
+    // Up to 64 rows of A on whole 128-weight segments: the short-chunk GEMM reads the blocks as they lie, where
+    // that pays or the well has no room for the copy.
+    if (a_rows <= kSkinnyMaxRows && gemm_raw_ok(A, a_cols, blocks, ggml_type, b_rows) &&
+        (raw_pays(ggml_type, a_rows, a_cols, b_rows) ||
+         ((ctx->well_offset + 127) & ~int64_t(127)) + b_rows * a_cols > ctx->well_capacity))
         return launch_gemm_raw(ctx, A, a_rows, a_cols, blocks, ggml_type, b_rows, C);
     // More rows on whole 128-weight segments of a repacked type: the blocks are repacked into the
     // tiled planes for the wide-tile matrix-core GEMM, which dequantizes them in registers (it copies A

@@ -28,6 +28,10 @@ SkinnyPlan skinny_plan(int64_t M, int64_t K, int64_t N, int32_t type, SkinnySpli
     // a sum launch costs more than it gains once 4-wave workgroups alone reach most CUs
     const bool may_split = split == kSplitFree || (split == kSplitPaid && (N + 63) / 64 < kSkinnyWgTarget * 5 / 8);
     p.nw = type != AESIR_GGML_F16 && t8 * (may_split ? 8 : 1) >= kSkinnyWgTarget * 3 / 4 ? 8 : 4;
+    // packed Q6_K blocks with 33 rows or more: 4 waves and their splits up to 8192 weight rows (us per call, 8 / 4
+    // waves, 64 rows: 4096 x 4096 23.9 / 19.7, 6144 x 4096 32.9 / 28.8, 3072 x 3072 24.3 / 18.0, 8000 x 6144 38.8 /
+    // 39.7, 32000 x 2048 41.8 / 44.2)
+    if (raw && type == AESIR_GGML_Q6_K && M > 32 && N <= 8192) p.nw = 4;
     if (may_split) {
         const int64_t tiles = (N + 16 * p.nw - 1) / (16 * p.nw), most = K / (2 * kSeg);
         int64_t s = kSkinnyWgTarget / tiles;

@@ -1,5 +1,9 @@
-"""The short-chunk GEMM (1 to 64 activation rows) at the edges of its tiles, on f16 rows and on packed
+"""The per-op products of 1 to 64 activation rows at the edges of their tiles, on f16 rows and on packed
 GGUF blocks of every type, and the repacked route above 64 rows on the same blocks.
+
+f16: the 32-row kernel, and from 33 rows on 8129 weight rows or more the short-chunk GEMM. Blocks: the short-chunk
+GEMM where it pays (every type but Q8_0, Q3_K and Q6_K always; see the cases of the lines between), else Q8_0's
+GEMV per row and an f16 copy for the other two.
 
 Rows on both sides of the 16-row activation tiles, weight rows that end inside a 16-row block, a
 workgroup (64 or 128 rows) or a group of 4, one and an odd number of 128-wide K segments, and K splits.
@@ -88,3 +92,26 @@ def test_packed_blocks(A, ctx, oracle, kind, M, K, N, offset):
     got = c.numpy()
     check(got[:M], a, w)
     assert np.all(got[M] == 7.0)
+
+
+@pytest.mark.parametrize("M,K,N", [(32, 1024, 8130), (33, 1024, 8128), (33, 1024, 8129), (48, 1152, 8200), (64, 2176, 8191),
+                                   (64, 896, 8200)])
+def test_f16_rule(A, ctx, M, K, N):
+    """Both sides of the lines between the 32-row kernel and the short-chunk GEMM."""
+    test_f16_edges(A, ctx, M, K, N)
+
+
+@pytest.mark.parametrize("kind,M,K,N", [
+    # Q8_0: rows times weight rows below and above the line, one launch without K splits, several passes of 64 rows
+    ("q8_0", 12, 768, 2047), ("q8_0", 13, 768, 1900), ("q8_0", 2, 256, 33), ("q8_0", 17, 128, 65), ("q8_0", 33, 256, 130),
+    ("q8_0", 48, 640, 515), ("q8_0", 64, 640, 386), ("q8_0", 65, 256, 100), ("q8_0", 65, 1024, 770), ("q8_0", 130, 512, 700),
+    # Q3_K and Q6_K: the copy for short rows, one row, few bytes; the blocks in 4 and in 8 waves
+    ("q6_k", 16, 768, 341), ("q6_k", 17, 768, 341), ("q6_k", 16, 768, 342), ("q6_k", 1, 1792, 2400), ("q6_k", 1, 2048, 2049),
+    ("q6_k", 2, 1024, 2047), ("q6_k", 2, 1024, 2049), ("q6_k", 33, 1280, 1700), ("q6_k", 32, 1280, 1700), ("q6_k", 64, 2816, 1001),
+    ("q6_k", 40, 1024, 8192), ("q6_k", 40, 1024, 8200),
+    ("q3_k", 16, 768, 341), ("q3_k", 17, 768, 341), ("q3_k", 1, 2048, 2047), ("q3_k", 1, 2048, 2049), ("q3_k", 33, 1280, 1700),
+    ("q3_k", 64, 2816, 1001), ("q4_k", 1, 512, 700), ("q4_0", 1, 512, 700),
+])
+def test_packed_blocks_rule(A, ctx, oracle, kind, M, K, N):
+    """Both sides of the lines between the routes of packed blocks."""
+    test_packed_blocks(A, ctx, oracle, kind, M, K, N, 0)
