@@ -226,6 +226,7 @@ int32_t aesir_gemm_q8_0(aesir_ctx *ctx, const void *A, int64_t a_rows, int64_t a
     if (a_cols % 32 != 0) return fail(AESIR_ERR_SHAPE, "gemm_q8_0: inner dimension must be a multiple of 32");
     if (c_rows != a_rows || c_cols != b_rows) return fail(AESIR_ERR_SHAPE, "gemm_q8_0: output matrix shape mismatch");
     if (!A || !blocks || !C) return fail(AESIR_ERR_INVALID, "gemm_q8_0: null tensor pointer");
+    if (a_rows > 65535) return fail(AESIR_ERR_UNSUPPORTED, "gemm_q8_0: more than 65535 rows of A");
     if (q8_rows_pay(a_rows, a_cols, b_rows) && gemm_raw_ok(A, a_cols, blocks, AESIR_GGML_Q8_0, b_rows))
         return launch_gemm_raw(ctx, A, a_rows, a_cols, blocks, AESIR_GGML_Q8_0, b_rows, C);
     return launch_gemm_q8_0(ctx->stream, A, a_rows, a_cols, blocks, b_rows, C);

@@ -575,7 +575,7 @@ static int32_t q8_dispatch(hipStream_t s, const void *blocks, int64_t M, int64_t
 }
 
 int32_t launch_gemm_q8_0(hipStream_t s, const void *A, int64_t M, int64_t K, const void *blocks, int64_t N, void *C) {
-    if (M > 65535) return fail(AESIR_ERR_UNSUPPORTED, "gemm_q8_0: more than 65535 rows of A");
+    if (M > 65535) return fail(AESIR_ERR_UNSUPPORTED, "gemm_q8_0: more than 65535 rows of A");  // (the grid's y)
     if (((uintptr_t)blocks & 1) != 0) return fail(AESIR_ERR_INVALID, "gemm_q8_0: blocks must be 2-byte aligned");
     return q8_dispatch<false>(s, blocks, M, N, K, A, C);
 }

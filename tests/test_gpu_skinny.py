@@ -115,3 +115,16 @@ def test_f16_rule(A, ctx, M, K, N):
 def test_packed_blocks_rule(A, ctx, oracle, kind, M, K, N):
     """Both sides of the lines between the routes of packed blocks."""
     test_packed_blocks(A, ctx, oracle, kind, M, K, N, 0)
+
+
+def test_q8_0_row_limit(A, ctx):
+    """More than 65535 rows of A are refused whatever the alignment."""
+    a, c = ctx.tensor(65536, 32), ctx.tensor(65536, 1)
+    a256 = ctx.tensor(65536, 256)
+    blocks = ctx.tensor(1, 8 * 17)
+    for x, rows in ((a, 1), (a256, 1)):
+        with pytest.raises(A.AesirError, match="more than 65535 rows"):
+            A.gemm_q8_0(ctx, x, blocks.ptr, rows, c)
+    wide = ctx.tensor(65536, 1024)
+    with pytest.raises(A.AesirError, match="more than 65535 rows"):
+        A.gemm_q8_0(ctx, a256, ctx.tensor(1024, 8 * 17).ptr, 1024, wide)
