@@ -4,16 +4,17 @@
 // flop per weight byte, three times MI355X's ridge), which is where a library tile sized for that
 // regime pays off; the hand-written wide-tile kernel stays for the short chunks, where the weight
 // stream bounds it. The product is plain: D = A W^T with A [M][K] row-major f16 activations, W
-// [N][K] row-major f16 weights, f32 accumulation and one rounding of each output to f16, which is
-// the first rounding of every epilogue. The epilogues of the prefill (SwiGLU, residual add, RMSNorm)
-// stay hand-written row kernels, so the rounding points are the fused kernels' own.
+// [N][K] row-major f16 weights, f32 accumulation and one rounding of each output, to f16 or to
+// f32 for a row kernel that applies the rounding of the epilogue itself. The epilogues of the prefill
+// (SwiGLU, residual add, RMSNorm) stay hand-written row kernels, so the rounding points are the fused
+// kernels' own.
 //
 // In hipBLASLt's column-major terms D^T [N][M] = op(W) A^T with op = transpose on W stored as
 // K x N (leading dimension K), A^T as K x M (leading dimension K) and D^T as N x M (leading
 // dimension N, i.e. row-major [M][N]). The algorithm is the first of the library heuristic's choices
 // for the shape that it also runs (deterministic for a given library and device), cached per context with
 // its descriptors: for some shapes the first choice, one that splits the sum over a workspace, is refused at
-// the call (internal error; e.g. 256 x 4096 x 14336 and 804 x 2048 x 5632, 100 of 3600 products tried).
+// the call (internal error; e.g. 804 x 4096 x 14336 and 804 x 2048 x 5632, 33 of 3600 products tried).
 #include <hipblaslt/hipblaslt.h>
 
 #include <vector>
@@ -26,6 +27,7 @@ namespace {
 
 struct BlasPlan {
     int64_t M = 0, N = 0, K = 0;
+    bool f32_out = false;
     hipblasLtMatmulDesc_t desc = nullptr;
     hipblasLtMatrixLayout_t la = nullptr, lb = nullptr, ld = nullptr;
     std::vector<hipblasLtMatmulHeuristicResult_t> algos;  // not refused yet, in the heuristic's order
@@ -50,13 +52,14 @@ void destroy_plan(BlasPlan &p) {
 // Builds the descriptors and lists the algorithms for one shape; p.algos stays empty when the library
 // offers none within the workspace.
 void make_plan(hipblasLtHandle_t h, BlasPlan &p, size_t ws_bytes) {
+    const hipDataType dt = p.f32_out ? HIP_R_32F : HIP_R_16F;
     const hipblasOperation_t ta = HIPBLAS_OP_T, tb = HIPBLAS_OP_N;
     if (hipblasLtMatmulDescCreate(&p.desc, HIPBLAS_COMPUTE_32F, HIP_R_32F) != HIPBLAS_STATUS_SUCCESS ||
         hipblasLtMatmulDescSetAttribute(p.desc, HIPBLASLT_MATMUL_DESC_TRANSA, &ta, sizeof(ta)) != HIPBLAS_STATUS_SUCCESS ||
         hipblasLtMatmulDescSetAttribute(p.desc, HIPBLASLT_MATMUL_DESC_TRANSB, &tb, sizeof(tb)) != HIPBLAS_STATUS_SUCCESS ||
         hipblasLtMatrixLayoutCreate(&p.la, HIP_R_16F, p.K, p.N, p.K) != HIPBLAS_STATUS_SUCCESS ||
         hipblasLtMatrixLayoutCreate(&p.lb, HIP_R_16F, p.K, p.M, p.K) != HIPBLAS_STATUS_SUCCESS ||
-        hipblasLtMatrixLayoutCreate(&p.ld, HIP_R_16F, p.N, p.M, p.N) != HIPBLAS_STATUS_SUCCESS)
+        hipblasLtMatrixLayoutCreate(&p.ld, dt, p.N, p.M, p.N) != HIPBLAS_STATUS_SUCCESS)
         return;
     hipblasLtMatmulPreference_t pref = nullptr;
     if (hipblasLtMatmulPreferenceCreate(&pref) != HIPBLAS_STATUS_SUCCESS) return;
@@ -75,7 +78,7 @@ void make_plan(hipblasLtHandle_t h, BlasPlan &p, size_t ws_bytes) {
 }  // namespace
 
 int32_t blas_gemm_nt(aesir_ctx *ctx, hipStream_t s, const void *A, int64_t M, int64_t K, const void *W, int64_t N,
-                     void *D, void *ws, int64_t ws_bytes) {
+                     void *D, bool f32_out, void *ws, int64_t ws_bytes) {
     if (M <= 0 || N <= 0 || K <= 0) return fail(AESIR_ERR_INVALID, "blas_gemm_nt: empty shape");
     if (!ctx->blas) {
         auto *st = new BlasState;
@@ -88,7 +91,7 @@ int32_t blas_gemm_nt(aesir_ctx *ctx, hipStream_t s, const void *A, int64_t M, in
     auto *st = static_cast<BlasState *>(ctx->blas);
     BlasPlan *plan = nullptr;
     for (BlasPlan &p : st->plans)
-        if (p.M == M && p.N == N && p.K == K) plan = &p;
+        if (p.M == M && p.N == N && p.K == K && p.f32_out == f32_out) plan = &p;
     if (!plan) {
         // every distinct chunk length brings its shapes: keep the most recent kMaxPlans
         if (st->plans.size() >= kMaxPlans) {
@@ -96,7 +99,7 @@ int32_t blas_gemm_nt(aesir_ctx *ctx, hipStream_t s, const void *A, int64_t M, in
             st->plans.erase(st->plans.begin());
         }
         BlasPlan p;
-        p.M = M, p.N = N, p.K = K;
+        p.M = M, p.N = N, p.K = K, p.f32_out = f32_out;
         make_plan(st->handle, p, (size_t)ws_bytes);
         st->plans.push_back(p);
         plan = &st->plans.back();

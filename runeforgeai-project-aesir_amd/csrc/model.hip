@@ -637,7 +637,7 @@ int32_t model_create(aesir_ctx *ctx, const aesir_model_config *cfg, const Weight
     take(pr * d * 2, &m->pf_att);
     take(pr * f * 2, &m->pf_act);
     // chunks of many rows run their GEMMs on hipBLASLt (quantized matrices through the f16 copy in
-    // pf_wdeq), whose gate/up and residual products (f16) pass through pf_gu
+    // pf_wdeq), whose gate/up (f16) and residual (f32) products pass through pf_gu
     const bool blas = pr >= prefill_blas_min_rows();
     if (!prefill_gemm_shapes_ok(pr, d, d + 2 * kvd, f) || blas)
         take(pr * 2 * f * 2 > pr * d * 4 ? pr * 2 * f * 2 : pr * d * 4, &m->pf_gu);

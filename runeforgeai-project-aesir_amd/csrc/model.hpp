@@ -108,7 +108,7 @@ struct aesir_model {
     float *attn_part = nullptr;
     int64_t attn_max_split = 1;
     // batched prefill workspace: pf_rows rows of x, normed x, q|k|v, q, attention out, act,
-    // gate/up products (non-MFMA shapes, and the library GEMMs' f16 gate/up or residual
+    // gate/up products (non-MFMA shapes, and the library GEMMs' f16 gate/up or f32 residual
     // products) and the rows' token IDs; the library GEMMs' workspace
     int64_t pf_rows = 0;
     void *pf_x = nullptr, *pf_xn = nullptr, *pf_qkv = nullptr, *pf_q = nullptr, *pf_att = nullptr, *pf_act = nullptr;

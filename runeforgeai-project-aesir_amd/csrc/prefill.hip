@@ -669,32 +669,33 @@ static int32_t launch_q8_dequant_rows(hipStream_t s, const void *q, const void *
 constexpr int64_t kBlasMinRows = 256;
 constexpr int64_t kBlasWorkspace = 32 << 20;
 
-// The library path of prefill_gemm: the plain product in f16, each sum rounded once as every epilogue
-// rounds it first (store; gate/up pairs, then the SwiGLU row kernel; residual: one partial for the
-// caller's fused residual + norm row kernel, or the residual add when not deferred). An f32 partial
-// carries nothing that the first rounding keeps and costs the row kernel twice the bytes (1024 rows at
-// the Llama-3 shape: 8.2 us per launch with f32, 6.9 with f16; the product itself 92 us either way).
+// The library path of prefill_gemm: the plain product in f16 (store; gate/up pairs, then the SwiGLU
+// row kernel) or in f32 (residual: one partial for the caller's fused residual + norm row kernel,
+// or gemm_reduce_kernel when not deferred), so every rounding is the epilogue's own.
 // AESIR_ERR_UNSUPPORTED when the library has no algorithm (the caller takes its own kernel).
 template <int EPI>
 static int32_t prefill_gemm_blas(aesir_model *m, hipStream_t s, const void *W, const void *A, int64_t M, int64_t K,
-                                 int64_t N, void *C, int64_t ldc, bool defer, int64_t *splits_out, const void **part_out) {
+                                 int64_t N, void *C, int64_t ldc, bool defer, int64_t *splits_out, const float **part_out) {
     aesir_ctx *ctx = m->ctx;
     if (EPI == kEpiStore) {
         if (ldc != N) return AESIR_ERR_UNSUPPORTED;
-        AESIR_TRY(blas_gemm_nt(ctx, s, A, M, K, W, N, C, m->pf_blas_ws, kBlasWorkspace));
+        AESIR_TRY(blas_gemm_nt(ctx, s, A, M, K, W, N, C, false, m->pf_blas_ws, kBlasWorkspace));
     } else if (EPI == kEpiSwiglu) {
         if (ldc != N / 2) return AESIR_ERR_UNSUPPORTED;
-        AESIR_TRY(blas_gemm_nt(ctx, s, A, M, K, W, N, m->pf_gu, m->pf_blas_ws, kBlasWorkspace));
+        AESIR_TRY(blas_gemm_nt(ctx, s, A, M, K, W, N, m->pf_gu, false, m->pf_blas_ws, kBlasWorkspace));
         AESIR_TRY(launch_swiglu_pairs(s, m->pf_gu, C, M * (N / 2)));
     } else {
-        if (ldc != N) return AESIR_ERR_UNSUPPORTED;
-        AESIR_TRY(blas_gemm_nt(ctx, s, A, M, K, W, N, m->pf_gu, m->pf_blas_ws, kBlasWorkspace));
+        const float *part = (const float *)m->pf_gu;
+        AESIR_TRY(blas_gemm_nt(ctx, s, A, M, K, W, N, m->pf_gu, true, m->pf_blas_ws, kBlasWorkspace));
         if (defer) {
             if (splits_out) *splits_out = 1;
-            if (part_out) *part_out = m->pf_gu;
+            if (part_out) *part_out = part;
             return AESIR_OK;
         }
-        AESIR_TRY(launch_residual_add(s, C, m->pf_gu, M * N));
+        const int64_t blocks = (M * N + 255) / 256;
+        hipLaunchKernelGGL(gemm_reduce_kernel<EPI>, dim3((unsigned)blocks), dim3(256), 0, s, part, (int64_t)1, M, N,
+                           (h16 *)C, ldc);
+        AESIR_LAUNCH_CHECK("gemm_reduce_kernel");
     }
     if (splits_out) *splits_out = 1;
     if (part_out) *part_out = nullptr;
@@ -735,7 +736,7 @@ static int32_t launch_skinny(hipStream_t s, const SkinnyMat &w, const void *A, i
 template <int EPI>
 static int32_t prefill_gemm(aesir_model *m, hipStream_t s, const WMat &w, const void *A, int64_t M, int64_t K, int64_t N,
                             void *C, int64_t ldc, const char *name, bool defer = false, int64_t *splits_out = nullptr,
-                            const void **part_out = nullptr) {
+                            const float **part_out = nullptr) {
     if (M >= kBlasMinRows && m->pf_blas_ws) {
         const void *W = nullptr;
         if (w.type == AESIR_GGML_F16) {
@@ -945,14 +946,12 @@ constexpr int kRowPasses = 2;  // rows up to 2 x 2048 columns keep their values 
 // SPL > 0: the launch has exactly SPL splits, and every split's partials are requested before the
 // first sum (one memory round trip instead of SPL); SPL = 0: any count, summed as loaded. Both
 // add the splits in split order.
-// H16: one partial, already rounded to f16 (the library's product).
-template <int SPL, bool H16 = false>
-__global__ __launch_bounds__(kPThreads) void reduce_residual_norm_rows_kernel(const void *__restrict__ Pv,
+template <int SPL>
+__global__ __launch_bounds__(kPThreads) void reduce_residual_norm_rows_kernel(const float *__restrict__ P,
                                                                               int64_t splits_rt, int64_t M, int64_t N,
                                                                               h16 *__restrict__ X, h16 *__restrict__ Xn,
                                                                               const h16 *__restrict__ w, float eps) {
     __shared__ float red[kPThreads / kWave];
-    const float *P = reinterpret_cast<const float *>(Pv);
     const int64_t splits = SPL > 0 ? SPL : splits_rt;
     const int64_t m = blockIdx.x;
     h16 *x = X + m * N;
@@ -966,15 +965,7 @@ __global__ __launch_bounds__(kPThreads) void reduce_residual_norm_rows_kernel(co
         float v[kRowVec];
 #pragma unroll
         for (int e = 0; e < kRowVec; e++) v[e] = 0.0f;
-        if constexpr (H16) {
-            const u32x4 p = ld16(reinterpret_cast<const h16 *>(Pv) + m * N + c0);
-#pragma unroll
-            for (int e = 0; e < kRowVec; e += 2) {
-                const h16x2 h = as_h2(p[e / 2]);
-                v[e] = (float)h.x;
-                v[e + 1] = (float)h.y;
-            }
-        } else if (SPL > 0) {
+        if (SPL > 0) {
             f32x4 a[SPL > 0 ? SPL : 1], b[SPL > 0 ? SPL : 1];
 #pragma unroll
             for (int z = 0; z < SPL; z++) {
@@ -1594,22 +1585,16 @@ static int32_t prefill_chunk(aesir_model *m, const int64_t *tokens_host, int64_t
     // residual GEMM into X, then X -> Xn normalized with `next_norm` (if any), fused when split
     auto residual_gemm = [&](const h16 *in, int64_t K, const WMat &w, const void *next_norm, const char *name) -> int32_t {
         int64_t splits = 1;
-        const void *part = nullptr;
+        const float *part = nullptr;
         AESIR_TRY(prefill_gemm<kEpiResidual>(m, s, w, in, n, K, d, X, d, name, next_norm && rowvec, &splits, &part));
         if (!next_norm) return AESIR_OK;
         if ((splits > 1 || part) && rowvec) {  // partials left for the fused residual + norm rows
-            const bool half = part != nullptr;  // the library's product, in f16
             if (!part) part = m->pf_part;
 #define AESIR_RRN(SV)                                                                                           \
     hipLaunchKernelGGL(reduce_residual_norm_rows_kernel<SV>, dim3((unsigned)n), dim3(kPThreads), 0, s,            \
                        part, splits, n, d, X, Xn, (const h16 *)next_norm, c.rms_eps)
             switch (splits) {
-                case 1:
-                    if (half)
-                        hipLaunchKernelGGL((reduce_residual_norm_rows_kernel<1, true>), dim3((unsigned)n), dim3(kPThreads), 0, s,
-                                           part, splits, n, d, X, Xn, (const h16 *)next_norm, c.rms_eps);
-                    else AESIR_RRN(1);
-                    break;
+                case 1: AESIR_RRN(1); break;
                 case 2: AESIR_RRN(2); break;
                 case 3: AESIR_RRN(3); break;
                 case 4: AESIR_RRN(4); break;
