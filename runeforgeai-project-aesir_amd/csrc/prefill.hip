@@ -562,7 +562,11 @@ int64_t prefill_part_floats(int64_t rows, int64_t dim, int64_t qkv_n, int64_t ff
             if (kn[0] % 64 != 0) continue;
             for (bool q8 : {false, true}) {
                 const WidePlan wp = wide_plan(m, kn[0], kn[1], q8);
-                const int64_t sp = wp.nt ? wp.splits : gemm_splits(m, kn[0], kn[1]);
+                int64_t sp = wp.nt ? wp.splits : gemm_splits(m, kn[0], kn[1]);
+                if (kn[1] != 2 * ffn) {  // (gate/up doesn't split there)
+                    const SkinnyPlan p = skinny_plan(m, kn[0], kn[1], q8 ? AESIR_GGML_Q8_0 : AESIR_GGML_F16, kSplitFree);
+                    if (p.nw && p.splits > sp) sp = p.splits;
+                }
                 if (sp > 1 && sp * m * kn[1] > most) most = sp * m * kn[1];
             }
         }

@@ -59,10 +59,12 @@ __device__ __forceinline__ constexpr int sk_granule(int g, int j) {
 // kernel, O 10.0 against 19. 37 rows after 500 positions on the Llama-3-8B shape in Q4_K_M: 11.9 ->
 // 3.8 ms. Not faster: three steps of weights in flight, two K groups of waves per workgroup, two row
 // blocks per wave (34 us: too few workgroups).
-template <int T, int MT, int NB, int NW, int SG, int D>
+constexpr int kSkSegs = 2;  // segments per step
+template <int T, int MT, int NW>
 __global__ __launch_bounds__(NW *kWave) void gemm_skinny_kernel(const h16 *__restrict__ A, int M, int K, SkinnyMat w,
                                                               int N, int epi, h16 *__restrict__ C, int64_t ldc,
                                                               float *__restrict__ P, int64_t ldp) {
+    constexpr int NB = 1, SG = kSkSegs, D = 2;     // row blocks per wave, segments per step, steps in flight
     constexpr int NT = NW * kWave;
     constexpr int STAGE = SG * MT * 4096;
     constexpr int RECS = SG * MT * 128;            // 16-element activation records of a step

@@ -11,10 +11,10 @@ namespace aesir {
 template <int T, int MT, int NW>
 int32_t launch_t(hipStream_t s, int epi, const SkinnyMat &w, const void *A, int64_t M, int64_t K, int64_t N, void *C,
                         int64_t ldc, float *part, int64_t ldp, int64_t splits) {
-    constexpr int SG = 2, lds = 2 * SG * MT * 4096;
+    constexpr int lds = 2 * kSkSegs * MT * 4096;
     static_assert(lds <= 64 * 1024, "within the default LDS limit");
     const dim3 grid((unsigned)((N + 16 * NW - 1) / (16 * NW)), (unsigned)splits);
-    hipLaunchKernelGGL((gemm_skinny_kernel<T, MT, 1, NW, SG, 2>), grid, dim3(NW * kWave), lds, s, (const h16 *)A, (int)M,
+    hipLaunchKernelGGL((gemm_skinny_kernel<T, MT, NW>), grid, dim3(NW * kWave), lds, s, (const h16 *)A, (int)M,
                        (int)K, w, (int)N, epi, (h16 *)C, ldc, part, ldp);
     AESIR_LAUNCH_CHECK("gemm_skinny_kernel");
     return AESIR_OK;
@@ -24,8 +24,9 @@ template <int T>
 int32_t launch_m(hipStream_t s, int epi, const SkinnyMat &w, const void *A, int64_t M, int64_t K, int64_t N, void *C,
                         int64_t ldc, float *part, int64_t ldp, const SkinnyPlan &p) {
 #define AESIR_SK(MTV)                                                                                       \
-    return p.nw == 8 ? launch_t<T, MTV, 8>(s, epi, w, A, M, K, N, C, ldc, part, ldp, p.splits)              \
-                     : launch_t<T, MTV, 4>(s, epi, w, A, M, K, N, C, ldc, part, ldp, p.splits)
+    if constexpr (T != AESIR_GGML_F16) /* (skinny_plan gives f16 4 waves) */                                \
+        if (p.nw == 8) return launch_t<T, MTV, 8>(s, epi, w, A, M, K, N, C, ldc, part, ldp, p.splits);      \
+    return launch_t<T, MTV, 4>(s, epi, w, A, M, K, N, C, ldc, part, ldp, p.splits)
     switch ((M + 15) / 16) {
         case 1: AESIR_SK(1);
         case 2: AESIR_SK(2);
