@@ -6,8 +6,8 @@ loading), against the CPU oracle.
   oracle's reference-order gemm_q4_0 / _q4_1 / _q5_0 / _q5_1 (core/compute.mojo:876-1036; beyond
   1 ulp only where f32 summation noise exceeds it); the K-quants against f64 on the oracle's
   f16 weights (the rule every kernel of the library applies) within one f16 rounding of the
-  output plus f32 summation noise. 16 or more rows of A, and rows whose length is not a multiple
-  of 128, take the F16 GEMM on the same f16 weights and are held to f64 on those.
+  output plus f32 summation noise. Rows whose length is not a multiple of 128, and short rows of
+  Q3_K and Q6_K, take the F16 GEMM on the same f16 weights and are held to f64 on those.
 - Models: the F16 oracle holding the weights the model reads back (get_tensor), which are the
   f16 weights the GEMVs and the prefill multiply for every type; Q4_0 tokens are identical, the
   others may differ only at a near tie of the oracle's logits, and logits are held to the
@@ -64,9 +64,10 @@ def lib_weights(oracle, kind, t):
                                    (20, 4096, 48), (1, 512, 16400), (2, 1536, 18000), (128, 2048, 96),
                                    (100, 4096, 200), (128, 1024, 5000)])
 def test_gemm_quant_vs_oracle(A, ctx, oracle, kind, M, K, N):
-    """M < 16: the decode GEMV per row on the repacked planes; M > 64: the wide-tile matrix-core
-    GEMM on the same planes (K splits with a reduce, M and N tails, 64- and 32-column tiles);
-    otherwise the F16 GEMM on dequantized weights."""
+    """M <= 64: the short-chunk GEMM on the blocks as they lie (Q3_K and Q6_K with few bytes or short
+    rows: the F16 GEMM on dequantized weights); M > 64: the wide-tile matrix-core GEMM on the
+    repacked planes (K splits with a reduce, M and N tails, 64- and 32-column tiles). The decode
+    GEMV of the planes runs in the models (test_gpu_quant_rows.py has its row lengths)."""
     t = random_tensor(A, kind, N, K, RNG)
     x = RNG.standard_normal((M, K)).astype(np.float16)
     c = ctx.tensor(M, N)
@@ -90,8 +91,8 @@ def test_gemm_quant_vs_oracle(A, ctx, oracle, kind, M, K, N):
 @pytest.mark.parametrize("kind", ("q4_0",) + LEGACY_KINDS)
 @pytest.mark.parametrize("M,K,N", [(1, 160, 24), (3, 96, 40), (1, 28704, 17)])
 def test_gemm_q4_0_rows_off_the_tile_grid(A, ctx, oracle, kind, M, K, N):
-    """Rows of the 32-weight block types whose length is not a multiple of 128 (or above the GEMV's
-    28672) take the f16 dequantization + F16 GEMM route: within 1 f16 ulp of the oracle's
+    """Rows of the 32-weight block types whose length is not a multiple of 128 take the f16
+    dequantization + F16 GEMM route: within 1 f16 ulp of the oracle's
     reference-order gemm_q4_0 / _q4_1 / _q5_0 / _q5_1 where f32 summation noise does not exceed it."""
     t = random_tensor(A, kind, N, K, RNG)
     x = RNG.standard_normal((M, K)).astype(np.float16)
@@ -108,9 +109,9 @@ def test_gemm_q4_0_rows_off_the_tile_grid(A, ctx, oracle, kind, M, K, N):
 @pytest.mark.parametrize("kind", ("q4_0", "q4_k", "q6_k"))
 @pytest.mark.parametrize("M", (1, 100))
 def test_gemm_quant_unaligned_a(A, ctx, oracle, kind, M):
-    """A as an offset view (2-byte aligned, not 16-byte): the repacked-plane routes need 16-byte
-    loads of A, so the call takes the dequantize-then-F16 route at 1 row (the GEMV's) and at 100
-    rows (the wide kernel's) and still matches f64 on the library's f16 weights."""
+    """A as an offset view (2-byte aligned, not 16-byte): the short-chunk GEMM and the wide kernel
+    need 16-byte loads of A, so the call takes the dequantize-then-F16 route at 1 row and at 100
+    rows and still matches f64 on the library's f16 weights."""
     K, N = 4096, 96
     t = random_tensor(A, kind, N, K, RNG)
     x = RNG.standard_normal((M, K)).astype(np.float16)
