@@ -31,6 +31,7 @@ struct BlasPlan {
     hipblasLtMatmulDesc_t desc = nullptr;
     hipblasLtMatrixLayout_t la = nullptr, lb = nullptr, ld = nullptr;
     std::vector<hipblasLtMatmulHeuristicResult_t> algos;  // not refused yet, in the heuristic's order
+    int asked = 0;  // how many the heuristic was asked for
 };
 
 constexpr size_t kMaxPlans = 256;
@@ -49,8 +50,25 @@ void destroy_plan(BlasPlan &p) {
     p = BlasPlan{};
 }
 
-// Builds the descriptors and lists the algorithms for one shape; p.algos stays empty when the library
-// offers none within the workspace.
+// Asks the heuristic for `count` algorithms; p.algos stays empty when the library offers none within the
+// workspace.
+void list_algos(hipblasLtHandle_t h, BlasPlan &p, size_t ws_bytes, int count) {
+    p.asked = count;
+    hipblasLtMatmulPreference_t pref = nullptr;
+    if (!p.ld || hipblasLtMatmulPreferenceCreate(&pref) != HIPBLAS_STATUS_SUCCESS) return;
+    const uint64_t wsl = ws_bytes;
+    hipblasLtMatmulHeuristicResult_t res[kMaxAlgos];
+    int n = 0;
+    const bool got = hipblasLtMatmulPreferenceSetAttribute(pref, HIPBLASLT_MATMUL_PREF_MAX_WORKSPACE_BYTES, &wsl,
+                                                           sizeof(wsl)) == HIPBLAS_STATUS_SUCCESS &&
+                     hipblasLtMatmulAlgoGetHeuristic(h, p.desc, p.la, p.lb, p.ld, p.ld, pref, count, res, &n) ==
+                         HIPBLAS_STATUS_SUCCESS;
+    (void)hipblasLtMatmulPreferenceDestroy(pref);
+    for (int i = 0; got && i < n; i++)
+        if (res[i].state == HIPBLAS_STATUS_SUCCESS && res[i].workspaceSize <= ws_bytes) p.algos.push_back(res[i]);
+}
+
+// Builds the descriptors and takes the heuristic's first choice.
 void make_plan(hipblasLtHandle_t h, BlasPlan &p, size_t ws_bytes) {
     const hipDataType dt = p.f32_out ? HIP_R_32F : HIP_R_16F;
     const hipblasOperation_t ta = HIPBLAS_OP_T, tb = HIPBLAS_OP_N;
@@ -61,18 +79,7 @@ void make_plan(hipblasLtHandle_t h, BlasPlan &p, size_t ws_bytes) {
         hipblasLtMatrixLayoutCreate(&p.lb, HIP_R_16F, p.K, p.M, p.K) != HIPBLAS_STATUS_SUCCESS ||
         hipblasLtMatrixLayoutCreate(&p.ld, dt, p.N, p.M, p.N) != HIPBLAS_STATUS_SUCCESS)
         return;
-    hipblasLtMatmulPreference_t pref = nullptr;
-    if (hipblasLtMatmulPreferenceCreate(&pref) != HIPBLAS_STATUS_SUCCESS) return;
-    const uint64_t wsl = ws_bytes;
-    hipblasLtMatmulHeuristicResult_t res[kMaxAlgos];
-    int n = 0;
-    const bool got = hipblasLtMatmulPreferenceSetAttribute(pref, HIPBLASLT_MATMUL_PREF_MAX_WORKSPACE_BYTES, &wsl,
-                                                           sizeof(wsl)) == HIPBLAS_STATUS_SUCCESS &&
-                     hipblasLtMatmulAlgoGetHeuristic(h, p.desc, p.la, p.lb, p.ld, p.ld, pref, kMaxAlgos, res, &n) ==
-                         HIPBLAS_STATUS_SUCCESS;
-    (void)hipblasLtMatmulPreferenceDestroy(pref);
-    for (int i = 0; got && i < n; i++)
-        if (res[i].state == HIPBLAS_STATUS_SUCCESS && res[i].workspaceSize <= ws_bytes) p.algos.push_back(res[i]);
+    list_algos(h, p, ws_bytes, 1);
 }
 
 }  // namespace
@@ -105,7 +112,10 @@ int32_t blas_gemm_nt(aesir_ctx *ctx, hipStream_t s, const void *A, int64_t M, in
         plan = &st->plans.back();
     }
     const float alpha = 1.0f, beta = 0.0f;
-    while (!plan->algos.empty()) {
+    for (;;) {
+        // (asking for one is cheap; the longer list, whose first entries may be refused again, only if need be)
+        if (plan->algos.empty() && plan->asked < kMaxAlgos) list_algos(st->handle, *plan, (size_t)ws_bytes, kMaxAlgos);
+        if (plan->algos.empty()) break;
         const hipblasLtMatmulHeuristicResult_t &r = plan->algos.front();
         if (hipblasLtMatmul(st->handle, plan->desc, &alpha, W, plan->la, A, plan->lb, &beta, D, plan->ld, D, plan->ld, &r.algo,
                             r.workspaceSize ? ws : nullptr, r.workspaceSize, s) == HIPBLAS_STATUS_SUCCESS)
