@@ -124,9 +124,9 @@ int32_t launch_qf_fill_random(hipStream_t s, const QFMat &w, int64_t rows, int64
                               uint64_t stream, float std);
 // GGUF blocks (rows x K, packed, device memory; Q8_0, Q4_0, Q4_1, Q5_0, Q5_1, Q2_K, Q3_K, Q4_K,
 // Q5_K or Q6_K) -> f16 rows of out_stride weights, straight from the blocks, the same f16 values
-// as launch_qf_dequant and the Q8_0 GEMV (the per-op GEMMs of 16 or more rows, row lengths the
-// GEMV does not take, the types without repacked planes, and the quantized parts of a model
-// matrix stored in f16).
+// as launch_qf_dequant and the Q8_0 GEMV (per-op products of row lengths and alignments that the
+// short-chunk and wide-tile GEMMs do not take, short rows of Q3_K and Q6_K, and the quantized parts
+// of a model matrix stored in f16).
 int32_t launch_gguf_dequant(hipStream_t s, int32_t type, const void *blocks, int64_t rows, int64_t K, void *out,
                             int64_t out_stride);
 // Weights per block of a GGML block type launch_gguf_dequant takes (32 or 256), else 0.

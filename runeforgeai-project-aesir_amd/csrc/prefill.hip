@@ -16,7 +16,8 @@
 //   partials are summed in a fixed order by the epilogue kernel (deterministic, no atomics).
 //   Chunks of up to 64 positions run on the short-chunk GEMM (skinny.hip) and longer ones on the
 //   wide-tile kernel below (the whole chunk in one 128-row M tile, 8 waves, 128-wide K chunks);
-//   this 32-row kernel serves the widths that are a multiple of 64 but not of 128.
+//   this 32-row kernel serves f16 matrices that the short-chunk GEMM gains nothing on
+//   (f16_skinny_pays) and the widths that are a multiple of 64 but not of 128.
 //   At M = 128 the GEMM is HBM-bound (128 flop/byte against MI355X's 312 flop/byte ridge).
 #include <cmath>
 #include <vector>
