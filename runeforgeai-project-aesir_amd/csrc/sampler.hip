@@ -94,9 +94,12 @@ __global__ void sampler_mark_kernel(const int64_t *__restrict__ ctx, int64_t n_c
 //      top_k below them, and those that share them (logits are f16, so distinct ones differ in these
 //      bits even after a temperature scale: in practice only ties share them)
 //   3. one workgroup sorts what was gathered as 64-bit values in LDS and keeps the first top_k;
-//      the pairs are distinct, so any correct sort gives the stable sort's order. Where more
-//      share the 22 bits than LDS holds (large ties), it finds the last digit and the lowest-index
-//      ties itself by scanning the keys (about 60 us more at 128256 logits that are all equal)
+//      the pairs are distinct, so any correct sort gives the stable sort's order. Where both kinds
+//      together are more than LDS holds (top_k near kSeqTile), those sharing the bits are sorted and
+//      cut first (128256 logits, top-k 4096 with top-p, us per call: 144, and 266 by scanning the keys);
+//      where they alone are more
+//      (large ties), it finds the last digit and the lowest-index ties itself by scanning the keys
+//      (about 60 us more at 128256 logits that are all equal)
 //   4. the same workgroup makes the truncations and the draw (sampler_select_draw_kernel)
 // Three launches where three digit passes, a count, an ordered compaction, a sort and a tail took seven.
 // Measured on MI355X, 128256 logits, 256 context tokens, top-k 40 with top-p, us per blocking call:
@@ -253,8 +256,8 @@ __global__ __launch_bounds__(kSThreads) void sampler_select_hist_kernel(const ui
         if (lh[b]) atomicAdd(&hist[kSelBins + b], lh[b]);
 }
 
-// Every (key, index) with top bits below the k-th key's, in cand[0, below), and those sharing them behind
-// (as many as fit kSeqTile); ctr: how many of each were met, `below` and the shared bits.
+// Every (key, index) with top bits below the k-th key's, in cand[0, below), and those sharing them from
+// cand[kSeqTile] on (as many as fit kSeqTile); ctr: how many of each were met, `below` and the shared bits.
 __global__ __launch_bounds__(kSThreads) void sampler_select_gather_kernel(const uint32_t *__restrict__ keys, int64_t V,
                                                                           const uint32_t *__restrict__ hist, uint32_t k,
                                                                           uint32_t *__restrict__ ctr,
@@ -285,10 +288,10 @@ __global__ __launch_bounds__(kSThreads) void sampler_select_gather_kernel(const 
         if (lane == 1 && same) at = atomicAdd(&ctr[1], (uint32_t)__popcll(same));
         const uint32_t a = __shfl(at, 0), b = __shfl(at, 1);
         const uint64_t before = (1ull << lane) - 1ull;
-        uint32_t slot = kSeqTile;
-        if (in && t < top) slot = a + (uint32_t)__popcll(below & before);
-        if (in && t == top) slot = st.lt + b + (uint32_t)__popcll(same & before);
-        if (slot < kSeqTile) cand[slot] = ((uint64_t)kv[j] << 32) | (uint64_t)i;
+        uint32_t slot = 2 * kSeqTile;
+        if (in && t < top) slot = a + (uint32_t)__popcll(below & before);  // (fewer than k of them)
+        if (in && t == top) slot = kSeqTile + b + (uint32_t)__popcll(same & before);
+        if (slot < 2 * kSeqTile) cand[slot] = ((uint64_t)kv[j] << 32) | (uint64_t)i;
     }
 }
 
@@ -451,13 +454,42 @@ __global__ __launch_bounds__(kSelSortThreads) void sampler_select_draw_kernel(co
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const uint32_t *ctr = hist + 2 * kSelBins;
     const int lt = (int)ctr[2];
-    int total = lt + (int)(ctr[1] < (uint32_t)(kSeqTile + 1) ? ctr[1] : kSeqTile + 1);
+    const int same = (int)(ctr[1] < (uint32_t)(kSeqTile + 1) ? ctr[1] : kSeqTile + 1);
+    int total = lt + same;
     const uint32_t top = ctr[3];
     for (int i = tid; i < kSelBins; i += kSelSortThreads) hist[i] = 0;
-    const bool all = total <= kSeqTile;
-    for (int i = tid; i < (all ? total : lt); i += kSelSortThreads) v[i] = cand[i];
-    if (!all) {  // the k - lt first (key, index) among those sharing the bits, found by scanning the keys
+    auto bitonic = [&](int count) {  // v[0, count) ascending (entered and left with v complete)
+        int m = 1;
+        while (m < count) m <<= 1;
+        for (int i = count + tid; i < m; i += kSelSortThreads) v[i] = ~0ull;
+        __syncthreads();
+        for (int size = 2; size <= m; size <<= 1) {
+            for (int stride = size >> 1; stride > 0; stride >>= 1) {
+                for (int i = tid; i < m; i += kSelSortThreads) {
+                    const int j = i ^ stride;
+                    if (j > i) {
+                        const bool up = (i & size) == 0;
+                        const uint64_t a = v[i], b = v[j];
+                        if ((a > b) == up) {
+                            v[i] = b;
+                            v[j] = a;
+                        }
+                    }
+                }
+                __syncthreads();
+            }
+        }
+    };
+    if (total <= kSeqTile) {
+        for (int i = tid; i < total; i += kSelSortThreads) v[i] = cand[i < lt ? i : kSeqTile + i - lt];
+    } else if (same <= kSeqTile) {  // too many together: the first k - lt of those sharing the bits, then the rest
+        for (int i = tid; i < same; i += kSelSortThreads) v[i] = cand[kSeqTile + i];
+        bitonic(same);
+        for (int i = tid; i < lt; i += kSelSortThreads) v[k - lt + i] = cand[i];
+        total = k;
+    } else {  // the k - lt first (key, index) among those sharing the bits, found by scanning the keys
         static_assert(kSelSortThreads == (int)kSelLow + 1, "one bin per thread");
+        for (int i = tid; i < lt; i += kSelSortThreads) v[i] = cand[i];
         lh[tid] = 0;
         __syncthreads();
         for (int64_t i = tid; i < V; i += kSelSortThreads)
@@ -507,26 +539,7 @@ __global__ __launch_bounds__(kSelSortThreads) void sampler_select_draw_kernel(co
             if (r < k) order[r] = (int32_t)(mine & 0xFFFFFFFFull);
         }
     } else {
-        int m = 1;
-        while (m < total) m <<= 1;
-        for (int i = total + tid; i < m; i += kSelSortThreads) v[i] = ~0ull;
-        __syncthreads();
-        for (int size = 2; size <= m; size <<= 1) {
-            for (int stride = size >> 1; stride > 0; stride >>= 1) {
-                for (int i = tid; i < m; i += kSelSortThreads) {
-                    const int j = i ^ stride;
-                    if (j > i) {
-                        const bool up = (i & size) == 0;
-                        const uint64_t a = v[i], b = v[j];
-                        if ((a > b) == up) {
-                            v[i] = b;
-                            v[j] = a;
-                        }
-                    }
-                }
-                __syncthreads();
-            }
-        }
+        bitonic(total);
         for (int i = tid; i < k; i += kSelSortThreads) order[i] = (int32_t)(v[i] & 0xFFFFFFFFull);
     }
     __syncthreads();
@@ -1228,7 +1241,7 @@ struct SamplerWork {
     bool in_flight = false;              // a call ended before its final wait: lists_host may still be read
     int64_t *result = nullptr;           // the context's pinned words: (token, whether a random number was used)
     uint32_t *sel_hist = nullptr;  // top-k selection: 2 digit histograms of kSelBins (the first kept zero between calls), kSelCtrs counters
-    uint64_t *sel_cand = nullptr;  // the selected (key, index) values, kSeqTile
+    uint64_t *sel_cand = nullptr;  // the gathered (key, index) values, 2 kSeqTile
     float *gpv = nullptr;      // the greedy branch's per-workgroup best values
     int64_t *gpi = nullptr;    // and their indices
     void *sort_tmp = nullptr;
@@ -1284,7 +1297,7 @@ static int32_t ensure_work(aesir_ctx *ctx, int64_t V, int64_t n_lists) {
         AESIR_HIP_TRY(hipMalloc((void **)&w->slow_list, (size_t)kSlowListMax * 4));
         AESIR_HIP_TRY(hipMalloc((void **)&w->sel_hist, (size_t)(2 * kSelBins + kSelCtrs) * 4));
         w->in_flight = true;  // its first histogram is not zero yet
-        AESIR_HIP_TRY(hipMalloc((void **)&w->sel_cand, (size_t)kSeqTile * 8));
+        AESIR_HIP_TRY(hipMalloc((void **)&w->sel_cand, (size_t)2 * kSeqTile * 8));
         AESIR_HIP_TRY(hipMalloc((void **)&w->marks, (size_t)(nbat + 1) * 4));
         size_t bytes = 0;
         AESIR_HIP_TRY(rocprim::radix_sort_pairs(nullptr, bytes, w->keys, w->keys_out, w->idx, w->idx_out,

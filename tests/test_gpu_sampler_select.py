@@ -1,5 +1,6 @@
 """The sampler's top-k selection and token lists where their route changes: more ties at the k-th logit
-than the sorting workgroup holds (constant logits, three levels), exactly as many candidates as top_k
+than the sorting workgroup holds (constant logits, three levels), fewer ties but more together with the
+candidates above them, exactly as many candidates as top_k
 leaves, token lists on both sides of the length that the prepare kernel scans itself, ids outside the
 vocabulary, vocabularies around a workgroup's 1024 entries. Token and RuneRNG state equal the oracle's
 (exact: both sides run the reference's f32 sums in the reference's order)."""
@@ -20,6 +21,9 @@ def A():
     (128256, 1, 40, 0, 0), (128256, 1, 4096, 5, 0), (128256, 3, 1000, 300, 2), (60000, 2, 3000, 8192, 0),
     (60000, 200, 64, 8190, 3), (1023, 1, 1000, 10, 0), (1024, 60, 1023, 0, 1), (1025, 60, 40, 2000, 10),
     (4097, 1, 4096, 1, 1), (2, 1, 1, 0, 0),
+    # more gathered than the workgroup holds, of which those that share the k-th key's bits are fewer
+    (60000, 200, 4090, 10, 0), (60000, 200, 4096, 0, 2), (60000, 20, 4096, 0, 0), (128256, 4000, 4096, 256, 0),
+    (30000, 8, 4000, 0, 0), (8192, 2, 4095, 0, 0), (8193, 2, 4096, 0, 0),
 ])
 def test_selection(A, oracle, vocab, levels, top_k, n_context, n_suppress):
     rng = np.random.default_rng(vocab + top_k + n_context)
