@@ -96,10 +96,11 @@ __global__ void sampler_mark_kernel(const int64_t *__restrict__ ctx, int64_t n_c
 //   3. one workgroup sorts what was gathered as 64-bit values in LDS and keeps the first top_k;
 //      the pairs are distinct, so any correct sort gives the stable sort's order. Where both kinds
 //      together are more than LDS holds (top_k near kSeqTile), those sharing the bits are sorted and
-//      cut first (128256 logits, top-k 4096 with top-p, us per call: 144, and 266 by scanning the keys);
-//      where they alone are more
-//      (large ties), it finds the last digit and the lowest-index ties itself by scanning the keys
-//      (about 60 us more at 128256 logits that are all equal)
+//      cut first (128256 logits, top-k 4096 with top-p, us per call: 144, and 266 by scanning the keys).
+//      Where they alone are more (large ties: masked logits), it takes the lowest-index ones by scanning
+//      the keys in index order, as far as it needs where the gather saw only one key among them, else
+//      twice over all keys for the last digit too (128256 logits, 10 of them not masked, top-k 40, us per
+//      call: 65, and 252 by two scans of all keys)
 //   4. the same workgroup makes the truncations and the draw (sampler_select_draw_kernel)
 // Three launches where three digit passes, a count, an ordered compaction, a sort and a tail took seven.
 // Measured on MI355X, 128256 logits, 256 context tokens, top-k 40 with top-p, us per blocking call:
@@ -109,7 +110,8 @@ constexpr int kSelPer = 4;                              // keys per thread of th
 constexpr int kSelBlock = kSThreads * kSelPer;          // keys per workgroup
 constexpr int kSelShift[2] = {21, 10};
 constexpr uint32_t kSelLow = 0x3FFu;  // the bits below both digits
-constexpr int kSelCtrs = 4;           // after the two histograms: gathered below / sharing, keys below, the shared bits
+constexpr int kSelCtrs = 6;           // after the two histograms: gathered below / sharing, keys below, the shared bits,
+                                      // of the sharing keys' low bits the largest, and kSelLow minus the smallest
 
 struct SelState {
     uint32_t prefix;  // digits fixed so far
@@ -277,6 +279,8 @@ __global__ __launch_bounds__(kSThreads) void sampler_select_gather_kernel(const 
         ctr[2] = st.lt;
         ctr[3] = top;
     }
+    uint32_t most = 0, least = 0;  // of the low bits: the largest, and kSelLow minus the smallest
+    bool any = false;
 #pragma unroll
     for (int j = 0; j < kSelPer; j++) {
         const int64_t i = base + j * kSThreads + tid;
@@ -288,10 +292,22 @@ __global__ __launch_bounds__(kSThreads) void sampler_select_gather_kernel(const 
         if (lane == 1 && same) at = atomicAdd(&ctr[1], (uint32_t)__popcll(same));
         const uint32_t a = __shfl(at, 0), b = __shfl(at, 1);
         const uint64_t before = (1ull << lane) - 1ull;
+        if (in && t == top) {
+            most = max(most, kv[j] & kSelLow);
+            least = max(least, kSelLow - (kv[j] & kSelLow));
+        }
+        any |= same != 0;  // uniform over the wave
         uint32_t slot = 2 * kSeqTile;
         if (in && t < top) slot = a + (uint32_t)__popcll(below & before);  // (fewer than k of them)
         if (in && t == top) slot = kSeqTile + b + (uint32_t)__popcll(same & before);
         if (slot < 2 * kSeqTile) cand[slot] = ((uint64_t)kv[j] << 32) | (uint64_t)i;
+    }
+    if (any) {
+        for (int o = 32; o > 0; o >>= 1) {
+            most = max(most, (uint32_t)__shfl_xor((int)most, o));
+            least = max(least, (uint32_t)__shfl_xor((int)least, o));
+        }
+        if (lane < 2) atomicMax(&ctr[4 + lane], lane == 0 ? most : least);
     }
 }
 
@@ -490,22 +506,30 @@ __global__ __launch_bounds__(kSelSortThreads) void sampler_select_draw_kernel(co
     } else {  // the k - lt first (key, index) among those sharing the bits, found by scanning the keys
         static_assert(kSelSortThreads == (int)kSelLow + 1, "one bin per thread");
         for (int i = tid; i < lt; i += kSelSortThreads) v[i] = cand[i];
-        lh[tid] = 0;
-        __syncthreads();
-        for (int64_t i = tid; i < V; i += kSelSortThreads)
-            if (keys[i] >> kSelShift[1] == top) atomicAdd(&lh[keys[i] & kSelLow], 1u);
-        __syncthreads();
-        const uint32_t mine = lh[tid], need = (uint32_t)(k - lt);
-        for (int o = 1; o < kSelSortThreads; o <<= 1) {  // inclusive sums
-            const uint32_t t = tid >= o ? lh[tid - o] : 0u;
+        const uint32_t need = (uint32_t)(k - lt);
+        if (ctr[4] + ctr[5] == kSelLow) {  // one key
+            if (tid == 0) {
+                sh[0] = ctr[4];
+                sh[1] = sh[2] = 0;
+            }
+        } else {
+            lh[tid] = 0;
             __syncthreads();
-            lh[tid] += t;
+            for (int64_t i = tid; i < V; i += kSelSortThreads)
+                if (keys[i] >> kSelShift[1] == top) atomicAdd(&lh[keys[i] & kSelLow], 1u);
             __syncthreads();
-        }
-        if (lh[tid] >= need && lh[tid] - mine < need) {
-            sh[0] = (uint32_t)tid;          // the last digit of the k-th key
-            sh[1] = lh[tid] - mine;         // keys with a smaller one
-            sh[2] = 0;
+            const uint32_t mine = lh[tid];
+            for (int o = 1; o < kSelSortThreads; o <<= 1) {  // inclusive sums
+                const uint32_t t = tid >= o ? lh[tid - o] : 0u;
+                __syncthreads();
+                lh[tid] += t;
+                __syncthreads();
+            }
+            if (lh[tid] >= need && lh[tid] - mine < need) {
+                sh[0] = (uint32_t)tid;          // the last digit of the k-th key
+                sh[1] = lh[tid] - mine;         // keys with a smaller one
+                sh[2] = 0;
+            }
         }
         __syncthreads();
         const uint32_t T = (top << kSelShift[1]) | sh[0], less = sh[1];
@@ -526,6 +550,7 @@ __global__ __launch_bounds__(kSelSortThreads) void sampler_select_draw_kernel(co
             r += (uint32_t)__popcll(eq & ((1ull << lane) - 1ull));
             if (in && key == T && r < need - less) v[lt + less + r] = ((uint64_t)key << 32) | (uint64_t)i;
             __syncthreads();
+            if (less == 0 && met >= need) break;  // uniform
         }
         total = k;
     }

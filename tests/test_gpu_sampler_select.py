@@ -58,3 +58,40 @@ def test_truncations_of_the_selection(A, oracle, top_k, top_p, min_p):
             want, o_state = oracle.sample_token_f16(logits, oracle.SamplerConfig(**cfg), o_state, [], [])
             assert got == want, d
             assert g_rng.state == o_state, d
+
+
+@pytest.mark.parametrize("vocab,live,top_k", [(128256, 10, 40), (128256, 0, 40), (32000, 60, 1000), (4097, 3, 4), (4100, 1, 4096),
+                                              (20000, 39, 40), (20000, 40, 40)])
+def test_masked_logits(A, oracle, vocab, live, top_k):
+    """Nearly all logits masked to -inf (sanitized to one value): the selection is filled up with the masked ones
+    of the lowest indices."""
+    rng = np.random.default_rng(vocab + live)
+    cfg = dict(temperature=0.8, top_k=top_k, top_p=1.0, min_p=0.0, repetition_penalty=1.1)
+    g_rng, o_state = A.RuneRNG(4), oracle.rune_rng_state(4)
+    with A.Context(64 << 20) as ctx:
+        for d in range(3):
+            logits = np.full(vocab, -np.inf, np.float16)
+            logits[rng.permutation(vocab)[:live]] = rng.standard_normal(live).astype(np.float16) if d else np.float16(-6e4)
+            context = rng.integers(0, vocab, 5).tolist()
+            got = A.sample_token(ctx, ctx.from_numpy(logits.reshape(1, -1)), A.SamplerConfig(**cfg), g_rng, context, [])
+            want, o_state = oracle.sample_token_f16(logits, oracle.SamplerConfig(**cfg), o_state, context, [])
+            assert got == want, d
+            assert g_rng.state == o_state, d
+
+
+@pytest.mark.parametrize("plain,top_k", [(50, 40), (50, 50), (50, 51), (50, 100), (12000, 64), (12000, 4096)])
+def test_ties_that_differ_in_their_last_bits(A, oracle, plain, top_k):
+    """More logits than the selecting workgroup holds share all but the last bits of their key: equal ones, part of
+    them moved by a repetition penalty next to 1."""
+    vocab = 20000
+    rng = np.random.default_rng(plain + top_k)
+    cfg = dict(temperature=1.0, top_k=top_k, top_p=1.0, min_p=0.0, repetition_penalty=1.00001)
+    g_rng, o_state = A.RuneRNG(6), oracle.rune_rng_state(6)
+    logits = np.full(vocab, -1.6, np.float16)
+    with A.Context(64 << 20) as ctx:
+        for d in range(3):
+            context = rng.permutation(vocab)[plain:].tolist()
+            got = A.sample_token(ctx, ctx.from_numpy(logits.reshape(1, -1)), A.SamplerConfig(**cfg), g_rng, context, [])
+            want, o_state = oracle.sample_token_f16(logits, oracle.SamplerConfig(**cfg), o_state, context, [])
+            assert got == want, d
+            assert g_rng.state == o_state, d
