@@ -29,8 +29,8 @@ def f64_attention(q, K, V, hd, nq, nkv):
     return np.einsum("hs,shd->hd", p, Vd).reshape(-1), np.einsum("hs,shd->hd", p, np.abs(Vd)).reshape(-1), top
 
 
-# positions per wave 64 up to head_dim 32, 32 above; one launch up to 512, 512, 512, 64 and 128 positions,
-# one split up to 512 and 256 positions at head_dim 64 and 128
+# positions per wave 64 up to head_dim 32, 32 above; one launch up to 512 positions, 256 at head_dim 128
+# (a decode step of head_dim 64 and 128: 64 and 128 cache rows, then rounds of 64 positions up to these)
 VIEWS = {8: (1, 63, 64, 65, 511, 512, 513), 16: (1, 63, 64, 65, 511, 512, 513), 32: (1, 63, 64, 65, 511, 512, 513),
          64: (1, 31, 32, 33, 63, 64, 65, 511, 512, 513), 128: (1, 31, 32, 33, 127, 128, 129, 255, 256, 257)}
 
