@@ -638,10 +638,11 @@ __global__ __launch_bounds__(kAThreads) void attn_fast_merge_kernel(AttnArgs a) 
 // share costs elsewhere. Measured on MI355X, us per step of the device loop, this kernel against the others at
 // an early and a late position: 5 layers of head_dim 8 at 512 rows 93 against 106 and 115 (splits of 64
 // positions and their merge); 8 of head_dim 16 140 against 158 and 176; 8 of head_dim 32 176 against 180 and
-// 198; 22 of head_dim 64 (8 heads per KV head) 566 against 578 at 64 rows, but 589 against 578 and 581 at
-// 128, 600 against 579 and 591 at 256 and 634 against 578 and 634 at 448 rows; 4 of head_dim 128 337.5
-// against 339 and 340 at 128 rows, 342 against 339 and 350 at 256. Not faster: two lanes per K row (each
-// load then touches 32 lines).
+// 198; 22 of head_dim 64 (8 heads per KV head, f16 weights) 567 against 579 and 579 at 64 rows, 577 against 579
+// and 583 at 96, but 588 against 578 and 581 at 112, 600 against 579 and 591 at 256 and 634 against 578 and 634 at
+// 448; 4 of head_dim 128 (4 heads per KV head) 337.5 against 339 and 340 at 128 rows, 342 against 339 and 348 at 160;
+// 10 with 2 heads 276 against 275 and 278 at 128; 10 with one head per KV head 281 against 281 and 282 at 64, 285
+// against 281 and 284 at 96. Not faster: two lanes per K row (each load then touches 32 lines).
 template <int HD>
 __global__ __launch_bounds__(1024) void attn_short_kernel(AttnArgs a) {
     constexpr int CH = HD / 8;                       // lanes (16-byte chunks) per row
@@ -750,12 +751,14 @@ static int fast_group(const AttnArgs &a) {
 
 // Decode steps over at most this many cache rows run on attn_short_kernel (both sides of each line are measured
 // there).
-static int64_t short_view_max(int64_t hd) { return hd == 8 || hd == 16 || hd == 32 ? 512 : hd == 64 ? 64 : hd == 128 ? 128 : 0; }
+static int64_t short_view_max(int64_t hd, int64_t G) {
+    return hd == 8 || hd == 16 || hd == 32 ? 512 : hd == 64 ? 96 : hd == 128 ? (G > 1 ? 128 : 64) : 0;
+}
 
 // Views of at most this many positions run as one split: attn_short_kernel, or (head_dim 64 and 128)
 // one workgroup per head group with groups of 256 threads taking two rounds each at most, and no
 // merge launch.
-static int64_t single_split_max(int64_t hd) { return hd == 64 ? 8 * kRound : hd == 128 ? 4 * kRound : short_view_max(hd); }
+static int64_t single_split_max(int64_t hd) { return hd == 64 ? 8 * kRound : hd == 128 ? 4 * kRound : short_view_max(hd, 1); }
 
 // Split count: one split for short views (above); otherwise one 64-position round per split up
 // to 64 splits (more splits cost more in the merge than they gain in parallelism on MI355X;
@@ -786,7 +789,7 @@ int32_t launch_attention_decode(hipStream_t s, const AttnArgs &a) {
     // a view known at the launch (no rows past it are requested) takes the short-view kernel at any length of
     // one split: 32 heads of 128 over 8 KV heads, us per call, 100 positions 4.9 -> 3.9, 256 7.2 -> 4.5; 32 heads of
     // 64 over 4, 300 positions 5.2 -> 4.2, 512 5.6 -> 4.7
-    if (a.max_split == 1 && a.max_seq <= (a.seq_len > 0 ? single_split_max(a.hd) : short_view_max(a.hd)) &&
+    if (a.max_split == 1 && a.max_seq <= (a.seq_len > 0 ? single_split_max(a.hd) : short_view_max(a.hd, G)) &&
         a.nq <= 65535 && rows_16(a)) {
         const int pw = a.hd >= 64 ? 32 : 64;  // positions per wave (attn_short_kernel)
         const dim3 grid((unsigned)a.nq), block((unsigned)((a.max_seq + pw - 1) / pw * kWave));

@@ -30,7 +30,7 @@ def f64_attention(q, K, V, hd, nq, nkv):
 
 
 # positions per wave 64 up to head_dim 32, 32 above; one launch up to 512 positions, 256 at head_dim 128
-# (a decode step of head_dim 64 and 128: 64 and 128 cache rows, then rounds of 64 positions up to these)
+# (a decode step of head_dim 64 and 128: 96 and 128 cache rows, then rounds of 64 positions up to these)
 VIEWS = {8: (1, 63, 64, 65, 511, 512, 513), 16: (1, 63, 64, 65, 511, 512, 513), 32: (1, 63, 64, 65, 511, 512, 513),
          64: (1, 31, 32, 33, 63, 64, 65, 511, 512, 513), 128: (1, 31, 32, 33, 127, 128, 129, 255, 256, 257)}
 
@@ -57,8 +57,8 @@ def test_view_edges(A, hd, offset):
 
 
 @pytest.mark.parametrize("heads,kv,hd,ctx_len", [(8, 4, 8, 200), (8, 4, 8, 512), (8, 2, 16, 140), (4, 2, 32, 200),
-                                                 (4, 1, 64, 64), (4, 1, 64, 200), (4, 2, 64, 700), (4, 4, 128, 128),
-                                                 (4, 1, 128, 200)])
+                                                 (4, 1, 64, 64), (4, 1, 64, 96), (4, 1, 64, 97), (4, 1, 64, 200), (4, 2, 64, 700),
+                                                 (4, 4, 128, 64), (4, 4, 128, 128), (4, 1, 128, 128), (4, 1, 128, 200)])
 def test_rows_behind_the_position_do_not_count(A, oracle, heads, kv, hd, ctx_len):
     """The cache behind the position holds infinities and NaN (steps of a token whose K and V overflow);
     the steps before them, on both sides of a wave's last position, equal those on a zeroed cache bit for
